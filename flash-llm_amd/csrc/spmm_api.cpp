@@ -35,6 +35,64 @@ int check_shape(const void* comp, const int* offs, const void* b, const void* c,
     return hipSuccess;
 }
 
+// What a call at N <= 64 takes with k_waves waves on each (row tile, slice), in units of about 0.2 us:
+//     k tiles of the longest wave x (a + waves on its CU)  +  adding up k_waves sums  +  a second launch and its slabs.
+// A wave needs a fixed time per tile plus what its neighbours on the CU take from it (LDS and issue slots are
+// shared), so more waves only help while they shorten the longest run faster than they crowd the CU.  A CU holds
+// eight waves; workgroups beyond one round of the GPU wait for a whole round.  The waves on a CU count as a mean of
+// their average and, more so, of the fullest CU's (workgroups of eight waves fill CUs unevenly, e.g. 288 of them).
+// Fitted to whole-call times of nineteen weight shapes (1024 x 1024 .. 49152 x 12288, among them the reference's,
+// kernel_benchmark/benchmark.sh:13-14) x N in {8, 16, 32, 64} x Split_K 1..32 x 1 / 2 / 4 / 8 waves at 70, 80 and
+// 90 % sparsity: N <= 32 the best (Split_K, waves) by this cost is on average 0.4 %, at most 4.3 % above the best
+// measured, N = 64 0.2 % and 2.2 %; the number of waves at a given Split_K is 0.1 % above the best on average.
+double stream_cost(int m, int n, int k, int split_k, int k_waves)
+{
+    const int    units   = m / 128;  // N <= 64: one column group
+    const int    slice   = (k / 64 - 1) / split_k + 1;
+    const double scale   = n / 16.0 * m / 36864.0;
+    const double average = static_cast<double>(units) * split_k / 256.0;  // workgroups per CU
+    if (flashllm_hip_rows_per_workgroup(n, m, split_k) == 8)  // eight row tiles per workgroup sharing B
+        return 1.18 * slice * (3.15 + 0.94 * average) + (split_k > 1 ? 7.8 + split_k * (0.46 + 0.37 * scale) : 0.0);
+    const double resident = 8 / k_waves;
+    const double fullest  = std::ceil(average) < resident ? std::ceil(average) : resident;
+    const double typical  = average < resident ? average : resident;
+    const double rounds   = std::ceil(average / resident);
+    const int    longest  = (slice - 1) / k_waves + 1;
+    const double adding   = k_waves > 1 ? 0.15 * k_waves : 0.0;
+    if (n < 64)
+        return longest * (3.67 + k_waves * (0.7 * fullest + 0.3 * typical)) * rounds + adding + (split_k > 1 ? 18.0 + split_k * (0.84 + 0.22 * scale) : 0.0);
+    return longest * (4.0 + k_waves * (0.86 * fullest + 0.14 * typical)) * rounds + adding + (split_k > 1 ? 7.8 + split_k * (0.46 + 0.37 * scale) : 0.0);
+}
+
+// Whether the GPU (256 CUs of eight waves) holds all workgroups of such a call at once.
+bool one_round(int m, int split_k, int k_waves)
+{
+    return static_cast<long>(m / 128) * split_k <= 256L * (8 / k_waves);
+}
+
+// Waves that share one (row tile, slice) of a call at N <= 64: 1, 2, 4 or 8, by the cost above.  With a Split_K that
+// leaves CUs idle this is most of the call's parallelism (4736 x 5184, N = 32, Split_K 4: 35.9 us with one wave per
+// slice, 13.8 with eight); with a Split_K of the library's choice it replaces slabs, whose reduction costs a launch
+// and about 3 us, by sums in LDS (28672 x 7168, N = 16: Split_K 8 33.1 us, Split_K 1 with eight waves 32.1;
+// 7168 x 7168, N = 64: Split_K 16 23.8, Split_K 4 with eight waves 20.8).  N = 64 keeps one wave on slices of fewer
+// than twelve tiles: there its sums are those of the kernel for wide B, bit for bit.
+int waves_per_slice(int m, int n, int k, int split_k)
+{
+    const int slice = (k / 64 - 1) / split_k + 1;
+    int       best  = 1;
+    if (n > 64 || flashllm_hip_rows_per_workgroup(n, m, split_k) == 8 || (n == 64 && slice < 12))
+        return 1;
+    double best_cost = stream_cost(m, n, k, split_k, 1);
+    for (int w = 2; w <= 8 && w <= slice && one_round(m, split_k, w); w *= 2) {
+        const double cost = stream_cost(m, n, k, split_k, w);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best      = w;
+        }
+    }
+    return best;
+}
+
 bool known_order(int slab_order)
 {
     return slab_order == FLASHLLM_SLABS_PLAIN || slab_order == FLASHLLM_SLABS_BY_WORKGROUP;
@@ -43,10 +101,10 @@ bool known_order(int slab_order)
 int launch_partials(void* stream, const void* comp, const int* offs, const void* b, int ldb, void* c, int m, int n, int k, void* ws, int split_k, int slab_order)
 {
     const int pages = slab_order == FLASHLLM_SLABS_BY_WORKGROUP;
-    // wide B: four waves share every scattered tile; otherwise one wave per (row tile, slice, column group)
+    // wide B: four waves share every scattered tile; otherwise each wave has its own (row tile, run of k tiles)
     if (n % 128 == 0)
         return flashllm_hip_launch_spmm_group(stream, comp, offs, b, ldb, split_k == 1 ? c : ws, m, n, k, split_k, pages);
-    return flashllm_hip_launch_spmm(stream, comp, offs, b, ldb, split_k == 1 ? c : ws, m, n, k, split_k, pages);
+    return flashllm_hip_launch_spmm(stream, comp, offs, b, ldb, split_k == 1 ? c : ws, m, n, k, split_k, pages, waves_per_slice(m, n, k, split_k));
 }
 
 // SpMM_SplitK_API with B's columns ldb halfs apart (the public entry points take a dense column-major B: ldb = K)
@@ -202,17 +260,6 @@ size_t flashllm_workspace_bytes(int m, int n, int split_k)
     return static_cast<size_t>(split_k) * m * n * sizeof(uint16_t);
 }
 
-// One wave streams one (row tile, K slice, column group); a CU holds eight of them (two per SIMD, what the
-// registers allow at N >= 32), so 2048 fit at once and a grid beyond that runs a second, mostly empty round
-// (36864x9216, N = 32: 56 us at 7 slices = 2016 waves, 74 us at 8).  Among the Split_K values of one round the
-// time follows
-//     longest slice (k tiles) x (2 + resident waves per CU)  +  Split_K x (0.5 + 0.5 x (N/16) x (M/36864)):
-// a wave needs a fixed time per tile plus what its neighbours on the CU take from it (LDS and issue slots
-// are shared), so more slices only help while they shorten the longest slice faster than they crowd the CU
-// (12288x12288: 16 slices of 12 tiles beat 20 slices of which the last has 2); every slab costs a write and
-// a read of M*N halfs and a step of the reduction.  Constants fitted to the whole-call times of the
-// reference's twelve weight shapes (kernel_benchmark/benchmark.sh:13-14) x N in {8,16,32,64} at 80 %
-// sparsity: mean 0.3 % and at most 4.6 % above the best Split_K of each case.
 int flashllm_splitk_heuristic(int m, int n, int k)
 {
     if (m <= 0 || k <= 0 || n <= 0 || m % 128 || k % 64)
@@ -241,24 +288,12 @@ int flashllm_splitk_heuristic(int m, int n, int k)
         }
         return best;
     }
-    const int    col_groups = n <= 64 ? 1 : n / 64;
-    const long   units      = static_cast<long>(m / 128) * col_groups;
-    const long   slots      = 256L * 8;
-    int          best       = 1;
-    double       best_cost  = 1e30;
+    int    best      = 1;
+    double best_cost = 1e30;
     for (int s = 1; s <= 32 && s <= kt; s++) {  // workspace sizes in existing callers assume at most 32 slabs
-        if (s > 1 && units * s > slots)
+        if (s > 1 && !one_round(m, s, 1))
             break;
-        // N = 64 with eight row tiles per workgroup (what the launch does for this Split_K when its workgroups
-        // fill between three quarters and all of the CUs): the same form fitted to the same twelve shapes again,
-        // mean 0.5 %, at most 5.7 % above the best.  Crowding costs less there (the waves of a CU no longer fetch
-        // B eight times), so the pick is mostly the largest Split_K whose workgroups fit the 256 CUs.
-        const bool   by_eight = flashllm_hip_rows_per_workgroup(n, m, s) == 8;
-        const double fixed    = by_eight ? 4.0 : 2.0;
-        const double crowding = by_eight ? 0.5 : 1.0;
-        const double per_slab = by_eight ? 1.0 + 0.125 * (n / 16.0) * (m / 36864.0) : 0.5 + 0.5 * (n / 16.0) * (m / 36864.0);
-        const int    longest  = (kt - 1) / s + 1;
-        const double cost     = longest * (fixed + crowding * units * s / 256.0) + (s > 1 ? s * per_slab : 0.0);
+        const double cost = stream_cost(m, n, k, s, waves_per_slice(m, n, k, s));
         if (cost < best_cost) {
             best_cost = cost;
             best      = s;

@@ -252,6 +252,57 @@ __device__ __forceinline__ void load_to_lds_16(const void* src, uint32_t lds)
         : "memory");
 }
 
+// The end of a workgroup whose KS waves share a slice: every wave leaves its accumulators in its own 16 KB of LDS
+// (its tile, no longer needed; NB = 4 in two halves), then the waves divide the blocks of 32 rows x 16 columns among
+// themselves, add the KS contributions to each in the order of k and store it like the one-wave form does.
+template<int NB, int KS>
+__device__ __forceinline__ void add_up_and_store(
+    floatx4* lds, const floatx4 (&acc)[NB][8], _Float16* out, int pages, int M, int N, int col0, int rowtile, int slice, int wave, int lane, unsigned w, unsigned launch)
+{
+    constexpr int kAtOnce  = NB < 2 ? NB : 2;             // column blocks whose sums fit the LDS of a wave at once
+    constexpr int kPerWave = kTileHalfs * 2 / 16;         // 16-byte places per wave
+    const int     cols = N < 16 ? 8 : 16, r16 = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int part = 0; part < NB / kAtOnce; part++) {
+        if (part > 0)
+            __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kAtOnce; i++)
+#pragma unroll
+            for (int rb = 0; rb < 8; rb++)
+                lds[wave * kPerWave + (i * 8 + rb) * kLanes + lane] = acc[part * kAtOnce + i][rb];
+        __syncthreads();
+        for (int u = wave; u < kAtOnce * 4; u += KS) {  // rows 32q .. +31 of column block nb
+            const int i = u / 4, q = u % 4, nb = part * kAtOnce + i;
+            floatx4   lo = lds[(i * 8 + 2 * q) * kLanes + lane], hi = lds[(i * 8 + 2 * q + 1) * kLanes + lane];
+#pragma unroll
+            for (int v = 1; v < KS; v++) {
+                lo += lds[v * kPerWave + (i * 8 + 2 * q) * kLanes + lane];
+                hi += lds[v * kPerWave + (i * 8 + 2 * q + 1) * kLanes + lane];
+            }
+            half4 l, h;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                l[e] = static_cast<_Float16>(lo[e]);
+                h[e] = static_cast<_Float16>(hi[e]);
+            }
+            if (r16 >= cols)
+                continue;
+            if (pages) {
+                uint4* page = reinterpret_cast<uint4*>(out) + (static_cast<size_t>(nb) * launch + w) * (cols * 16);
+                const uint2 a = __builtin_bit_cast(uint2, l), b = __builtin_bit_cast(uint2, h);
+                page[q * (4 * cols) + g * cols + r16] = uint4{a.x, a.y, b.x, b.y};
+            }
+            else {
+                _Float16* o = out + static_cast<size_t>(slice) * M * N + static_cast<size_t>(col0 + nb * 16 + r16) * M
+                              + static_cast<size_t>(rowtile) * kTileRows + q * 32 + g * 4;
+                *reinterpret_cast<half4*>(o)      = l;
+                *reinterpret_cast<half4*>(o + 16) = h;
+            }
+        }
+    }
+}
+
 // NB: 16-column blocks per wave (1 for N <= 16, 2 for N = 32, 4 for N >= 64).
 // DEPTH: ring slots = 1 KB chunks in flight per wave.
 // W: waves per workgroup.  W == 1: a wave is a workgroup and fetches its own B fragments from L2.
@@ -271,8 +322,13 @@ __device__ __forceinline__ void load_to_lds_16(const void* src, uint32_t lds)
 //   * a tile's fragments are 2*NB plain 16-byte LDS reads issued with the operand exchanges.
 // A wave without nonzeros in the slice, or beyond the last row tile, still fetches its pieces and attends
 // every barrier.
-template<int NB, int DEPTH, int W, int G>
-__global__ __launch_bounds__(kLanes* W) void spmm_stream_kernel(const uint4* __restrict__ comp,
+//
+// KS: waves of a workgroup that share one (row tile, slice) (W == 1 only).  They take the slice's k tiles in KS
+// consecutive runs, each with a tile and a stream of its own and without meeting, and at the end add their
+// accumulators up in fp32 through LDS, in the order of k.  The slab they store is that of the whole slice: to the
+// workspace and the reduction a workgroup of KS waves is a workgroup.
+template<int NB, int DEPTH, int W, int G, int KS>
+__global__ __launch_bounds__(kLanes* W* KS) void spmm_stream_kernel(const uint4* __restrict__ comp,
                                                                 const int* __restrict__ offs,
                                                                 const _Float16* __restrict__ B,
                                                                 int ldb,
@@ -290,11 +346,12 @@ __global__ __launch_bounds__(kLanes* W) void spmm_stream_kernel(const uint4* __r
     constexpr int kPieces = W > 1 ? G * 2 * NB / W : 0;    // 1 KB pieces of a window each wave fetches
     static_assert(W == 1 || (G * 2 * NB) % W == 0, "the pieces of a window must divide among the waves");
     static_assert((G & (G - 1)) == 0, "G must be a power of two");
+    static_assert(W == 1 || KS == 1, "waves share either B or a slice");
     // the windows of B first (the LDS address of a direct load travels in M0 and stays small), then the waves' tiles
-    __shared__ __attribute__((aligned(16))) unsigned char lds[kBBytes + W * kTileHalfs * 2];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kBBytes + W * KS * kTileHalfs * 2];
 
     const int lane = threadIdx.x & (kLanes - 1);
-    const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes) : 0;
+    const int wave = W * KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes) : 0;
     uint16_t* const tile = reinterpret_cast<uint16_t*>(lds + kBBytes) + wave * kTileHalfs;
     const int r16  = lane & 15;  // row inside a 16-row block / output column
     const int g    = lane >> 4;  // which 8-wide k chunk of a 32-wide k step
@@ -317,6 +374,11 @@ __global__ __launch_bounds__(kLanes* W) void spmm_stream_kernel(const uint4* __r
     kb            = kb < kt ? kb : kt;
     int ke        = kb + avg;
     ke            = ke < kt ? ke : kt;
+    if constexpr (KS > 1) {  // this wave's run of the slice's tiles
+        const int tiles = ke - kb, base = kb;
+        kb = base + tiles * wave / KS;
+        ke = base + tiles * (wave + 1) / KS;
+    }
 
     floatx4 acc[NB][8];
 #pragma unroll
@@ -514,6 +576,10 @@ __global__ __launch_bounds__(kLanes* W) void spmm_stream_kernel(const uint4* __r
 
     if (!have_rows)
         return;
+    if constexpr (KS > 1) {
+        add_up_and_store<NB, KS>(reinterpret_cast<floatx4*>(lds), acc, out, pages, M, N, col0, rowtile, slice, wave, lane, place.w, units * split_k);
+        return;
+    }
     // D layout of the 16x16 MFMA: lane holds column r16, rows 4*g .. 4*g+3 of each 16-row block.
     if (pages) {  // a workgroup's pages: wave by wave, NB each
         store_pages<NB>(out, acc, wave * NB, N, lane, place.w, units * split_k);
@@ -952,13 +1018,13 @@ __global__ __launch_bounds__(256) void take_rows_kernel(uint4* __restrict__ dst,
     dst[i] = src[static_cast<long>(j) * ld8 + r];
 }
 
-template<int NB, int DEPTH, int W, int G>
+template<int NB, int DEPTH, int W, int G, int KS>
 int launch_spmm(hipStream_t stream, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int col_groups, int pages)
 {
     const unsigned units = (static_cast<unsigned>(m / kTileRows) + W - 1) / W * col_groups;
-    hipLaunchKernelGGL((spmm_stream_kernel<NB, DEPTH, W, G>),
+    hipLaunchKernelGGL((spmm_stream_kernel<NB, DEPTH, W, G, KS>),
                        grid_of(units, split_k),
-                       dim3(kLanes * W),
+                       dim3(kLanes * W * KS),
                        0,
                        stream,
                        static_cast<const uint4*>(comp),
@@ -974,6 +1040,16 @@ int launch_spmm(hipStream_t stream, const void* comp, const int* offs, const voi
                        pages,
                        units);
     return static_cast<int>(hipGetLastError());
+}
+
+template<int KS>
+int launch_by_columns(hipStream_t s, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int pages)
+{
+    if (n <= 16)
+        return launch_spmm<1, 8, 1, 1, KS>(s, comp, offs, b, ldb, out, m, n, k, split_k, 1, pages);
+    if (n == 32)
+        return launch_spmm<2, 8, 1, 1, KS>(s, comp, offs, b, ldb, out, m, n, k, split_k, 1, pages);
+    return launch_spmm<4, 6, 1, 1, KS>(s, comp, offs, b, ldb, out, m, n, k, split_k, n / 64, pages);
 }
 
 // Row tiles per workgroup of the launch for B of n columns, A of m rows and split_k slices: 8 (a CU's eight waves
@@ -1034,17 +1110,19 @@ extern "C" int flashllm_hip_static_workspace(void** ptr)
 
 // pages != 0 (Split_K > 1 only): the slabs go to the workspace by workgroup, for flashllm_hip_launch_reduce_pages
 extern "C" int flashllm_hip_launch_spmm(
-    void* stream, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int pages)
+    void* stream, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int pages, int k_waves)
 {
     hipStream_t s = static_cast<hipStream_t>(stream);
     pages         = pages && split_k > 1;
-    if (n <= 16)
-        return launch_spmm<1, 8, 1, 1>(s, comp, offs, b, ldb, out, m, n, k, split_k, 1, pages);
-    if (n == 32)
-        return launch_spmm<2, 8, 1, 1>(s, comp, offs, b, ldb, out, m, n, k, split_k, 1, pages);
-    if (rows_per_workgroup(n, m, split_k) == 8)
-        return launch_spmm<4, 8, 8, 2>(s, comp, offs, b, ldb, out, m, n, k, split_k, 1, pages);
-    return launch_spmm<4, 6, 1, 1>(s, comp, offs, b, ldb, out, m, n, k, split_k, n / 64, pages);
+    if (n == 64 && rows_per_workgroup(n, m, split_k) == 8)
+        return launch_spmm<4, 8, 8, 2, 1>(s, comp, offs, b, ldb, out, m, n, k, split_k, 1, pages);
+    if (k_waves == 8)
+        return launch_by_columns<8>(s, comp, offs, b, ldb, out, m, n, k, split_k, pages);
+    if (k_waves == 4)
+        return launch_by_columns<4>(s, comp, offs, b, ldb, out, m, n, k, split_k, pages);
+    if (k_waves == 2)
+        return launch_by_columns<2>(s, comp, offs, b, ldb, out, m, n, k, split_k, pages);
+    return launch_by_columns<1>(s, comp, offs, b, ldb, out, m, n, k, split_k, pages);
 }
 
 extern "C" void flashllm_hip_set_rows_per_workgroup(int rows)

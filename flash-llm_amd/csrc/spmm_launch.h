@@ -22,6 +22,8 @@ int flashllm_hip_static_workspace(void** ptr);
 // pages != 0: each workgroup's 128 x 16 blocks of partial sums as 4 KB pages in workgroup order
 // (for flashllm_hip_launch_reduce_pages; needs out 16-byte aligned).
 // ldb: halfs between consecutive columns of B (>= K, a multiple of 8; K for a dense column-major B).
+// k_waves: 1, 2, 4 or 8 waves per workgroup divide each (row tile, slice) among themselves along K (ignored by a
+// launch that takes eight row tiles per workgroup, below).
 // Requires M % 128 == 0, K % 64 == 0, N in {8,16,32,64} or N % 64 == 0.
 int flashllm_hip_launch_spmm(void*       stream,
                              const void* compressed_a,
@@ -33,7 +35,8 @@ int flashllm_hip_launch_spmm(void*       stream,
                              int         n,
                              int         k,
                              int         split_k,
-                             int         pages);
+                             int         pages,
+                             int         k_waves);
 
 // Row tiles per workgroup of flashllm_hip_launch_spmm for n columns, m rows and split_k slices: 8 for n = 64
 // when m / 128 is a multiple of 8 and (m / 1024) * split_k lies in 192 .. 256, otherwise 1.
