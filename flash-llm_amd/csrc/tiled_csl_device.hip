@@ -15,11 +15,15 @@
 //   * The drain's tail-then-main fill and its last-in-first-out write-out
 //     (csrc/SpMM_API.cu:306-346) map j to one output index.
 //
-// One workgroup of four waves per 128x64 tile: the tile is laid out bank-major
-// in LDS, each wave takes eight banks, bank fills and first-zero positions
-// come from 64-lane ballots, and each nonzero writes itself to its final
-// place.  Three kernels: vectors per tile, an in-place prefix sum
-// (TileOffsets), the encoder.
+// Three kernels: vectors per tile, an in-place prefix sum (TileOffsets), the encoder.
+//
+// The path has to read A twice (the caller allocates Compressed_A between the two passes) and to write Compressed_A
+// once: 1.2 GB at 27648 x 9216 and 80 %, HBM-bound when every access is a whole line.  So the count reads 1 KB of a
+// row per load, and the encoder sorts a tile into output order in LDS and stores it as consecutive 16-byte vectors:
+// with every item storing its own 4 bytes at its destination (a line of its own per lane) and one wave counting 128-byte
+// pieces of eight rows at a time the call took 550 us; now 268, and 243 with non-temporal loads and stores (a trace of
+// the former: count 95, encoder 147, i.e. 5.3 and 4.9 TB/s).  About 40 us are a fixed cost: launches, the prefix sum
+// and the copy of its total to the host (2048 x 4096: 43.6 us).
 #include "spmm_launch.h"
 
 #include <hip/hip_runtime.h>
@@ -30,9 +34,8 @@ namespace {
 constexpr int kTileRows = 128;
 constexpr int kTileCols = 64;
 constexpr int kBanks    = 32;
-constexpr int kPerBank  = kTileRows * kTileCols / kBanks;  // 256 positions of a tile map to one bank
 constexpr int kLanes    = 64;
-constexpr int kMaxFill  = kPerBank + 3;  // at most three padding items
+constexpr int kMaxFill  = kTileRows * kTileCols / kBanks + 3;  // 256 positions of a tile map to one bank; at most three padding items
 
 // What the encoder found wrong since the word was last read (FLASHLLM_ENCODE_* bits), one word per GPU.  The host
 // compressor returns an error in these cases; a kernel cannot, so it records them here and carries on.
@@ -43,16 +46,48 @@ __device__ __forceinline__ void report(unsigned int what)
     atomicOr(&g_encode_status, what);
 }
 
-// |x| > 0 in the reference's float compare (csrc/SpMM_API.cu:183): drops +0, -0 and NaN.
-__device__ __forceinline__ bool keeps(uint32_t h)
+// |x| > 0 in the reference's float compare (csrc/SpMM_API.cu:183: drops +0, -0 and NaN) of both halfs of a word at
+// once, as bits 0 and 16
+__device__ __forceinline__ uint32_t keeps_pair(uint32_t w)
 {
-    const uint32_t mag = h & 0x7fffu;
-    return mag != 0 && mag <= 0x7c00u;
+    using ushort2v          = uint16_t __attribute__((ext_vector_type(2)));
+    const ushort2v below    = __builtin_bit_cast(ushort2v, w & 0x7fff7fffu) - ushort2v{1, 1};  // +-0 becomes 0xffff
+    const ushort2v distance = __builtin_elementwise_sub_sat(ushort2v{0x7c00, 0x7c00}, below);  // 0 for +-0 and NaN
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(distance, ushort2v{1, 1}));
 }
 
-__device__ __forceinline__ int lanes_below(uint64_t mask)
+// Every kernel here reads and writes each line once: non-temporal loads and stores throughout.
+using uintx4 = uint32_t __attribute__((ext_vector_type(4)));
+
+// Reductions over the 32 lanes of each half wave, the result in all of them: rotations inside the rows of sixteen
+// lanes, then the other row of the half.
+template<int CTRL>
+__device__ __forceinline__ int dpp(int x)
 {
-    return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0));
+    return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true);
+}
+
+template<typename F>
+__device__ __forceinline__ int over_half_wave(int x, F&& f)
+{
+    x = f(x, dpp<0x128>(x));  // row_ror:8, 4, 2, 1
+    x = f(x, dpp<0x124>(x));
+    x = f(x, dpp<0x122>(x));
+    x = f(x, dpp<0x121>(x));
+    return f(x, __builtin_amdgcn_ds_swizzle(x, 0x401f));  // lane ^ 16
+}
+
+__device__ __forceinline__ int half_sum(int x)
+{
+    return over_half_wave(x, [](int a, int b) { return a + b; });
+}
+__device__ __forceinline__ int half_min(int x)
+{
+    return over_half_wave(x, [](int a, int b) { return a < b ? a : b; });
+}
+__device__ __forceinline__ int half_max(int x)
+{
+    return over_half_wave(x, [](int a, int b) { return a > b ? a : b; });
 }
 
 __device__ __forceinline__ const uint16_t* tile_base(const uint16_t* a, int k, int tiles_per_row, int t)
@@ -61,161 +96,271 @@ __device__ __forceinline__ const uint16_t* tile_base(const uint16_t* a, int k, i
     return a + static_cast<size_t>(ti) * kTileRows * k + static_cast<size_t>(tj) * kTileCols;
 }
 
-// offs[t + 1] = 16-byte vectors of tile t (nonzeros rounded up to a multiple of four, over four)
-__global__ __launch_bounds__(kLanes) void count_tiles_kernel(const uint16_t* __restrict__ a, int k, int tiles_per_row, int* __restrict__ offs)
+// offs[t + 1] = 16-byte vectors of tile t (nonzeros rounded up to a multiple of four, over four).
+// A workgroup counts eight tiles side by side: a load takes 1 KB of a row (eight lanes per tile), wave w the rows
+// 16w .. 16w + 15, all of them in flight at once.
+constexpr int kCountWaves = 8;
+constexpr int kCountTiles = kLanes * 8 / kTileCols;
+
+__global__ __launch_bounds__(kLanes* kCountWaves) void count_tiles_kernel(
+    const uint16_t* __restrict__ a, int k, int tiles_per_row, int strips, int* __restrict__ offs)
 {
-    const int       t    = blockIdx.x;
-    const int       lane = threadIdx.x;
-    const uint16_t* base = tile_base(a, k, tiles_per_row, t);
-    int             n    = 0;
-#pragma unroll 4
-    for (int it = 0; it < kTileRows / 8; it++) {
-        const int   m = it * 8 + (lane >> 3);
-        const uint4 v = *reinterpret_cast<const uint4*>(base + static_cast<size_t>(m) * k + (lane & 7) * 8);
-        n += keeps(v.x & 0xffffu) + keeps(v.x >> 16) + keeps(v.y & 0xffffu) + keeps(v.y >> 16) + keeps(v.z & 0xffffu) +
-             keeps(v.z >> 16) + keeps(v.w & 0xffffu) + keeps(v.w >> 16);
+    constexpr int  kRows = kTileRows / kCountWaves;
+    __shared__ int part[kCountWaves][kCountTiles];
+    const int      lane  = threadIdx.x & (kLanes - 1), wave = threadIdx.x / kLanes;
+    const int      ti    = blockIdx.x / strips, strip = blockIdx.x % strips;
+    const int      tj    = strip * kCountTiles + lane / 8;  // this lane's tile
+    int            n     = 0;
+    if (tj < tiles_per_row) {
+        const uint16_t* base = a + (static_cast<size_t>(ti) * kTileRows + wave * kRows) * k + static_cast<size_t>(strip) * (kLanes * 8) + lane * 8;
+        uintx4          v[kRows];
+#pragma unroll
+        for (int i = 0; i < kRows; i++)
+            v[i] = __builtin_nontemporal_load(reinterpret_cast<const uintx4*>(base + static_cast<size_t>(i) * k));
+        uint32_t both = 0;
+#pragma unroll
+        for (int i = 0; i < kRows; i++)  // at most 64 per half: the two counts do not meet
+            both += keeps_pair(v[i][0]) + keeps_pair(v[i][1]) + keeps_pair(v[i][2]) + keeps_pair(v[i][3]);
+        n = static_cast<int>((both & 0xffffu) + (both >> 16));
     }
 #pragma unroll
-    for (int s = 32; s >= 1; s >>= 1)
+    for (int s = 4; s >= 1; s >>= 1)
         n += __shfl_xor(n, s);
-    if (lane == 0)
-        offs[t + 1] = (n + 3) / 4;
+    if ((lane & 7) == 0)
+        part[wave][lane / 8] = n;
+    __syncthreads();
+    const int t = strip * kCountTiles + threadIdx.x;
+    if (threadIdx.x < kCountTiles && t < tiles_per_row) {
+        int sum = 0;
+#pragma unroll
+        for (int w = 0; w < kCountWaves; w++)
+            sum += part[w][threadIdx.x];
+        offs[static_cast<size_t>(ti) * tiles_per_row + t + 1] = (sum + 3) / 4;
+    }
 }
 
 // in place: offs[0] = 0, offs[t + 1] = sum of the counts up to tile t, offs[tiles + 1] = offs[tiles].
-// One workgroup; every thread sums a contiguous run of tiles, the 1024 run totals are scanned once.
-__global__ __launch_bounds__(1024) void scan_offsets_kernel(int* __restrict__ offs, int tiles)
+// One workgroup, latency-bound: up to 16 x 1024 counts are loaded in one round trip (wave w a contiguous run, 64 at a
+// time), scanned across lanes with DPP and across waves in LDS.
+constexpr int kScanWaves = 16;
+constexpr int kScanRuns  = 16;
+
+__device__ __forceinline__ int wave_scan(int x)  // inclusive
 {
-    __shared__ int part[1024];
-    const int      tid = threadIdx.x;
-    const int      run = (tiles + 1023) / 1024;
-    const int      lo  = tid * run < tiles ? tid * run : tiles;
-    const int      hi  = lo + run < tiles ? lo + run : tiles;
-    int            sum = 0;
-    for (int i = lo; i < hi; i++)
-        sum += offs[i + 1];
-    part[tid] = sum;
-    __syncthreads();
-    for (int s = 1; s < 1024; s <<= 1) {
-        const int add = tid >= s ? part[tid - s] : 0;
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1, 2, 4, 8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+    return x;
+}
+
+__global__ __launch_bounds__(kLanes* kScanWaves) void scan_offsets_kernel(int* __restrict__ offs, int tiles)
+{
+    __shared__ int total[kScanWaves];
+    const int      lane  = threadIdx.x & (kLanes - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    int            carry = 0;
+    for (int first = 0; first < tiles;) {
+        const int left = tiles - first, most = (left - 1) / (kLanes * kScanWaves) + 1;
+        const int runs = most < kScanRuns ? most : kScanRuns;
+        const int mine = wave * runs * kLanes + lane;  // counted from `first`
+        int       x[kScanRuns];
+#pragma unroll
+        for (int r = 0; r < kScanRuns; r++) {
+            x[r] = 0;
+            if (r < runs && mine + r * kLanes < left)
+                x[r] = offs[first + mine + r * kLanes + 1];
+        }
+        int sum = 0;
+#pragma unroll
+        for (int r = 0; r < kScanRuns; r++) {
+            x[r] = wave_scan(x[r]) + sum;
+            sum  = __builtin_amdgcn_readlane(x[r], kLanes - 1);
+        }
+        if (lane == 0)
+            total[wave] = sum;
         __syncthreads();
-        part[tid] += add;
+        int before = carry;
+#pragma unroll
+        for (int w = 0; w < kScanWaves; w++) {
+            const int s = total[w];
+            before += w < wave ? s : 0;
+            carry += s;
+        }
         __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kScanRuns; r++)
+            if (r < runs && mine + r * kLanes < left)
+                offs[first + mine + r * kLanes + 1] = x[r] + before;
+        first += left < runs * kLanes * kScanWaves ? left : runs * kLanes * kScanWaves;
     }
-    int acc = part[tid] - sum;  // total of the runs before this one
-    for (int i = lo; i < hi; i++) {
-        acc += offs[i + 1];
-        offs[i + 1] = acc;
-    }
-    if (tid == 1023) {
+    if (threadIdx.x == 0) {
         offs[0]         = 0;
-        offs[tiles + 1] = part[1023];
+        offs[tiles + 1] = carry;
     }
 }
 
-// One workgroup of four waves per tile; wave w owns banks 8w .. 8w+7.
-constexpr int kEncodeWaves  = 4;
-constexpr int kBanksPerWave = kBanks / kEncodeWaves;
+// The encoder: one workgroup of four waves per tile.
+//
+// Element (m, n) lives at swizzled column sw = n ^ ((m % 8) << 3) (csrc/SpMM_API.cu:252-256); bank sw / 2 owns the word
+// sw / 2 of every swizzled row.  Thread (bank, segment) loads its bank's words of rows 16*segment .. +15 (32 lanes take
+// one 128-byte line), i.e. 32 elements of the bank in scan order, and keeps them in registers.  Then
+//   1. counts of all (bank, segment) meet in LDS: fills, heights, padding (every wave works it out for itself);
+//   2. every thread lists its nonzeros by (height, bank) in LDS;
+//   3. level by level: an item of the level is pop number  (items on higher levels) + (banks before it that reach the
+//      level), a sum and a ballot over the half wave that holds the level; the items move to that place, through
+//      registers because the list and the pops share their LDS;
+//   4. vector v of the tile gathers its four items, which lie 32 pops apart, and is stored whole.
+// The list holds 128 levels (16 KB, eight workgroups per CU); a tile in which a bank holds more (about half of all its
+// elements) has every nonzero store itself to its final place in memory instead.
+constexpr int kEncodeThreads = 256;
+constexpr int kSegments      = kEncodeThreads / kBanks;
+constexpr int kRowsOfThread  = kTileRows / kSegments;
+constexpr int kLevels        = 128;
+constexpr int kLevelsAtOnce  = kEncodeThreads / kBanks;
+static_assert(kLevels == kTileRows, "the list's LDS also holds a tile's words");
 
-__global__ __launch_bounds__(kLanes* kEncodeWaves) void encode_tiles_kernel(const uint16_t* __restrict__ a,
-                                                                            int k,
-                                                                            int tiles_per_row,
-                                                                            const int* __restrict__ offs,
-                                                                            uint32_t* __restrict__ out)
+__global__ __launch_bounds__(kEncodeThreads, 6) void encode_tiles_kernel(const uint16_t* __restrict__ a,
+                                                                       int k,
+                                                                       int tiles_per_row,
+                                                                       const int* __restrict__ offs,
+                                                                       uint32_t* __restrict__ out)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t vals[kBanks][kPerBank];  // bank-major: [bank][2*row + (column & 1)]
-    __shared__ int                                   fill_s[kBanks];
-    __shared__ int                                   first_zero_s[kBanks];    // in-tile position of the bank's first zero, -1: none
-    __shared__ int                                   pad_s[3][3];             // bank, height, position of each padding item
-    __shared__ int                                   npad_s;
-    __shared__ int                                   above[kMaxFill + 2];     // items higher than h, over all banks
-    __shared__ uint32_t                              reach[kMaxFill + 2];     // banks holding at least h items
-    __shared__ uint16_t                              tail_dest[4 * kBanks];   // output index of the first 4*rem pops
+    __shared__ uint32_t list[kLevels * kBanks];            // [height - 1][bank]; then the pops in order
+    __shared__ __attribute__((aligned(8))) uint8_t count_s[kBanks][kSegments];
+    __shared__ __attribute__((aligned(8))) uint8_t zero_s[kBanks][kSegments];  // the segment's first zero, 0xff: none
+    __shared__ int      fill_s[kBanks];                    // from here on only for tiles beyond the list
+    __shared__ int      above[kMaxFill + 2];               // items higher than h, over all banks
+    __shared__ uint32_t reach[kMaxFill + 2];               // banks holding at least h items
 
     const int       t    = blockIdx.x;
     const int       tid  = threadIdx.x;
-    const int       lane = tid & (kLanes - 1);
-    const int       wave = tid >> 6;
-    const uint16_t* base = tile_base(a, k, tiles_per_row, t);
+    const int       bank = tid & (kBanks - 1), segment = tid / kBanks;
+    const uint16_t* base = tile_base(a, k, tiles_per_row, t) + static_cast<size_t>(segment) * kRowsOfThread * k;
 
-    // Element (m, n) lives at swizzled column sw = n ^ ((m % 8) << 3) (csrc/SpMM_API.cu:252-256): the
-    // 8-column chunk c of row m becomes chunk c ^ (m % 8), order inside the chunk unchanged, so the four
-    // 32-bit words of a thread's 16 bytes are the four banks (c ^ (m % 8)) * 4 + w at in-bank index 2m, 2m+1.
+    uint32_t word[kRowsOfThread];
 #pragma unroll
-    for (int it = 0; it < kTileRows / 32; it++) {
-        const int   m  = it * 32 + (tid >> 3);
-        const uint4 v  = *reinterpret_cast<const uint4*>(base + static_cast<size_t>(m) * k + (tid & 7) * 8);
-        const int   b0 = ((tid & 7) ^ (m & 7)) * 4;
-        *reinterpret_cast<uint32_t*>(&vals[b0 + 0][2 * m]) = v.x;
-        *reinterpret_cast<uint32_t*>(&vals[b0 + 1][2 * m]) = v.y;
-        *reinterpret_cast<uint32_t*>(&vals[b0 + 2][2 * m]) = v.z;
-        *reinterpret_cast<uint32_t*>(&vals[b0 + 3][2 * m]) = v.w;
+    for (int i = 0; i < kRowsOfThread; i++)
+        word[i] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(base + static_cast<size_t>(i) * k + (((bank >> 2) ^ (i & 7)) * 4 + (bank & 3)) * 2));
+    const int first = offs[t], room = (offs[t + 1] - first) * 4;
+
+    uint32_t kept = 0;  // bit i + 16e: half e of row i
+#pragma unroll
+    for (int i = 0; i < kRowsOfThread; i++)
+        kept |= keeps_pair(word[i]) << i;
+    {
+        const int lo = __builtin_ctz(~kept | 0x10000u), hi = __builtin_ctz((~kept >> 16) | 0x10000u);
+        const int zero = 2 * lo < 2 * hi + 1 ? 2 * lo : 2 * hi + 1;
+        count_s[bank][segment] = static_cast<uint8_t>(__builtin_popcount(kept));
+        zero_s[bank][segment]  = static_cast<uint8_t>(zero < 2 * kRowsOfThread ? zero : 0xff);
     }
     __syncthreads();
 
-    // fill and first zero (in scan order) of this wave's banks
-    for (int bi = 0; bi < kBanksPerWave; bi++) {
-        const int b   = wave * kBanksPerWave + bi;
-        int       cnt = 0, fz = -1;
-#pragma unroll
-        for (int q = 0; q < kPerBank / kLanes; q++) {
-            const uint64_t mask = __builtin_amdgcn_ballot_w64(keeps(vals[b][q * kLanes + lane]));
-            cnt += __builtin_popcountll(mask);
-            if (fz < 0 && ~mask != 0)
-                fz = q * kLanes + __builtin_ctzll(~mask);
+    // this thread's bank: its fill (both halves of every wave hold all banks) and the items below this segment
+    int fill, below;
+    {
+        const uint2    c    = *reinterpret_cast<const uint2*>(&count_s[bank][0]);
+        const uint32_t low  = segment < 4 ? (1u << (8 * segment)) - 1u : 0xffffffffu;
+        const uint32_t high = segment < 4 ? 0u : (1u << (8 * (segment - 4))) - 1u;
+        fill  = static_cast<int>(__builtin_amdgcn_sad_u8(c.y, 0u, __builtin_amdgcn_sad_u8(c.x, 0u, 0u)));
+        below = static_cast<int>(__builtin_amdgcn_sad_u8(c.y & high, 0u, __builtin_amdgcn_sad_u8(c.x & low, 0u, 0u)));
+    }
+    // Padding to a multiple of four: each padding item goes on top of the emptiest bank (lowest index on ties) at that
+    // bank's first zero position, value 0 (csrc/SpMM_API.cu:274-287).
+    const int unpadded = fill;
+    const int nnz      = __builtin_amdgcn_readfirstlane(half_sum(fill));
+    const int pad      = (4 - nnz % 4) % 4;
+    for (int p = 0; p < pad; p++)
+        fill += (half_min((fill << 5) | bank) & (kBanks - 1)) == bank;
+    uint32_t pad_item = 0;
+    if (fill > unpadded) {
+        const uint64_t z = *reinterpret_cast<const uint64_t*>(&zero_s[bank][0]);
+        if (~z == 0) {  // cannot happen: the emptiest bank holds fewer than 256 items
+            if (segment == 0)
+                report(FLASHLLM_ENCODE_NO_ZERO);
         }
-        if (lane == 0) {
-            fill_s[b]       = cnt;
-            first_zero_s[b] = fz < 0 ? -1 : (fz >> 1) * kTileCols + 2 * b + (fz & 1);
+        else {
+            const int s = __builtin_ctzll(~z) / 8;
+            const int i = s * (2 * kRowsOfThread) + static_cast<int>((z >> (8 * s)) & 0xff);
+            pad_item    = static_cast<uint32_t>((i >> 1) * kTileCols + 2 * bank + (i & 1)) << 16;
         }
     }
-    __syncthreads();
+    const int count = nnz + pad;
+    const int top   = __builtin_amdgcn_readfirstlane(half_max(fill));
 
-    // Padding to a multiple of four: each padding item goes on top of the emptiest bank (lowest index
-    // on ties) at that bank's first zero position, value 0 (csrc/SpMM_API.cu:274-287).  Wave 0 decides.
-    if (wave == 0) {
-        int fill = lane < kBanks ? fill_s[lane] : 0;
-        int nnz  = fill;
-#pragma unroll
-        for (int s = 32; s >= 1; s >>= 1)
-            nnz += __shfl_xor(nnz, s);
-        const int pad = (4 - nnz % 4) % 4;
-        for (int p = 0; p < pad; p++) {
-            int key = lane < kBanks ? (fill << 5) | lane : 0x7fffffff;
-#pragma unroll
-            for (int s = 32; s >= 1; s >>= 1) {
-                const int other = __shfl_xor(key, s);
-                key             = other < key ? other : key;
-            }
-            const int b = key & 31;
-            if (lane == b) {
-                const int fz = first_zero_s[b];
-                pad_s[p][0]  = b;
-                pad_s[p][1]  = fill + 1;
-                pad_s[p][2]  = fz < 0 ? 0 : fz;  // the emptiest bank holds fewer than 256 items, so it has a zero
-                if (fz < 0)
-                    report(FLASHLLM_ENCODE_NO_ZERO);
-                fill++;
-            }
-        }
-        if (lane < kBanks)
-            fill_s[lane] = fill;
-        if (lane == 0)
-            npad_s = pad;
-    }
-    __syncthreads();
-
-    int count = 0, top = 0;
-    for (int b = 0; b < kBanks; b++) {
-        const int f = fill_s[b];
-        count += f;
-        top = f > top ? f : top;
-    }
     const int vectors    = count / 4;
     const int rep        = vectors / kBanks, rem = vectors % kBanks;
     const int tail_items = rem * 4;
+    uint32_t* out_tile   = out + static_cast<size_t>(first) * 4;
+    // Never write outside this tile's range of Compressed_A, whatever TileOffsets says: with offsets that were
+    // not computed from this very matrix the output is meaningless, but it stays inside the caller's buffer.
+    const int space = count < room ? count : room;
+    if (room != count && tid == 0)
+        report(FLASHLLM_ENCODE_OFFSETS);
+    const uint32_t first_position = static_cast<uint32_t>(segment * kRowsOfThread * kTileCols + 2 * bank) << 16;
 
-    for (int h = tid; h <= top + 1; h += kLanes * kEncodeWaves) {
+    if (top <= kLevels) {
+        uint32_t* at = &list[below * kBanks + bank];
+#pragma unroll
+        for (int i = 0; i < kRowsOfThread; i++) {
+            const uint32_t position = first_position + (static_cast<uint32_t>(i * kTileCols) << 16);
+            if (kept & (1u << i)) {
+                *at = (word[i] & 0xffffu) | position;
+                at += kBanks;
+            }
+            if (kept & (1u << (i + 16))) {
+                *at = (word[i] >> 16) | (position + 0x10000u);
+                at += kBanks;
+            }
+        }
+        if (segment == 0)
+            for (int h = unpadded; h < fill; h++)
+                list[h * kBanks + bank] = pad_item;
+        __syncthreads();
+
+        uint32_t item[kLevels / kLevelsAtOnce];
+        int      pop[kLevels / kLevelsAtOnce];
+#pragma unroll
+        for (int i = 0; i < kLevels / kLevelsAtOnce; i++) {
+            pop[i] = -1;
+            if (i * kLevelsAtOnce < top) {
+                const int      h      = i * kLevelsAtOnce + segment + 1;
+                const uint64_t have   = __builtin_amdgcn_ballot_w64(fill >= h);  // one level per half wave
+                const int      higher = half_sum(fill > h ? fill - h : 0);
+                if (fill >= h) {
+                    const int before = (tid & 32) ? __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(have >> 32), 0u)
+                                                  : __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(have), 0u);
+                    item[i] = list[(h - 1) * kBanks + bank];
+                    pop[i]  = higher + before;
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kLevels / kLevelsAtOnce; i++) {
+            if (pop[i] >= count) {  // cannot happen while the closed form is right
+                report(FLASHLLM_ENCODE_RANGE);
+                pop[i] = -1;
+            }
+            if (pop[i] >= 0)
+                list[pop[i]] = item[i];
+        }
+        __syncthreads();
+        for (int v = tid; v < space / 4; v += kEncodeThreads) {
+            // a vector of the main part: pops of four passes, last pass first; of the tail (drained first): every rem-th
+            const bool main = v < rep * kBanks;
+            const int  step = main ? kBanks : rem;
+            const int  last = main ? tail_items + (rep - 1 - v / kBanks) * (4 * kBanks) + v % kBanks : v - rep * kBanks;
+            __builtin_nontemporal_store(uintx4{list[last + 3 * step], list[last + 2 * step], list[last + step], list[last]}, reinterpret_cast<uintx4*>(out_tile) + v);
+        }
+        return;
+    }
+
+    if (tid < kBanks)
+        fill_s[bank] = fill;
+    __syncthreads();
+    for (int h = tid; h <= top + 1; h += kEncodeThreads) {
         int      g = 0;
         uint32_t r = 0;
         for (int b = 0; b < kBanks; b++) {
@@ -226,24 +371,16 @@ __global__ __launch_bounds__(kLanes* kEncodeWaves) void encode_tiles_kernel(cons
         above[h] = g;
         reach[h] = r;
     }
-    // the first 4*rem pops are drained first, lane-major per pass; each lane is written back to front
-    if (tid < tail_items)
-        tail_dest[tid] = static_cast<uint16_t>(rep * 4 * kBanks + (tid % rem) * 4 + (3 - tid / rem));
+#pragma unroll
+    for (int i = 0; i < kRowsOfThread; i++)  // the words go to LDS so that the loop below need not be unrolled
+        list[(segment * kRowsOfThread + i) * kBanks + bank] = word[i];
     __syncthreads();
-
-    uint32_t* out_tile = out + static_cast<size_t>(offs[t]) * 4;
-    // Never write outside this tile's range of Compressed_A, whatever TileOffsets says: with offsets that were
-    // not computed from this very matrix the output is meaningless, but it stays inside the caller's buffer.
-    const int room = (offs[t + 1] - offs[t]) * 4;
-    const int full = count;
-    if (room != full && tid == 0)
-        report(FLASHLLM_ENCODE_OFFSETS);
-    count = count < room ? count : room;
-    auto      emit     = [&](int b, int h, uint32_t item) {
-        const int j = above[h] + __builtin_popcount(reach[h] & ((1u << b) - 1u));
+    auto emit = [&](int h, uint32_t item) {
+        const int j = above[h] + __builtin_popcount(reach[h] & ((1u << bank) - 1u));
         int       d;
-        if (j < tail_items) {
-            d = tail_dest[j];
+        if (j < tail_items) {  // the first 4*rem pops, lane-major per pass; each lane is written back to front
+            const int pass = (j >= rem) + (j >= 2 * rem) + (j >= 3 * rem);
+            d              = rep * 4 * kBanks + (j - pass * rem) * 4 + 3 - pass;
         }
         else {
             const int q    = j - tail_items;
@@ -251,31 +388,23 @@ __global__ __launch_bounds__(kLanes* kEncodeWaves) void encode_tiles_kernel(cons
             const int w    = rep * 4 - 1 - pass;           // its place in emission order
             d              = (w / 4) * (4 * kBanks) + ln * 4 + (w % 4);
         }
-        if (d >= 0 && d < count)
+        if (d >= 0 && d < space)
             out_tile[d] = item;
-        if (d < 0 || d >= full)  // cannot happen while the closed form above is right
+        if (d < 0 || d >= count)  // cannot happen while the closed form above is right
             report(FLASHLLM_ENCODE_RANGE);
     };
-
-    for (int bi = 0; bi < kBanksPerWave; bi++) {
-        const int b     = wave * kBanksPerWave + bi;
-        int       below = 0;
-#pragma unroll
-        for (int q = 0; q < kPerBank / kLanes; q++) {
-            const int      i    = q * kLanes + lane;
-            const uint32_t v    = vals[b][i];
-            const bool     keep = keeps(v);
-            const uint64_t mask = __builtin_amdgcn_ballot_w64(keep);
-            if (keep) {
-                const int      h   = below + lanes_below(mask) + 1;
-                const uint32_t pos = static_cast<uint32_t>((i >> 1) * kTileCols + 2 * b + (i & 1));
-                emit(b, h, v | (pos << 16));
-            }
-            below += __builtin_popcountll(mask);
-        }
+    int h = below;
+    for (int i = 0; i < kRowsOfThread; i++) {
+        const uint32_t w        = list[(segment * kRowsOfThread + i) * kBanks + bank];
+        const uint32_t position = first_position + (static_cast<uint32_t>(i * kTileCols) << 16);
+        if (kept & (1u << i))
+            emit(++h, (w & 0xffffu) | position);
+        if (kept & (1u << (i + 16)))
+            emit(++h, (w >> 16) | (position + 0x10000u));
     }
-    if (tid < npad_s)
-        emit(pad_s[tid][0], pad_s[tid][1], static_cast<uint32_t>(pad_s[tid][2]) << 16);
+    if (segment == 0)
+        for (int p = unpadded; p < fill; p++)
+            emit(p + 1, pad_item);
 }
 
 }  // namespace
@@ -285,11 +414,13 @@ extern "C" int flashllm_hip_launch_tile_offsets(void* stream, const void* a, int
     const int   tiles_per_row = k / kTileCols;
     const int   tiles         = (m / kTileRows) * tiles_per_row;
     hipStream_t s             = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(count_tiles_kernel, dim3(tiles), dim3(kLanes), 0, s, static_cast<const uint16_t*>(a), k, tiles_per_row, offs);
+    const int   strips        = (tiles_per_row - 1) / kCountTiles + 1;
+    hipLaunchKernelGGL(count_tiles_kernel, dim3((m / kTileRows) * strips), dim3(kLanes * kCountWaves), 0, s, static_cast<const uint16_t*>(a),
+                       k, tiles_per_row, strips, offs);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return static_cast<int>(e);
-    hipLaunchKernelGGL(scan_offsets_kernel, dim3(1), dim3(1024), 0, s, offs, tiles);
+    hipLaunchKernelGGL(scan_offsets_kernel, dim3(1), dim3(kLanes * kScanWaves), 0, s, offs, tiles);
     return static_cast<int>(hipGetLastError());
 }
 
@@ -314,7 +445,7 @@ extern "C" int flashllm_hip_launch_encode(void* stream, const void* a, int m, in
     const int tiles         = (m / kTileRows) * tiles_per_row;
     hipLaunchKernelGGL(encode_tiles_kernel,
                        dim3(tiles),
-                       dim3(kLanes * kEncodeWaves),
+                       dim3(kEncodeThreads),
                        0,
                        static_cast<hipStream_t>(stream),
                        static_cast<const uint16_t*>(a),

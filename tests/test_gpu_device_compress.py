@@ -85,6 +85,27 @@ def test_uneven_banks(product, oracle, torch_gpu):
     check_against_oracle(product, oracle, torch_gpu, a, "uneven banks")
 
 
+@pytest.mark.parametrize("top", [127, 128, 129, 255, 256])
+def test_tallest_bank(product, oracle, torch_gpu, top):
+    # one bank holds `top` nonzeros beside sparse ones: 128 is the last tile the encoder sorts in LDS
+    rng = np.random.default_rng(top)
+    tiles = []
+    for extra in range(4):  # every padding count
+        rows = np.zeros((128, 32, 2), dtype=np.float16)  # [row][bank]: the two swizzled columns of a bank
+        flat = rows.reshape(128, 64)
+        flat[rng.random((128, 64)) < 0.2] = 0.5
+        bank = np.zeros(256, dtype=np.float16)
+        bank[rng.choice(256, size=top, replace=False)] = rng.uniform(0.5, 1.0, size=top).astype(np.float16)
+        rows[:, 7 * extra + 3, :] = bank.reshape(128, 2)
+        other = np.flatnonzero(rows[:, 0, 0] == 0)[:extra]
+        rows[other, 0, 0] = 0.25
+        column = np.arange(64)[None, :] ^ ((np.arange(128)[:, None] % 8) << 3)
+        tile = np.zeros((128, 64), dtype=np.float16)
+        np.put_along_axis(tile, column, flat, axis=1)
+        tiles.append(tile)
+    check_against_oracle(product, oracle, torch_gpu, np.concatenate(tiles, axis=1), f"tallest bank {top}")
+
+
 def test_special_values(product, oracle, torch_gpu):
     # -0 and NaN are dropped, subnormals and infinities are kept (the reference's float compare)
     rng = np.random.default_rng(7)
