@@ -93,6 +93,16 @@ int waves_per_slice(int m, int n, int k, int split_k)
     return best;
 }
 
+// Groups of four waves that divide a slice of a call at N % 128 == 0: three where the launch gives a CU at most one
+// workgroup and the runs are long enough to pay for their own fill and the sum (measured in us with one / three:
+// 7168 x 7168, N = 128, slices of 112 tiles 90.6 / 71.6, of 56 50.2 / 44.7, of 28 31.4 / 31.7; 2048 x 8192, N = 384, of 32
+// 33.0 / 30.9; 9216 x 36864, N = 128, of 192 152.9 / 123.9), otherwise one.
+int runs_per_slice(int m, int n, int k, int split_k)
+{
+    const int slice = (k / 64 - 1) / split_k + 1;
+    return static_cast<long>(m / 128) * (n / 128) * split_k <= 256 && slice >= 32 ? 3 : 1;
+}
+
 bool known_order(int slab_order)
 {
     return slab_order == FLASHLLM_SLABS_PLAIN || slab_order == FLASHLLM_SLABS_BY_WORKGROUP;
@@ -103,7 +113,7 @@ int launch_partials(void* stream, const void* comp, const int* offs, const void*
     const int pages = slab_order == FLASHLLM_SLABS_BY_WORKGROUP;
     // wide B: four waves share every scattered tile; otherwise each wave has its own (row tile, run of k tiles)
     if (n % 128 == 0)
-        return flashllm_hip_launch_spmm_group(stream, comp, offs, b, ldb, split_k == 1 ? c : ws, m, n, k, split_k, pages);
+        return flashllm_hip_launch_spmm_group(stream, comp, offs, b, ldb, split_k == 1 ? c : ws, m, n, k, split_k, pages, runs_per_slice(m, n, k, split_k));
     return flashllm_hip_launch_spmm(stream, comp, offs, b, ldb, split_k == 1 ? c : ws, m, n, k, split_k, pages, waves_per_slice(m, n, k, split_k));
 }
 

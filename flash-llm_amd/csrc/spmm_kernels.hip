@@ -621,12 +621,21 @@ __global__ __launch_bounds__(kLanes* W* KS) void spmm_stream_kernel(const uint4*
 // places are exact counts that never drain the stream, and the accumulators stay where they are (with early
 // exits from the unrolled round the register allocation more than doubled).  A tile with more than R*256
 // vectors takes its remaining rounds on a slow path.
+//
+// KS > 1: KS such groups of four waves form one workgroup and divide the slice's k tiles in KS consecutive runs, each
+// with its own three tile buffers (3 x 48 KB of LDS: the CU's).  Nothing but the meetings is shared until the end,
+// when the first group adds the others' accumulators to its own, in fp32 and in the order of k, through LDS.  It is
+// for launches of at most one workgroup per CU, which a caller's Split_K can ask for: the step is a chain of waits
+// that one group leaves unfilled.  Split_K = 1, 80 %: 7168 x 28672, N = 512 340 -> 258 us, 7168 x 7168, N = 512
+// 91 -> 73, 2048 x 8192, N = 384 102 -> 81; with more than one workgroup per CU it loses what the meetings couple
+// (36864 x 9216, N = 128 166 -> 172).
+constexpr int kSliceRuns    = 3;
 constexpr int kGroupWaves   = 4;
 constexpr int kGroupThreads = kGroupWaves * kLanes;
 constexpr int kAhead        = 3;  // tiles of the stream in flight per wave = the three buffers' rotation
 
-template<int NBW, int R>
-__device__ __forceinline__ void spmm_group_body(uint16_t (&tiles)[3][kTileHalfs],
+template<int NBW, int R, int KS>
+__device__ __forceinline__ void spmm_group_body(uint16_t (*const all_tiles)[kTileHalfs],
                                                 const uint4* __restrict__ comp,
                                                 const int* __restrict__ toff,
                                                 const _Float16* __restrict__ B,
@@ -637,14 +646,16 @@ __device__ __forceinline__ void spmm_group_body(uint16_t (&tiles)[3][kTileHalfs]
                                                 int K,
                                                 int kb,
                                                 int ke,
+                                                int steps,
                                                 int col0,
                                                 int vmax,
                                                 int pages,
                                                 unsigned w,
                                                 unsigned launch)
 {
+    uint16_t (*const tiles)[kTileHalfs] = all_tiles + (KS > 1 ? threadIdx.x / kGroupThreads * 3 : 0);
     const int lane = threadIdx.x & (kLanes - 1);
-    const int wave = threadIdx.x / kLanes;
+    const int wave = KS > 1 ? threadIdx.x / kLanes % kGroupWaves : threadIdx.x / kLanes;
 
     floatx4 acc[NBW][8];
 #pragma unroll
@@ -686,7 +697,7 @@ __device__ __forceinline__ void spmm_group_body(uint16_t (&tiles)[3][kTileHalfs]
         }
     };
     auto load_b = [&](int t) {  // always issued: past the end the last tile's lines are fetched again
-        const int tc = t < ke ? t : ke - 1;
+        const int tc = t < ke ? t : (KS > 1 && ke == 0 ? 0 : ke - 1);
 #pragma unroll
         for (int i = 0; i < 2 * NBW; i++)
             braw[i] = *reinterpret_cast<const uintx4*>(bptr + static_cast<size_t>(i) * 8 * ldb + tc * kTileCols);
@@ -782,7 +793,8 @@ __device__ __forceinline__ void spmm_group_body(uint16_t (&tiles)[3][kTileHalfs]
         clear_quarter(tiles[(j + 2) % 3]);
         meet();
     };
-    for (int t = kb; t < ke; t += kAhead) {
+    const int end = KS > 1 ? kb + steps : ke;
+    for (int t = kb; t < end; t += kAhead) {
         step(std::integral_constant<int, 0>{}, t);
         step(std::integral_constant<int, 1>{}, t + 1);
         step(std::integral_constant<int, 2>{}, t + 2);
@@ -795,6 +807,28 @@ __device__ __forceinline__ void spmm_group_body(uint16_t (&tiles)[3][kTileHalfs]
     // coordinates are derived afresh (through an opaque statement) so that nothing is carried round the loop for this.
     int lane_again = threadIdx.x & (kLanes - 1);
     asm volatile("" : "+v"(lane_again));
+    if constexpr (KS > 1) {
+        // the runs' sums meet in the first run's waves: everybody is past its last read of a tile (the last meeting)
+        constexpr int kSums = NBW * 8 * kLanes;
+        floatx4*      sums  = reinterpret_cast<floatx4*>(&all_tiles[0][0]);
+        const int     run   = threadIdx.x / kGroupThreads;
+        if (run > 0)
+#pragma unroll
+            for (int nb = 0; nb < NBW; nb++)
+#pragma unroll
+                for (int rb = 0; rb < 8; rb++)
+                    sums[((run - 1) * kGroupWaves + wave) * kSums + (nb * 8 + rb) * kLanes + lane_again] = acc[nb][rb];
+        __syncthreads();
+        if (run > 0)
+            return;
+#pragma unroll
+        for (int r = 0; r < KS - 1; r++)
+#pragma unroll
+            for (int nb = 0; nb < NBW; nb++)
+#pragma unroll
+                for (int rb = 0; rb < 8; rb++)
+                    acc[nb][rb] += sums[(r * kGroupWaves + wave) * kSums + (nb * 8 + rb) * kLanes + lane_again];
+    }
     if (pages) {  // o is the workspace itself here; this wave's NBW pages follow those of the waves before it
         store_pages<NBW>(o, acc, static_cast<int>(threadIdx.x / kLanes) * NBW, N, lane_again, w, launch);
         return;
@@ -817,8 +851,8 @@ __device__ __forceinline__ void spmm_group_body(uint16_t (&tiles)[3][kTileHalfs]
     }
 }
 
-template<int NBW>
-__global__ __launch_bounds__(kGroupThreads, 3) void spmm_group_kernel(const uint4* __restrict__ comp,
+template<int NBW, int KS>
+__global__ __launch_bounds__(kGroupThreads* KS, 3) void spmm_group_kernel(const uint4* __restrict__ comp,
                                                                   const int* __restrict__ offs,
                                                                   const _Float16* __restrict__ B,
                                                                   int ldb,
@@ -831,20 +865,28 @@ __global__ __launch_bounds__(kGroupThreads, 3) void spmm_group_kernel(const uint
                                                                   int pages,
                                                                   unsigned units)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t tiles[3][kTileHalfs];
+    __shared__ __attribute__((aligned(16))) uint16_t tiles[3 * KS][kTileHalfs];
     const int   kt    = K / kTileCols;
     const Place place = place_of_workgroup(units, split_k);
     if (!place.valid)
         return;
     const int unit = place.unit, slice = place.part;
     const int rowtile = unit / col_groups;
-    const int col0    = (unit % col_groups) * (kGroupWaves * 16 * NBW) + (threadIdx.x / kLanes) * (16 * NBW);
+    const int col0    = (unit % col_groups) * (kGroupWaves * 16 * NBW) + (threadIdx.x / kLanes % kGroupWaves) * (16 * NBW);
     // the reference's slicing (csrc/SpMM_Kernel.cuh:196-204), clamped to K
     const int avg = (kt - 1) / split_k + 1;
     int       kb  = slice * avg;
     kb            = kb < kt ? kb : kt;
     int ke        = kb + avg;
     ke            = ke < kt ? ke : kt;
+    int steps = ke - kb;  // every wave's, also one whose run is a tile shorter
+    if constexpr (KS > 1) {
+        const int tiles_of_slice = ke - kb, base = kb;
+        const int run = __builtin_amdgcn_readfirstlane(threadIdx.x / kGroupThreads);
+        kb    = base + tiles_of_slice * run / KS;
+        ke    = base + tiles_of_slice * (run + 1) / KS;
+        steps = (tiles_of_slice - 1) / KS + 1;
+    }
     const int* toff = offs + static_cast<size_t>(rowtile) * kt;
     _Float16*  o    = pages ? out : out + static_cast<size_t>(slice) * M * N + static_cast<size_t>(rowtile) * kTileRows;
     // last vector any load of this slice may touch (clamped loads re-read it)
@@ -858,9 +900,9 @@ __global__ __launch_bounds__(kGroupThreads, 3) void spmm_group_kernel(const uint
     if (whole == 0)
         comp = reinterpret_cast<const uint4*>(B);
     if (whole <= 440LL * (M / kTileRows) * kt)
-        spmm_group_body<NBW, 2>(tiles, comp, toff, B, ldb, o, M, N, K, kb, ke, col0, vmax, pages, place.w, units * split_k);
+        spmm_group_body<NBW, 2, KS>(tiles, comp, toff, B, ldb, o, M, N, K, kb, ke, steps, col0, vmax, pages, place.w, units * split_k);
     else
-        spmm_group_body<NBW, 3>(tiles, comp, toff, B, ldb, o, M, N, K, kb, ke, col0, vmax, pages, place.w, units * split_k);
+        spmm_group_body<NBW, 3, KS>(tiles, comp, toff, B, ldb, o, M, N, K, kb, ke, steps, col0, vmax, pages, place.w, units * split_k);
 }
 
 __device__ __forceinline__ void add_slab(float (&s)[4], const uint2 v)
@@ -1136,13 +1178,20 @@ extern "C" int flashllm_hip_rows_per_workgroup(int n, int m, int split_k)
 }
 
 extern "C" int flashllm_hip_launch_spmm_group(
-    void* stream, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int pages)
+    void* stream, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int pages, int runs)
 {
     // 128 columns per workgroup (four waves x 32); requires n % 128 == 0
     const unsigned units = static_cast<unsigned>(m / kTileRows) * (n / 128);
-    hipLaunchKernelGGL(spmm_group_kernel<2>, grid_of(units, split_k), dim3(kGroupThreads), 0, static_cast<hipStream_t>(stream),
-                       static_cast<const uint4*>(comp), offs, static_cast<const _Float16*>(b), ldb, static_cast<_Float16*>(out),
-                       m, n, k, split_k, n / 128, pages && split_k > 1, units);
+    const dim3     grid  = grid_of(units, split_k);
+    hipStream_t    s     = static_cast<hipStream_t>(stream);
+    const uint4*   cp    = static_cast<const uint4*>(comp);
+    const _Float16* bp   = static_cast<const _Float16*>(b);
+    _Float16*      op    = static_cast<_Float16*>(out);
+    pages                = pages && split_k > 1;
+    if (runs == kSliceRuns)
+        hipLaunchKernelGGL((spmm_group_kernel<2, kSliceRuns>), grid, dim3(kGroupThreads * kSliceRuns), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, pages, units);
+    else
+        hipLaunchKernelGGL((spmm_group_kernel<2, 1>), grid, dim3(kGroupThreads), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, pages, units);
     return static_cast<int>(hipGetLastError());
 }
 

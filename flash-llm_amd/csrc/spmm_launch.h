@@ -47,6 +47,7 @@ void flashllm_hip_set_rows_per_workgroup(int rows);
 int  flashllm_hip_rows_per_workgroup(int n, int m, int split_k);
 
 // The same product for wide B (n % 128 == 0) by workgroups of four waves that share each scattered tile.
+// runs: 1, or 3 for workgroups of three such groups that divide each slice along K.
 int flashllm_hip_launch_spmm_group(void*       stream,
                                    const void* compressed_a,
                                    const int*  tile_offsets,
@@ -57,7 +58,8 @@ int flashllm_hip_launch_spmm_group(void*       stream,
                                    int         n,
                                    int         k,
                                    int         split_k,
-                                   int         pages);
+                                   int         pages,
+                                   int         runs);
 
 // c[e] = rn16(sum_s float(ws[s*mn + e])), through max(., 0) first when relu != 0; requires mn % 4 == 0.
 int flashllm_hip_launch_reduce(void* stream, void* c, const void* ws, long mn, int split_k, int relu);
