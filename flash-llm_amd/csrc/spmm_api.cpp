@@ -276,21 +276,15 @@ int flashllm_splitk_heuristic(int m, int n, int k)
         return 1;
     const int kt = k / 64;
     if (n % 128 == 0) {
-        // Wide B goes to the four-wave kernel: a workgroup per (row tile, slice, 128 columns), up to three resident
-        // per CU (768 at once), handed out as earlier ones finish, so more than one round is no loss by itself.
-        // A tile costs a workgroup 1.4 / 1.8 times as long when two / three share the CU as when it has the CU to
-        // itself; every slab costs a write and a read of M*N halfs.  Fitted to whole-call times of seven of the
-        // reference's weight shapes at N = 128 / 256 and Split_K 1..12: mean 1.6 %, at most 10 % above the best.
-        const long   units     = static_cast<long>(m / 128) * (n / 128);
-        const double slab_cost = 2.75 * 4.0 * m * n / 5e6;
+        // Wide B: the slice's tiles at the time of a step, and what a slab costs: M*N halfs written and read at about
+        // 6 TB/s, beside the second launch (3 us).
+        const double slab_cost = 4e-6 / 6.0 * m * n;
         int          best      = 1;
         double       best_cost = 1e30;
         for (int s = 1; s <= 32 && s <= kt; s++) {
-            const long   wgs      = units * s;
-            const long   per_cu   = (wgs + 255) / 256 < 3 ? (wgs + 255) / 256 : 3;
-            const double rounds   = wgs > 768 ? std::pow(wgs / 768.0, 0.8) : 1.0;
-            const int    longest  = (kt - 1) / s + 1;
-            const double cost     = longest * (1.0 + 0.4 * (per_cu - 1)) * rounds + (s > 1 ? s * slab_cost : 0.0);
+            const int    longest = (kt - 1) / s + 1;
+            const double step    = runs_per_slice(m, n, k, s) == 1 ? flashllm_hip_wide_b_step(n, m, s) : 0.6;
+            const double cost    = longest * step + (s > 1 ? 3.0 + s * slab_cost : 0.0);
             if (cost < best_cost) {
                 best_cost = cost;
                 best      = s;

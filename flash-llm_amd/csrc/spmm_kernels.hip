@@ -252,6 +252,21 @@ __device__ __forceinline__ void load_to_lds_16(const void* src, uint32_t lds)
         : "memory");
 }
 
+// The same with the lanes' byte offsets from a common address.
+__device__ __forceinline__ void load_to_lds_16(const void* base, uint32_t offset, uint32_t lds)
+{
+    uint32_t saved;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "v"(offset), "s"(base), "s"(lds)
+        : "memory");
+}
+
 // The end of a workgroup whose KS waves share a slice: every wave leaves its accumulators in its own 16 KB of LDS
 // (its tile, no longer needed; NB = 4 in two halves), then the waves divide the blocks of 32 rows x 16 columns among
 // themselves, add the KS contributions to each in the order of k and store it like the one-wave form does.
@@ -905,6 +920,246 @@ __global__ __launch_bounds__(kGroupThreads* KS, 3) void spmm_group_kernel(const 
         spmm_group_body<NBW, 3, KS>(tiles, comp, toff, B, ldb, o, M, N, K, kb, ke, steps, col0, vmax, pages, place.w, units * split_k);
 }
 
+// ------------------------------------------------------------------------------------------------
+// spmm_wide_kernel: four waves share every scattered tile as above, but each multiplies it by 64 columns, 256 per
+// workgroup (N a multiple of 256).  The 16 KB of operands a wave reads out of LDS per tile then feed 64 MFMAs instead
+// of 32, and the scatter and the clearing are paid once per 256 columns.  128 accumulator registers leave room for two
+// waves per SIMD, and no room to hold B a tile ahead in registers: a tile's lines of B (whole 128-byte lines, piece
+// (l % 8) ^ (l / 8) of a line to slot l % 8) go straight from memory to 8 KB of LDS that belong to the wave, requested
+// as soon as the previous tile's have been read out, i.e. a whole step ahead, and without a meeting.  Fetched in the
+// operand layout instead, where neighbouring lanes hold neighbouring columns, the loads themselves are the bound: 9.7
+// TB/s out of L2 against 32 with neighbouring lanes on one line (256 columns x 7168, all CUs; in this kernel 231 against
+// 206 us at 28672 x 7168, N = 512).
+// A wave's tile is taken in quarters, the reads of one ahead of the MFMAs of the one before; the order is fixed by
+// scheduling barriers, because left alone the reads sink to their first use and because two waits count on it:
+//   * vmcnt(R) at the head of a step: the R loads of the stream, which request() puts behind the fetch of B, are the
+//     only younger ones;
+//   * the statement that names every fragment of B in front of the next fetch: they are out of LDS.
+// 80 KB of LDS, two workgroups per CU.  A step takes 1.15 us alone on a CU and 1.78 us for two, where the four-wave
+// kernel above takes 0.76 / 1.13 / 1.6 us for one / two / three workgroups with half the columns.  Measured, 80 %:
+// 28672 x 7168, N = 512, Split_K 1 246 -> 206 us, 21504 x 7168, N = 512 182 (Split_K 1) -> 163 (3), 36864 x 9216,
+// N = 256 206 -> 192, 7168 x 28672, N = 512 262 (2) -> 216 (4).
+constexpr int kWideWaves = 4;
+constexpr int kWideCols  = kWideWaves * 64;
+
+template<int R>
+__device__ __forceinline__ void spmm_wide_body(unsigned char* lds,
+                                               const uint4* __restrict__ comp,
+                                               const int* __restrict__ toff,
+                                               const _Float16* __restrict__ B,
+                                               int ldb,
+                                               _Float16* __restrict__ o,
+                                               int M,
+                                               int kb,
+                                               int ke,
+                                               int col0,
+                                               int vmax,
+                                               int pages,
+                                               unsigned w,
+                                               unsigned launch)
+{
+    constexpr int NW = kWideWaves, NBW = 4;
+    constexpr int kThreads   = NW * kLanes;
+    constexpr int kTileBytes = kTileHalfs * 2;
+    const int     lane = threadIdx.x & (kLanes - 1);
+    const int     wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    const int     r16 = lane & 15, g = lane >> 4;
+    unsigned char* const tiles = lds + NW * NBW * 2048;
+
+    floatx4 acc[NBW][8];
+#pragma unroll
+    for (int nb = 0; nb < NBW; nb++)
+#pragma unroll
+        for (int rb = 0; rb < 8; rb++)
+            acc[nb][rb] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    // operand of this lane inside a 16-row block: row r16, 16-byte chunk (ks*4 + g) ^ (row%8)
+    const int      a_off0 = r16 * (kTileCols * 2) + ((g ^ (r16 & 7)) << 4);
+    const int      a_off1 = a_off0 ^ 64;
+    // this wave's columns of B
+    const _Float16* bwave  = B + static_cast<size_t>(col0 + wave * (16 * NBW)) * ldb;
+    const unsigned  b_voff = (static_cast<unsigned>(lane >> 3) * static_cast<unsigned>(ldb) + (((lane & 7) ^ (lane >> 3)) << 3)) * 2;
+    unsigned char* const bwin = lds + wave * (NBW * 2048);
+    const uint32_t  bwin_lds  = __builtin_amdgcn_readfirstlane(lds_offset(bwin));
+    auto fetch_b = [&](int t) {  // past the end the last tile's lines are fetched again
+        const _Float16* p = bwave + (t < ke ? t : ke - 1) * kTileCols;
+#pragma unroll
+        for (int i = 0; i < 2 * NBW; i++)
+            load_to_lds_16(p + static_cast<size_t>(i) * 8 * ldb, b_voff, bwin_lds + i * 1024);
+    };
+    half8 bfrag[2][NBW];
+    auto  read_b = [&](int ks) {
+#pragma unroll
+        for (int nb = 0; nb < NBW; nb++)
+            bfrag[ks][nb] = *reinterpret_cast<const half8*>(bwin + nb * 2048 + (ks ? a_off1 : a_off0));
+    };
+    uint4 ring[R];
+    int   ring_lo, ring_n;
+    int   ahead_lo = toff[kb], ahead_hi = toff[kb + 1 < ke ? kb + 1 : ke];  // range of the tile the next request is for
+    auto  request = [&](int t) {  // this wave's part of tile t (empty past the end), always issued
+        ring_lo           = ahead_lo;
+        ring_n            = ahead_hi - ahead_lo;
+        const uint4* from = comp;
+        asm volatile("" : "+s"(from)::"memory");  // behind the fetch of B
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            int v   = ring_lo + (r * NW + wave) * kLanes + lane;
+            v       = v < vmax ? v : vmax;
+            ring[r] = load_stream(from + v);
+        }
+        ahead_lo = ahead_hi;
+        ahead_hi = toff[t + 2 < ke ? t + 2 : ke];
+    };
+    auto scatter = [&](int buf) {
+        uint16_t* tile = reinterpret_cast<uint16_t*>(tiles + buf);
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            if ((r * NW + wave) * kLanes + lane < ring_n)
+                scatter_vector(tile, ring[r]);
+        for (int r = R; r * kThreads < ring_n; r++) {  // a tile longer than R rounds: the rest straight from memory
+            const int i = (r * NW + wave) * kLanes + lane;
+            if (i < ring_n)
+                scatter_vector(tile, load_stream(comp + ring_lo + i));
+        }
+    };
+    auto clear_part = [&](int buf) {
+        const uint4 zero = {0u, 0u, 0u, 0u};
+        uint4*      q    = reinterpret_cast<uint4*>(tiles + buf) + wave * (kTileBytes / 16 / NW);
+#pragma unroll
+        for (int i = 0; i < kTileBytes / 16 / kThreads; i++)
+            q[i * kLanes + lane] = zero;
+    };
+    half8 a[2][4];
+    auto  read_a = [&](auto cc, int buf) {  // quarter c of the tile: k step c / 2, row blocks 4*(c % 2) .. +3
+        constexpr int        c    = decltype(cc)::value;
+        const unsigned char* base = tiles + buf + (c / 2 ? a_off1 : a_off0) + (c % 2) * (64 * kTileCols * 2);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            a[c % 2][i] = *reinterpret_cast<const half8*>(base + i * (16 * kTileCols * 2));
+    };
+    auto multiply = [&](auto cc) {
+        constexpr int c = decltype(cc)::value;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int nb = 0; nb < NBW; nb++)
+                acc[nb][4 * (c % 2) + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[c % 2][i], bfrag[c / 2][nb], acc[nb][4 * (c % 2) + i], 0, 0, 0);
+    };
+    constexpr std::integral_constant<int, 0> q0{};
+    constexpr std::integral_constant<int, 1> q1{};
+    constexpr std::integral_constant<int, 2> q2{};
+    constexpr std::integral_constant<int, 3> q3{};
+    auto meet = [&]() {
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        asm volatile("" ::"s"(ahead_hi));  // here the wait for a scalar load, which shares the counter of LDS, costs nothing
+    };
+    auto keep_in_order = [&]() { __builtin_amdgcn_sched_barrier(0); };
+
+    int cur = 0, next = kTileBytes, old = 2 * kTileBytes;
+    request(kb);
+    fetch_b(kb);
+    clear_part(cur);
+    clear_part(next);
+    meet();
+    scatter(cur);
+    request(kb + 1);
+    meet();
+    for (int t = kb; t < ke; t++) {
+        // this tile's lines of B have landed: only the R loads of the stream are younger
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R) : "memory");
+        read_b(0);
+        read_b(1);
+        read_a(q0, cur);
+        keep_in_order();
+        // ... and are in registers before the next tile's may overwrite them
+        asm volatile("" ::"v"(bfrag[0][0]), "v"(bfrag[0][1]), "v"(bfrag[0][2]), "v"(bfrag[0][3]), "v"(bfrag[1][0]), "v"(bfrag[1][1]), "v"(bfrag[1][2]), "v"(bfrag[1][3]) : "memory");
+        if (t + 1 < ke)
+            fetch_b(t + 1);
+        keep_in_order();
+        read_a(q1, cur);
+        keep_in_order();
+        multiply(q0);
+        keep_in_order();
+        read_a(q2, cur);
+        keep_in_order();
+        multiply(q1);
+        keep_in_order();
+        read_a(q3, cur);
+        clear_part(old);
+        keep_in_order();
+        multiply(q2);
+        keep_in_order();
+        scatter(next);  // tile t + 1 (empty past the end)
+        keep_in_order();
+        request(t + 2);
+        keep_in_order();
+        multiply(q3);
+        meet();
+        const int done = cur;
+        cur  = next;
+        next = old;
+        old  = done;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may land in LDS that is no longer this workgroup's
+
+    if (pages) {
+        store_pages<NBW>(o, acc, wave * NBW, 16 * NBW, lane, w, launch);
+        return;
+    }
+#pragma unroll
+    for (int nb = 0; nb < NBW; nb++) {
+        const int n = col0 + (wave * NBW + nb) * 16 + r16;
+#pragma unroll
+        for (int rb = 0; rb < 8; rb++) {
+            half4 h;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                h[e] = static_cast<_Float16>(acc[nb][rb][e]);
+            *reinterpret_cast<half4*>(o + static_cast<size_t>(n) * M + g * 4 + rb * 16) = h;
+        }
+    }
+}
+
+__global__ __launch_bounds__(kWideWaves* kLanes, 2) void spmm_wide_kernel(const uint4* __restrict__ comp,
+                                                                 const int* __restrict__ offs,
+                                                                 const _Float16* __restrict__ B,
+                                                                 int ldb,
+                                                                 _Float16* __restrict__ out,
+                                                                 int M,
+                                                                 int N,
+                                                                 int K,
+                                                                 int split_k,
+                                                                 int col_groups,
+                                                                 int pages,
+                                                                 unsigned units)
+{
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kWideWaves * 8192 + 3 * kTileHalfs * 2];
+    const int   kt    = K / kTileCols;
+    const Place place = place_of_workgroup(units, split_k);
+    if (!place.valid)
+        return;
+    const int unit = place.unit, slice = place.part;
+    const int rowtile = unit / col_groups;
+    const int col0    = (unit % col_groups) * kWideCols;
+    // slices, the last vector a load may touch and the empty matrix as in spmm_group_kernel
+    const int avg = (kt - 1) / split_k + 1;
+    int       kb  = slice * avg;
+    kb            = kb < kt ? kb : kt;
+    int ke        = kb + avg;
+    ke            = ke < kt ? ke : kt;
+    const int* toff = offs + static_cast<size_t>(rowtile) * kt;
+    _Float16*  o    = pages ? out : out + static_cast<size_t>(slice) * M * N + static_cast<size_t>(rowtile) * kTileRows;
+    int vmax = toff[ke] - 1;
+    vmax     = vmax > 0 ? vmax : 0;
+    const int whole = offs[static_cast<size_t>(M / kTileRows) * kt];
+    if (whole == 0)
+        comp = reinterpret_cast<const uint4*>(B);
+    if (whole <= 440LL * (M / kTileRows) * kt)
+        spmm_wide_body<2>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, vmax, pages, place.w, units * split_k);
+    else
+        spmm_wide_body<3>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, vmax, pages, place.w, units * split_k);
+}
+
 __device__ __forceinline__ void add_slab(float (&s)[4], const uint2 v)
 {
     const half4 h = __builtin_bit_cast(half4, v);
@@ -1118,6 +1373,33 @@ int rows_per_workgroup(int n, int m, int split_k)
     return workgroups >= 192 && workgroups <= 256 ? 8 : 1;
 }
 
+// Columns per workgroup of a launch at N a multiple of 128: 128 (spmm_group_kernel, three workgroups per CU) or 256
+// (spmm_wide_kernel, two), by the time of a step with the workgroups that share a CU (us, fitted to 36864 x 9216,
+// 21504 x 7168, 28672 x 7168 and 7168 x 28672 at N = 256 / 512 and Split_K 1 .. 4), beyond a full round the whole rounds and
+// what the rest of the last one adds.  The four-wave kernel wins where 256 columns would leave CUs to one workgroup
+// or none (21504 x 7168, N = 512, Split_K 1: 182 against 203 us).
+double group_step(long workgroups)
+{
+    if (workgroups <= 768)
+        return workgroups <= 256 ? 0.76 : workgroups <= 512 ? 1.13 : 1.6;
+    const long rest = workgroups % 768;
+    return 1.6 * (workgroups / 768 + (rest == 0 ? 0.0 : rest <= 256 ? 0.47 : rest <= 512 ? 0.7 : 1.0));
+}
+
+double wide_step(long workgroups)
+{
+    if (workgroups <= 512)
+        return workgroups <= 256 ? 1.15 : 1.78;
+    const long rest = workgroups % 512;
+    return 1.78 * (workgroups / 512 + (rest == 0 ? 0.0 : rest <= 256 ? 0.6 : 1.0));
+}
+
+int columns_per_workgroup(int n, int m, int split_k)
+{
+    const long workgroups = static_cast<long>(m / kTileRows) * (n / 128) * split_k;
+    return n % kWideCols == 0 && wide_step(workgroups / 2) < group_step(workgroups) ? kWideCols : 128;
+}
+
 constexpr int      kMaxDevices = 64;
 std::atomic<void*> g_scratch_ptr[kMaxDevices];
 
@@ -1177,18 +1459,31 @@ extern "C" int flashllm_hip_rows_per_workgroup(int n, int m, int split_k)
     return rows_per_workgroup(n, m, split_k);
 }
 
+extern "C" int flashllm_hip_columns_per_workgroup(int n, int m, int split_k)
+{
+    return columns_per_workgroup(n, m, split_k);
+}
+
+extern "C" double flashllm_hip_wide_b_step(int n, int m, int split_k)
+{
+    const long workgroups = static_cast<long>(m / kTileRows) * (n / 128) * split_k;
+    return columns_per_workgroup(n, m, split_k) == kWideCols ? wide_step(workgroups / 2) : group_step(workgroups);
+}
+
 extern "C" int flashllm_hip_launch_spmm_group(
     void* stream, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int pages, int runs)
 {
-    // 128 columns per workgroup (four waves x 32); requires n % 128 == 0
-    const unsigned units = static_cast<unsigned>(m / kTileRows) * (n / 128);
-    const dim3     grid  = grid_of(units, split_k);
-    hipStream_t    s     = static_cast<hipStream_t>(stream);
-    const uint4*   cp    = static_cast<const uint4*>(comp);
-    const _Float16* bp   = static_cast<const _Float16*>(b);
-    _Float16*      op    = static_cast<_Float16*>(out);
-    pages                = pages && split_k > 1;
-    if (runs == kSliceRuns)
+    const int       cols  = columns_per_workgroup(n, m, split_k);
+    const unsigned  units = static_cast<unsigned>(m / kTileRows) * (n / cols);
+    const dim3      grid  = grid_of(units, split_k);
+    hipStream_t     s     = static_cast<hipStream_t>(stream);
+    const uint4*    cp    = static_cast<const uint4*>(comp);
+    const _Float16* bp    = static_cast<const _Float16*>(b);
+    _Float16*       op    = static_cast<_Float16*>(out);
+    pages                 = pages && split_k > 1;
+    if (cols == kWideCols)
+        hipLaunchKernelGGL(spmm_wide_kernel, grid, dim3(kWideWaves * kLanes), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / cols, pages, units);
+    else if (runs == kSliceRuns)
         hipLaunchKernelGGL((spmm_group_kernel<2, kSliceRuns>), grid, dim3(kGroupThreads * kSliceRuns), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, pages, units);
     else
         hipLaunchKernelGGL((spmm_group_kernel<2, 1>), grid, dim3(kGroupThreads), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, pages, units);
@@ -1212,11 +1507,12 @@ extern "C" int flashllm_hip_launch_reduce(void* stream, void* c, const void* ws,
 extern "C" int flashllm_hip_launch_reduce_pages(void* stream, void* c, const void* ws, int m, int n, int split_k, int relu)
 {
     // the units of the SpMM launch for this N: `rows` row tiles x 16*blocks columns (a wave's columns in
-    // spmm_stream_kernel, a workgroup's 128 in spmm_group_kernel)
+    // spmm_stream_kernel, a workgroup's 128 or 256 at n % 128 == 0)
     const bool     group      = n % 128 == 0;
     const int      rows       = group ? 1 : rows_per_workgroup(n, m, split_k);
-    const int      blocks     = group ? 8 : (n <= 16 ? 1 : (n == 32 ? 2 : 4));
-    const int      col_groups = group ? n / 128 : (n <= 64 ? 1 : n / 64);
+    const int      cols       = group ? columns_per_workgroup(n, m, split_k) : (n <= 16 ? 16 : n == 32 ? 32 : 64);
+    const int      blocks     = cols / 16;
+    const int      col_groups = n <= 64 ? 1 : n / cols;
     const unsigned units      = (static_cast<unsigned>(m / kTileRows) + rows - 1) / rows * col_groups;
     const int      pages_per_unit = blocks * rows;
     const dim3     grid = grid_of(units, pages_per_unit);

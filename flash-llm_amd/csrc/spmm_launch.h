@@ -46,8 +46,9 @@ int flashllm_hip_launch_spmm(void*       stream,
 void flashllm_hip_set_rows_per_workgroup(int rows);
 int  flashllm_hip_rows_per_workgroup(int n, int m, int split_k);
 
-// The same product for wide B (n % 128 == 0) by workgroups of four waves that share each scattered tile.
-// runs: 1, or 3 for workgroups of three such groups that divide each slice along K.
+// The same product for wide B (n % 128 == 0) by workgroups of four waves that share each scattered tile, 128 or 256
+// columns each (a rule of n, m and split_k, which the reduction of its pages follows too).
+// runs: 1, or 3 for workgroups of three such groups (of 128 columns) that divide each slice along K.
 int flashllm_hip_launch_spmm_group(void*       stream,
                                    const void* compressed_a,
                                    const int*  tile_offsets,
@@ -60,6 +61,11 @@ int flashllm_hip_launch_spmm_group(void*       stream,
                                    int         split_k,
                                    int         pages,
                                    int         runs);
+
+int flashllm_hip_columns_per_workgroup(int n, int m, int split_k);
+
+// Time of such a launch per k tile of a slice, in us, with one group per workgroup: what Split_K is chosen by.
+double flashllm_hip_wide_b_step(int n, int m, int split_k);
 
 // c[e] = rn16(sum_s float(ws[s*mn + e])), through max(., 0) first when relu != 0; requires mn % 4 == 0.
 int flashllm_hip_launch_reduce(void* stream, void* c, const void* ws, long mn, int split_k, int relu);
