@@ -108,9 +108,10 @@ bool known_order(int slab_order)
     return slab_order == FLASHLLM_SLABS_PLAIN || slab_order == FLASHLLM_SLABS_BY_WORKGROUP;
 }
 
-int launch_partials(void* stream, const void* comp, const int* offs, const void* b, int ldb, void* c, int m, int n, int k, void* ws, int split_k, int slab_order)
+int launch_partials(void* stream, const void* comp, const int* offs, const void* b, int ldb, void* c, int m, int n, int k, void* ws, int split_k, int slab_order, int relu)
 {
-    const int pages = slab_order == FLASHLLM_SLABS_BY_WORKGROUP;
+    // with one slice the sums are final: the activation belongs to them
+    const int pages = split_k == 1 ? 2 * relu : slab_order == FLASHLLM_SLABS_BY_WORKGROUP;
     // wide B: four waves share every scattered tile; otherwise each wave has its own (row tile, run of k tiles)
     if (n % 128 == 0)
         return flashllm_hip_launch_spmm_group(stream, comp, offs, b, ldb, split_k == 1 ? c : ws, m, n, k, split_k, pages, runs_per_slice(m, n, k, split_k));
@@ -118,25 +119,26 @@ int launch_partials(void* stream, const void* comp, const int* offs, const void*
 }
 
 // SpMM_SplitK_API with B's columns ldb halfs apart (the public entry points take a dense column-major B: ldb = K)
-int spmm_splitk_ldb(void* stream, const void* comp, const int* offs, const void* b, int ldb, void* c, int m, int n, int k, void* ws, int split_k)
+// relu: C through max(., 0)
+int spmm_splitk_ldb(void* stream, const void* comp, const int* offs, const void* b, int ldb, void* c, int m, int n, int k, void* ws, int split_k, int relu)
 {
     int rc = check_shape(comp, offs, b, c, m, n, k, ws, split_k);
     if (rc)
         return rc;
     if (ldb < k || ldb % 8)
         return hipErrorInvalidValue;
-    rc = launch_partials(stream, comp, offs, b, ldb, c, m, n, k, ws, split_k, FLASHLLM_SLABS_BY_WORKGROUP);
+    rc = launch_partials(stream, comp, offs, b, ldb, c, m, n, k, ws, split_k, FLASHLLM_SLABS_BY_WORKGROUP, relu);
     if (rc || split_k == 1)
         return rc;
-    return flashllm_hip_launch_reduce_pages(stream, c, ws, m, n, split_k, 0);
+    return flashllm_hip_launch_reduce_pages(stream, c, ws, m, n, split_k, relu);
 }
 
 // The reduction behind launch_partials with the same slab_order.
-int reduce_slabs(void* stream, void* c, const void* ws, int m, int n, int split_k, int relu, int slab_order)
+int reduce_slabs(void* stream, void* c, const void* ws, int m, int n, int split_k, int slab_order)
 {
     if (slab_order == FLASHLLM_SLABS_BY_WORKGROUP)
-        return flashllm_hip_launch_reduce_pages(stream, c, ws, m, n, split_k, relu);
-    return flashllm_hip_launch_reduce(stream, c, ws, static_cast<long>(m) * n, split_k, relu);
+        return flashllm_hip_launch_reduce_pages(stream, c, ws, m, n, split_k, 0);
+    return flashllm_hip_launch_reduce(stream, c, ws, static_cast<long>(m) * n, split_k, 0);
 }
 
 }  // namespace
@@ -160,7 +162,7 @@ int flashllm_spmm_partials(void*       stream,
         return bad;
     if (!known_order(slab_order))
         return hipErrorInvalidValue;
-    return launch_partials(stream, comp, offs, b, k, c, m, n, k, ws, split_k, slab_order);
+    return launch_partials(stream, comp, offs, b, k, c, m, n, k, ws, split_k, slab_order, 0);
 }
 
 int flashllm_splitk_reduce(void* stream, void* c, const void* ws, int m, int n, int split_k, int slab_order)
@@ -171,7 +173,7 @@ int flashllm_splitk_reduce(void* stream, void* c, const void* ws, int m, int n, 
     // pages exist only for shapes the SpMM kernels take
     if (slab_order == FLASHLLM_SLABS_BY_WORKGROUP && (m % 128 || !supported_n(n) || reinterpret_cast<uintptr_t>(ws) % 16))
         return hipErrorInvalidValue;
-    return reduce_slabs(stream, c, ws, m, n, split_k, 0, slab_order);
+    return reduce_slabs(stream, c, ws, m, n, split_k, slab_order);
 }
 
 int flashllm_spmm_splitk(void*       stream,
@@ -190,7 +192,7 @@ int flashllm_spmm_splitk(void*       stream,
     int rc = flashllm_spmm_partials(stream, comp, offs, b, c, m, n, k, ws, split_k, FLASHLLM_SLABS_BY_WORKGROUP);
     if (rc || split_k == 1)
         return rc;
-    return reduce_slabs(stream, c, ws, m, n, split_k, 0, FLASHLLM_SLABS_BY_WORKGROUP);
+    return reduce_slabs(stream, c, ws, m, n, split_k, FLASHLLM_SLABS_BY_WORKGROUP);
 }
 
 // SpMM_SplitK_API for callers that must not allocate and hold no workspace: the slabs go to the
@@ -334,10 +336,10 @@ int flashllm_decoder_layer_linears(void*                         stream,
             return 1;
         return w.split_k > 0 ? w.split_k : flashllm_splitk_heuristic(w.m, tokens, w.k);
     };
-    auto linear = [&](const flashllm_sparse_weight& w, const void* in, int ld_in, void* out, int limit) {
-        return spmm_splitk_ldb(stream, w.nz_weights, w.tile_offsets, in, ld_in, out, w.m, tokens, w.k, ws, split(w, limit));
+    auto linear = [&](const flashllm_sparse_weight& w, const void* in, int ld_in, void* out, int limit, int relu) {
+        return spmm_splitk_ldb(stream, w.nz_weights, w.tile_offsets, in, ld_in, out, w.m, tokens, w.k, ws, split(w, limit), relu);
     };
-    int rc = linear(q, x, hidden, qkv_out, 64);
+    int rc = linear(q, x, hidden, qkv_out, 64, 0);
     if (rc)
         return rc;
     // The attention-output linear multiplies the first `hidden` rows of every column of qkv_out: it reads them
@@ -347,19 +349,14 @@ int flashllm_decoder_layer_linears(void*                         stream,
         if (rc)
             return rc;
     }
-    rc = linear(o, qkv_out, q.m, attn_out, 64);
+    rc = linear(o, qkv_out, q.m, attn_out, 64, 0);
     if (rc)
         return rc;
-    // FFN1 with the ReLU folded into its reduction when there is one
-    const int s1 = split(f1, 128);
-    rc = flashllm_spmm_partials(stream, f1.nz_weights, f1.tile_offsets, attn_out, ffn_mid, f1.m, tokens, f1.k, ws, s1, FLASHLLM_SLABS_BY_WORKGROUP);
+    // FFN1's ReLU rides in whatever stores its sums: the reduction, or the product itself when there is none
+    rc = linear(f1, attn_out, f1.k, ffn_mid, 128, 1);
     if (rc)
         return rc;
-    rc = s1 > 1 ? reduce_slabs(stream, ffn_mid, ws, f1.m, tokens, s1, 1, FLASHLLM_SLABS_BY_WORKGROUP)
-                : flashllm_hip_launch_relu(stream, ffn_mid, static_cast<long>(f1.m) * tokens);
-    if (rc)
-        return rc;
-    return linear(f2, ffn_mid, f2.k, y, 128);
+    return linear(f2, ffn_mid, f2.k, y, 128, 0);
 }
 
 }  // extern "C"

@@ -141,6 +141,18 @@ __device__ __forceinline__ void store_pages(_Float16* ws, const floatx4 (&acc)[N
     }
 }
 
+// How a launch stores its sums (its `store` argument): slabs like C (or C itself), pages (above), or C through max(., 0)
+constexpr int kStorePlain = 0, kStorePages = 1, kStoreRelu = 2;
+
+__device__ __forceinline__ half4 to_half4(const floatx4& x, int store)
+{
+    half4 h;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        h[e] = static_cast<_Float16>(store == kStoreRelu && !(x[e] > 0.f) ? 0.f : x[e]);  // NaN -> 0 like max(x, 0)
+    return h;
+}
+
 __device__ __forceinline__ void clear_tile(uint16_t* tile, int lane)
 {
     const uint4 zero = {0u, 0u, 0u, 0u};
@@ -272,7 +284,7 @@ __device__ __forceinline__ void load_to_lds_16(const void* base, uint32_t offset
 // themselves, add the KS contributions to each in the order of k and store it like the one-wave form does.
 template<int NB, int KS>
 __device__ __forceinline__ void add_up_and_store(
-    floatx4* lds, const floatx4 (&acc)[NB][8], _Float16* out, int pages, int M, int N, int col0, int rowtile, int slice, int wave, int lane, unsigned w, unsigned launch)
+    floatx4* lds, const floatx4 (&acc)[NB][8], _Float16* out, int store, int M, int N, int col0, int rowtile, int slice, int wave, int lane, unsigned w, unsigned launch)
 {
     constexpr int kAtOnce  = NB < 2 ? NB : 2;             // column blocks whose sums fit the LDS of a wave at once
     constexpr int kPerWave = kTileHalfs * 2 / 16;         // 16-byte places per wave
@@ -295,15 +307,10 @@ __device__ __forceinline__ void add_up_and_store(
                 lo += lds[v * kPerWave + (i * 8 + 2 * q) * kLanes + lane];
                 hi += lds[v * kPerWave + (i * 8 + 2 * q + 1) * kLanes + lane];
             }
-            half4 l, h;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                l[e] = static_cast<_Float16>(lo[e]);
-                h[e] = static_cast<_Float16>(hi[e]);
-            }
+            const half4 l = to_half4(lo, store), h = to_half4(hi, store);
             if (r16 >= cols)
                 continue;
-            if (pages) {
+            if (store == kStorePages) {
                 uint4* page = reinterpret_cast<uint4*>(out) + (static_cast<size_t>(nb) * launch + w) * (cols * 16);
                 const uint2 a = __builtin_bit_cast(uint2, l), b = __builtin_bit_cast(uint2, h);
                 page[q * (4 * cols) + g * cols + r16] = uint4{a.x, a.y, b.x, b.y};
@@ -353,7 +360,7 @@ __global__ __launch_bounds__(kLanes* W* KS) void spmm_stream_kernel(const uint4*
                                                                 int K,
                                                                 int split_k,
                                                                 int col_groups,
-                                                                int pages,
+                                                                int store,
                                                                 unsigned units)
 {
     constexpr int kBTile  = NB * 2048;                     // bytes of B per k tile in LDS: 16*NB columns x 128
@@ -592,11 +599,11 @@ __global__ __launch_bounds__(kLanes* W* KS) void spmm_stream_kernel(const uint4*
     if (!have_rows)
         return;
     if constexpr (KS > 1) {
-        add_up_and_store<NB, KS>(reinterpret_cast<floatx4*>(lds), acc, out, pages, M, N, col0, rowtile, slice, wave, lane, place.w, units * split_k);
+        add_up_and_store<NB, KS>(reinterpret_cast<floatx4*>(lds), acc, out, store, M, N, col0, rowtile, slice, wave, lane, place.w, units * split_k);
         return;
     }
     // D layout of the 16x16 MFMA: lane holds column r16, rows 4*g .. 4*g+3 of each 16-row block.
-    if (pages) {  // a workgroup's pages: wave by wave, NB each
+    if (store == kStorePages) {  // a workgroup's pages: wave by wave, NB each
         store_pages<NB>(out, acc, wave * NB, N, lane, place.w, units * split_k);
         return;
     }
@@ -607,12 +614,7 @@ __global__ __launch_bounds__(kLanes* W* KS) void spmm_stream_kernel(const uint4*
         if (n < N) {
 #pragma unroll
             for (int rb = 0; rb < 8; rb++) {
-                half4 h;
-                h[0] = static_cast<_Float16>(acc[nb][rb][0]);
-                h[1] = static_cast<_Float16>(acc[nb][rb][1]);
-                h[2] = static_cast<_Float16>(acc[nb][rb][2]);
-                h[3] = static_cast<_Float16>(acc[nb][rb][3]);
-                *reinterpret_cast<half4*>(o + static_cast<size_t>(n) * M + rb * 16) = h;
+                *reinterpret_cast<half4*>(o + static_cast<size_t>(n) * M + rb * 16) = to_half4(acc[nb][rb], store);
             }
         }
     }
@@ -664,7 +666,7 @@ __device__ __forceinline__ void spmm_group_body(uint16_t (*const all_tiles)[kTil
                                                 int steps,
                                                 int col0,
                                                 int vmax,
-                                                int pages,
+                                                int store,
                                                 unsigned w,
                                                 unsigned launch)
 {
@@ -844,7 +846,7 @@ __device__ __forceinline__ void spmm_group_body(uint16_t (*const all_tiles)[kTil
                 for (int rb = 0; rb < 8; rb++)
                     acc[nb][rb] += sums[(r * kGroupWaves + wave) * kSums + (nb * 8 + rb) * kLanes + lane_again];
     }
-    if (pages) {  // o is the workspace itself here; this wave's NBW pages follow those of the waves before it
+    if (store == kStorePages) {  // o is the workspace itself here; this wave's NBW pages follow those of the waves before it
         store_pages<NBW>(o, acc, static_cast<int>(threadIdx.x / kLanes) * NBW, N, lane_again, w, launch);
         return;
     }
@@ -855,12 +857,7 @@ __device__ __forceinline__ void spmm_group_body(uint16_t (*const all_tiles)[kTil
         if (n < N) {
 #pragma unroll
             for (int rb = 0; rb < 8; rb++) {
-                half4 h;
-                h[0] = static_cast<_Float16>(acc[nb][rb][0]);
-                h[1] = static_cast<_Float16>(acc[nb][rb][1]);
-                h[2] = static_cast<_Float16>(acc[nb][rb][2]);
-                h[3] = static_cast<_Float16>(acc[nb][rb][3]);
-                *reinterpret_cast<half4*>(o + static_cast<size_t>(n) * M + g * 4 + rb * 16) = h;
+                *reinterpret_cast<half4*>(o + static_cast<size_t>(n) * M + g * 4 + rb * 16) = to_half4(acc[nb][rb], store);
             }
         }
     }
@@ -877,7 +874,7 @@ __global__ __launch_bounds__(kGroupThreads* KS, 3) void spmm_group_kernel(const 
                                                                   int K,
                                                                   int split_k,
                                                                   int col_groups,
-                                                                  int pages,
+                                                                  int store,
                                                                   unsigned units)
 {
     __shared__ __attribute__((aligned(16))) uint16_t tiles[3 * KS][kTileHalfs];
@@ -903,7 +900,7 @@ __global__ __launch_bounds__(kGroupThreads* KS, 3) void spmm_group_kernel(const 
         steps = (tiles_of_slice - 1) / KS + 1;
     }
     const int* toff = offs + static_cast<size_t>(rowtile) * kt;
-    _Float16*  o    = pages ? out : out + static_cast<size_t>(slice) * M * N + static_cast<size_t>(rowtile) * kTileRows;
+    _Float16*  o    = store == kStorePages ? out : out + static_cast<size_t>(slice) * M * N + static_cast<size_t>(rowtile) * kTileRows;
     // last vector any load of this slice may touch (clamped loads re-read it)
     int vmax = toff[ke] - 1;
     vmax     = vmax > 0 ? vmax : 0;
@@ -915,9 +912,9 @@ __global__ __launch_bounds__(kGroupThreads* KS, 3) void spmm_group_kernel(const 
     if (whole == 0)
         comp = reinterpret_cast<const uint4*>(B);
     if (whole <= 440LL * (M / kTileRows) * kt)
-        spmm_group_body<NBW, 2, KS>(tiles, comp, toff, B, ldb, o, M, N, K, kb, ke, steps, col0, vmax, pages, place.w, units * split_k);
+        spmm_group_body<NBW, 2, KS>(tiles, comp, toff, B, ldb, o, M, N, K, kb, ke, steps, col0, vmax, store, place.w, units * split_k);
     else
-        spmm_group_body<NBW, 3, KS>(tiles, comp, toff, B, ldb, o, M, N, K, kb, ke, steps, col0, vmax, pages, place.w, units * split_k);
+        spmm_group_body<NBW, 3, KS>(tiles, comp, toff, B, ldb, o, M, N, K, kb, ke, steps, col0, vmax, store, place.w, units * split_k);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -954,7 +951,7 @@ __device__ __forceinline__ void spmm_wide_body(unsigned char* lds,
                                                int ke,
                                                int col0,
                                                int vmax,
-                                               int pages,
+                                               int store,
                                                unsigned w,
                                                unsigned launch)
 {
@@ -1102,7 +1099,7 @@ __device__ __forceinline__ void spmm_wide_body(unsigned char* lds,
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may land in LDS that is no longer this workgroup's
 
-    if (pages) {
+    if (store == kStorePages) {
         store_pages<NBW>(o, acc, wave * NBW, 16 * NBW, lane, w, launch);
         return;
     }
@@ -1111,11 +1108,7 @@ __device__ __forceinline__ void spmm_wide_body(unsigned char* lds,
         const int n = col0 + (wave * NBW + nb) * 16 + r16;
 #pragma unroll
         for (int rb = 0; rb < 8; rb++) {
-            half4 h;
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                h[e] = static_cast<_Float16>(acc[nb][rb][e]);
-            *reinterpret_cast<half4*>(o + static_cast<size_t>(n) * M + g * 4 + rb * 16) = h;
+            *reinterpret_cast<half4*>(o + static_cast<size_t>(n) * M + g * 4 + rb * 16) = to_half4(acc[nb][rb], store);
         }
     }
 }
@@ -1130,7 +1123,7 @@ __global__ __launch_bounds__(kWideWaves* kLanes, 2) void spmm_wide_kernel(const 
                                                                  int K,
                                                                  int split_k,
                                                                  int col_groups,
-                                                                 int pages,
+                                                                 int store,
                                                                  unsigned units)
 {
     __shared__ __attribute__((aligned(16))) unsigned char lds[kWideWaves * 8192 + 3 * kTileHalfs * 2];
@@ -1148,16 +1141,16 @@ __global__ __launch_bounds__(kWideWaves* kLanes, 2) void spmm_wide_kernel(const 
     int ke        = kb + avg;
     ke            = ke < kt ? ke : kt;
     const int* toff = offs + static_cast<size_t>(rowtile) * kt;
-    _Float16*  o    = pages ? out : out + static_cast<size_t>(slice) * M * N + static_cast<size_t>(rowtile) * kTileRows;
+    _Float16*  o    = store == kStorePages ? out : out + static_cast<size_t>(slice) * M * N + static_cast<size_t>(rowtile) * kTileRows;
     int vmax = toff[ke] - 1;
     vmax     = vmax > 0 ? vmax : 0;
     const int whole = offs[static_cast<size_t>(M / kTileRows) * kt];
     if (whole == 0)
         comp = reinterpret_cast<const uint4*>(B);
     if (whole <= 440LL * (M / kTileRows) * kt)
-        spmm_wide_body<2>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, vmax, pages, place.w, units * split_k);
+        spmm_wide_body<2>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, vmax, store, place.w, units * split_k);
     else
-        spmm_wide_body<3>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, vmax, pages, place.w, units * split_k);
+        spmm_wide_body<3>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, vmax, store, place.w, units * split_k);
 }
 
 __device__ __forceinline__ void add_slab(float (&s)[4], const uint2 v)
@@ -1294,18 +1287,6 @@ __global__ __launch_bounds__(kLanes) void xcd_probe_kernel(unsigned* __restrict_
         out[w] = __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11));  // XCC_ID, bits 3:0
 }
 
-__global__ __launch_bounds__(256) void relu_kernel(uint4* __restrict__ x, long n8)
-{
-    const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= n8)
-        return;
-    half8 h = __builtin_bit_cast(half8, x[i]);
-#pragma unroll
-    for (int j = 0; j < 8; j++)
-        h[j] = h[j] > static_cast<_Float16>(0) ? h[j] : static_cast<_Float16>(0);  // NaN -> 0 like max(x, 0)
-    x[i] = __builtin_bit_cast(uint4, h);
-}
-
 __global__ __launch_bounds__(256) void take_rows_kernel(uint4* __restrict__ dst, const uint4* __restrict__ src, int rows8, int cols, int ld8)
 {
     const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
@@ -1316,7 +1297,7 @@ __global__ __launch_bounds__(256) void take_rows_kernel(uint4* __restrict__ dst,
 }
 
 template<int NB, int DEPTH, int W, int G, int KS>
-int launch_spmm(hipStream_t stream, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int col_groups, int pages)
+int launch_spmm(hipStream_t stream, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int col_groups, int store)
 {
     const unsigned units = (static_cast<unsigned>(m / kTileRows) + W - 1) / W * col_groups;
     hipLaunchKernelGGL((spmm_stream_kernel<NB, DEPTH, W, G, KS>),
@@ -1334,19 +1315,19 @@ int launch_spmm(hipStream_t stream, const void* comp, const int* offs, const voi
                        k,
                        split_k,
                        col_groups,
-                       pages,
+                       store,
                        units);
     return static_cast<int>(hipGetLastError());
 }
 
 template<int KS>
-int launch_by_columns(hipStream_t s, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int pages)
+int launch_by_columns(hipStream_t s, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int store)
 {
     if (n <= 16)
-        return launch_spmm<1, 8, 1, 1, KS>(s, comp, offs, b, ldb, out, m, n, k, split_k, 1, pages);
+        return launch_spmm<1, 8, 1, 1, KS>(s, comp, offs, b, ldb, out, m, n, k, split_k, 1, store);
     if (n == 32)
-        return launch_spmm<2, 8, 1, 1, KS>(s, comp, offs, b, ldb, out, m, n, k, split_k, 1, pages);
-    return launch_spmm<4, 6, 1, 1, KS>(s, comp, offs, b, ldb, out, m, n, k, split_k, n / 64, pages);
+        return launch_spmm<2, 8, 1, 1, KS>(s, comp, offs, b, ldb, out, m, n, k, split_k, 1, store);
+    return launch_spmm<4, 6, 1, 1, KS>(s, comp, offs, b, ldb, out, m, n, k, split_k, n / 64, store);
 }
 
 // Row tiles per workgroup of the launch for B of n columns, A of m rows and split_k slices: 8 (a CU's eight waves
@@ -1432,21 +1413,21 @@ extern "C" int flashllm_hip_static_workspace(void** ptr)
     return 0;
 }
 
-// pages != 0 (Split_K > 1 only): the slabs go to the workspace by workgroup, for flashllm_hip_launch_reduce_pages
+// pages and the slabs of a Split_K > 1, max(., 0) only with Split_K == 1
 extern "C" int flashllm_hip_launch_spmm(
-    void* stream, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int pages, int k_waves)
+    void* stream, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int store, int k_waves)
 {
     hipStream_t s = static_cast<hipStream_t>(stream);
-    pages         = pages && split_k > 1;
+    store         = split_k > 1 ? store == kStorePages : store & kStoreRelu;
     if (n == 64 && rows_per_workgroup(n, m, split_k) == 8)
-        return launch_spmm<4, 8, 8, 2, 1>(s, comp, offs, b, ldb, out, m, n, k, split_k, 1, pages);
+        return launch_spmm<4, 8, 8, 2, 1>(s, comp, offs, b, ldb, out, m, n, k, split_k, 1, store);
     if (k_waves == 8)
-        return launch_by_columns<8>(s, comp, offs, b, ldb, out, m, n, k, split_k, pages);
+        return launch_by_columns<8>(s, comp, offs, b, ldb, out, m, n, k, split_k, store);
     if (k_waves == 4)
-        return launch_by_columns<4>(s, comp, offs, b, ldb, out, m, n, k, split_k, pages);
+        return launch_by_columns<4>(s, comp, offs, b, ldb, out, m, n, k, split_k, store);
     if (k_waves == 2)
-        return launch_by_columns<2>(s, comp, offs, b, ldb, out, m, n, k, split_k, pages);
-    return launch_by_columns<1>(s, comp, offs, b, ldb, out, m, n, k, split_k, pages);
+        return launch_by_columns<2>(s, comp, offs, b, ldb, out, m, n, k, split_k, store);
+    return launch_by_columns<1>(s, comp, offs, b, ldb, out, m, n, k, split_k, store);
 }
 
 extern "C" void flashllm_hip_set_rows_per_workgroup(int rows)
@@ -1471,7 +1452,7 @@ extern "C" double flashllm_hip_wide_b_step(int n, int m, int split_k)
 }
 
 extern "C" int flashllm_hip_launch_spmm_group(
-    void* stream, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int pages, int runs)
+    void* stream, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int store, int runs)
 {
     const int       cols  = columns_per_workgroup(n, m, split_k);
     const unsigned  units = static_cast<unsigned>(m / kTileRows) * (n / cols);
@@ -1480,13 +1461,13 @@ extern "C" int flashllm_hip_launch_spmm_group(
     const uint4*    cp    = static_cast<const uint4*>(comp);
     const _Float16* bp    = static_cast<const _Float16*>(b);
     _Float16*       op    = static_cast<_Float16*>(out);
-    pages                 = pages && split_k > 1;
+    store                 = split_k > 1 ? store == kStorePages : store & kStoreRelu;
     if (cols == kWideCols)
-        hipLaunchKernelGGL(spmm_wide_kernel, grid, dim3(kWideWaves * kLanes), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / cols, pages, units);
+        hipLaunchKernelGGL(spmm_wide_kernel, grid, dim3(kWideWaves * kLanes), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / cols, store, units);
     else if (runs == kSliceRuns)
-        hipLaunchKernelGGL((spmm_group_kernel<2, kSliceRuns>), grid, dim3(kGroupThreads * kSliceRuns), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, pages, units);
+        hipLaunchKernelGGL((spmm_group_kernel<2, kSliceRuns>), grid, dim3(kGroupThreads * kSliceRuns), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, store, units);
     else
-        hipLaunchKernelGGL((spmm_group_kernel<2, 1>), grid, dim3(kGroupThreads), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, pages, units);
+        hipLaunchKernelGGL((spmm_group_kernel<2, 1>), grid, dim3(kGroupThreads), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, store, units);
     return static_cast<int>(hipGetLastError());
 }
 
@@ -1532,14 +1513,6 @@ extern "C" int flashllm_hip_launch_xcd_probe(void* stream, unsigned* out, int wo
         return static_cast<int>(hipErrorInvalidValue);
     const dim3 grid(kXcds, 3, (static_cast<unsigned>(workgroups) + 3 * kXcds - 1) / (3 * kXcds));
     hipLaunchKernelGGL(xcd_probe_kernel, grid, dim3(kLanes), 0, static_cast<hipStream_t>(stream), out, static_cast<unsigned>(workgroups));
-    return static_cast<int>(hipGetLastError());
-}
-
-extern "C" int flashllm_hip_launch_relu(void* stream, void* x, long n)
-{
-    const long n8 = n / 8;
-    hipLaunchKernelGGL(relu_kernel, dim3(static_cast<unsigned>((n8 + 255) / 256)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), static_cast<uint4*>(x), n8);
     return static_cast<int>(hipGetLastError());
 }
 

@@ -19,8 +19,9 @@ int flashllm_hip_static_workspace(void** ptr);
 
 // out: C when split_k == 1, else the slab workspace (split_k * M * N halfs).
 // pages == 0: slab s is M*N halfs at s*M*N, laid out like C (for flashllm_hip_launch_reduce);
-// pages != 0: each workgroup's 128 x 16 blocks of partial sums as 4 KB pages in workgroup order
+// pages == 1: each workgroup's 128 x 16 blocks of partial sums as 4 KB pages in workgroup order
 // (for flashllm_hip_launch_reduce_pages; needs out 16-byte aligned).
+// pages == 2, split_k == 1: C through max(., 0), the activation between FFN1 and FFN2.
 // ldb: halfs between consecutive columns of B (>= K, a multiple of 8; K for a dense column-major B).
 // k_waves: 1, 2, 4 or 8 waves per workgroup divide each (row tile, slice) among themselves along K (ignored by a
 // launch that takes eight row tiles per workgroup, below).
@@ -79,9 +80,6 @@ int flashllm_hip_launch_reduce_pages(void* stream, void* c, const void* ws, int 
 // SpMM launches (a three-dimensional grid, eight wide, w counted x first, then y, then z): shows whether the
 // round-robin hand-out in that order, which the placement above counts on, holds on this machine.
 int flashllm_hip_launch_xcd_probe(void* stream, unsigned* out, int workgroups);
-
-// x[i] = max(x[i], 0) over n halfs (n % 8 == 0): the activation between FFN1 and FFN2.
-int flashllm_hip_launch_relu(void* stream, void* x, long n);
 
 // dst[j*rows + i] = src[j*src_ld + i] for i < rows, j < cols (rows % 8 == 0, src_ld % 8 == 0).
 int flashllm_hip_launch_take_rows(void* stream, void* dst, const void* src, int rows, int cols, int src_ld);

@@ -53,3 +53,31 @@ def test_256_columns_match_the_one_wave_kernel(product, m, k, n, split_k, sparsi
         got = plain.view(split_k, n, m)[:, part * 64:(part + 1) * 64]
         assert bool(torch.isfinite(want).all())
         assert torch.equal(got.reshape(-1).view(torch.int16), want.view(torch.int16)), part
+
+
+@pytest.mark.parametrize("tokens,ffn", [(8, 1024), (32, 1024), (64, 1024), (64, 25600), (128, 1024), (256, 4096), (512, 25600)])
+@pytest.mark.parametrize("split_k", [1, 2])
+def test_activation_is_stored_with_the_sums(product, tokens, ffn, split_k):
+    """FFN1's ReLU in every kernel that can store its sums (several waves or one per slice, groups of four waves, three
+    such groups, 256 columns) and in the reduction."""
+    import torch
+
+    print(f"activation tokens={tokens} ffn={ffn} split_k={split_k}", flush=True)
+    hidden = 2048 if ffn <= 4096 else 256
+
+    def weight(m, k, seed):
+        return product.SparseWeight(synth.sparse_matrix(m, k, 0.8, seed, dist="normal", sigma=0.05, threads=8), split_k=split_k)
+
+    layer = product.DecoderLayer(weight(3 * hidden, hidden, 1), weight(hidden, hidden, 2), weight(ffn, hidden, 3), weight(hidden, ffn, 4))
+    x = torch.from_numpy(synth.dense_b(hidden, tokens, 98, dist="normal")).cuda().view(-1)
+    x[:hidden] = float("nan")  # a column of NaN: 0 behind the activation
+    ws = torch.empty(split_k * max(3 * hidden, ffn) * tokens, dtype=torch.float16, device="cuda")
+    _, (_, _, attn_out, ffn_mid, _) = layer.forward(x, tokens, workspace=ws)
+    used = 1 if tokens > 128 else split_k
+    want = torch.empty_like(ffn_mid)
+    w = layer.weights[2]
+    product.spmm_splitk(w.comp, w.offs, attn_out, want, w.m, tokens, w.k, ws, used)
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(want[:w.m]).all()) and bool((want[w.m:] < 0).any())
+    want = torch.where(want > 0, want, torch.zeros_like(want))
+    assert torch.equal(ffn_mid.view(torch.int16), want.view(torch.int16))
