@@ -925,17 +925,23 @@ __global__ __launch_bounds__(kGroupThreads* KS, 3) void spmm_group_kernel(const 
 // (l % 8) ^ (l / 8) of a line to slot l % 8) go straight from memory to 8 KB of LDS that belong to the wave, requested
 // as soon as the previous tile's have been read out, i.e. a whole step ahead, and without a meeting.  Fetched in the
 // operand layout instead, where neighbouring lanes hold neighbouring columns, the loads themselves are the bound: 9.7
-// TB/s out of L2 against 32 with neighbouring lanes on one line (256 columns x 7168, all CUs; in this kernel 231 against
-// 206 us at 28672 x 7168, N = 512).
-// A wave's tile is taken in quarters, the reads of one ahead of the MFMAs of the one before; the order is fixed by
-// scheduling barriers, because left alone the reads sink to their first use and because two waits count on it:
-//   * vmcnt(R) at the head of a step: the R loads of the stream, which request() puts behind the fetch of B, are the
-//     only younger ones;
-//   * the statement that names every fragment of B in front of the next fetch: they are out of LDS.
-// 80 KB of LDS, two workgroups per CU.  A step takes 1.15 us alone on a CU and 1.78 us for two, where the four-wave
-// kernel above takes 0.76 / 1.13 / 1.6 us for one / two / three workgroups with half the columns.  Measured, 80 %:
-// 28672 x 7168, N = 512, Split_K 1 246 -> 206 us, 21504 x 7168, N = 512 182 (Split_K 1) -> 163 (3), 36864 x 9216,
-// N = 256 206 -> 192, 7168 x 28672, N = 512 262 (2) -> 216 (4).
+// TB/s out of L2 against 32 with neighbouring lanes on one line (256 columns x 7168, all CUs; 231 against 206 us in an
+// earlier form of this kernel at 28672 x 7168, N = 512).
+// A wave's tile is taken in quarters, the reads of one ahead of the MFMAs of the one before, in an order that scheduling
+// barriers fix (left alone the reads sink to their first use).  What a step asks of global memory is waited for at the
+// head of the next: the lines of B right after this tile's are out of LDS (the statement that names every fragment),
+// then, behind the first quarter's MFMAs, the wave's part of the stream two tiles on.  Both are asked for early and
+// needed a step later, so the wait is for everything and the scatter waits for nothing; the stream behind B, because B
+// is the longer fetch (the other order 213 us where this one takes 206, and with the stream asked for at the end of a
+// step and waited for in the scatter of the next, which then waits for the younger B too, 202).  28672 x 7168, N = 512, Split_K 1
+// with the requests of the stream one quarter earlier / later: 195 / 189 us, B asked for before / after the second
+// quarter's reads 188 / 186, clearing or scattering before the third quarter 198 .. 209.
+// 80 KB of LDS, two workgroups per CU.  A step takes 1.16 us alone on a CU and 1.64 us for two, where the four-wave
+// kernel above takes 0.76 / 1.13 / 1.6 us for one / two / three workgroups with half the columns.  The bound is LDS (144
+// KB to and from registers per tile and workgroup, about 0.6 us) beside the MFMAs (0.43 us), which the meetings keep
+// from overlapping fully.  Measured against the four-wave kernel, 80 %: 28672 x 7168, N = 512, Split_K 1 246 -> 186 us,
+// 21504 x 7168, N = 512 182 (Split_K 1) -> 152 (3), 36864 x 9216, N = 256 206 -> 176 (5), 7168 x 28672, N = 512 262
+// (2) -> 198 (4).
 constexpr int kWideWaves = 4;
 constexpr int kWideCols  = kWideWaves * 64;
 
@@ -990,33 +996,41 @@ __device__ __forceinline__ void spmm_wide_body(unsigned char* lds,
         for (int nb = 0; nb < NBW; nb++)
             bfrag[ks][nb] = *reinterpret_cast<const half8*>(bwin + nb * 2048 + (ks ? a_off1 : a_off0));
     };
-    uint4 ring[R];
-    int   ring_lo, ring_n;
+    struct Ring {
+        uintx4 v[R];
+        int    lo, n;
+    };
+    Ring  here, coming;
     int   ahead_lo = toff[kb], ahead_hi = toff[kb + 1 < ke ? kb + 1 : ke];  // range of the tile the next request is for
-    auto  request = [&](int t) {  // this wave's part of tile t (empty past the end), always issued
-        ring_lo           = ahead_lo;
-        ring_n            = ahead_hi - ahead_lo;
-        const uint4* from = comp;
-        asm volatile("" : "+s"(from)::"memory");  // behind the fetch of B
+    auto  request = [&](Ring& ring) {  // this wave's part of that tile (empty past the end), always issued
+        ring.lo           = ahead_lo;
+        ring.n            = ahead_hi - ahead_lo;
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            int v   = ring_lo + (r * NW + wave) * kLanes + lane;
-            v       = v < vmax ? v : vmax;
-            ring[r] = load_stream(from + v);
+            int v     = ring.lo + (r * NW + wave) * kLanes + lane;
+            v         = v < vmax ? v : vmax;
+            ring.v[r] = __builtin_bit_cast(uintx4, load_stream(comp + v));
         }
+    };
+    auto look_ahead = [&](int t) {  // behind the request for tile t
         ahead_lo = ahead_hi;
         ahead_hi = toff[t + 2 < ke ? t + 2 : ke];
     };
-    auto scatter = [&](int buf) {
+    auto landed = [&](Ring& ring) {  // the compiler's wait for these loads goes here instead of to their first use
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            asm volatile("" : "+v"(ring.v[r])::"memory");
+    };
+    auto scatter = [&](int buf, const Ring& ring) {
         uint16_t* tile = reinterpret_cast<uint16_t*>(tiles + buf);
 #pragma unroll
         for (int r = 0; r < R; r++)
-            if ((r * NW + wave) * kLanes + lane < ring_n)
-                scatter_vector(tile, ring[r]);
-        for (int r = R; r * kThreads < ring_n; r++) {  // a tile longer than R rounds: the rest straight from memory
+            if ((r * NW + wave) * kLanes + lane < ring.n)
+                scatter_vector(tile, __builtin_bit_cast(uint4, ring.v[r]));
+        for (int r = R; r * kThreads < ring.n; r++) {  // a tile longer than R rounds: the rest straight from memory
             const int i = (r * NW + wave) * kLanes + lane;
-            if (i < ring_n)
-                scatter_vector(tile, load_stream(comp + ring_lo + i));
+            if (i < ring.n)
+                scatter_vector(tile, load_stream(comp + ring.lo + i));
         }
     };
     auto clear_part = [&](int buf) {
@@ -1053,42 +1067,49 @@ __device__ __forceinline__ void spmm_wide_body(unsigned char* lds,
     auto keep_in_order = [&]() { __builtin_amdgcn_sched_barrier(0); };
 
     int cur = 0, next = kTileBytes, old = 2 * kTileBytes;
-    request(kb);
+    request(here);
+    look_ahead(kb);
     fetch_b(kb);
     clear_part(cur);
     clear_part(next);
     meet();
-    scatter(cur);
-    request(kb + 1);
+    scatter(cur, here);
+    request(coming);
+    look_ahead(kb + 1);
     meet();
     for (int t = kb; t < ke; t++) {
-        // this tile's lines of B have landed: only the R loads of the stream are younger
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R) : "memory");
+        // this tile's lines of B and the stream's part of the next tile were requested a step ago
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        landed(coming);
+        here = coming;
         read_b(0);
         read_b(1);
         read_a(q0, cur);
         keep_in_order();
         // ... and are in registers before the next tile's may overwrite them
         asm volatile("" ::"v"(bfrag[0][0]), "v"(bfrag[0][1]), "v"(bfrag[0][2]), "v"(bfrag[0][3]), "v"(bfrag[1][0]), "v"(bfrag[1][1]), "v"(bfrag[1][2]), "v"(bfrag[1][3]) : "memory");
+        read_a(q1, cur);
+        keep_in_order();
         if (t + 1 < ke)
             fetch_b(t + 1);
         keep_in_order();
-        read_a(q1, cur);
-        keep_in_order();
         multiply(q0);
+        keep_in_order();
+        request(coming);  // tile t + 2
         keep_in_order();
         read_a(q2, cur);
         keep_in_order();
         multiply(q1);
         keep_in_order();
         read_a(q3, cur);
+        keep_in_order();
         clear_part(old);
         keep_in_order();
         multiply(q2);
         keep_in_order();
-        scatter(next);  // tile t + 1 (empty past the end)
+        scatter(next, here);  // tile t + 1 (empty past the end)
         keep_in_order();
-        request(t + 2);
+        look_ahead(t + 2);
         keep_in_order();
         multiply(q3);
         meet();
@@ -1358,7 +1379,7 @@ int rows_per_workgroup(int n, int m, int split_k)
 // (spmm_wide_kernel, two), by the time of a step with the workgroups that share a CU (us, fitted to 36864 x 9216,
 // 21504 x 7168, 28672 x 7168 and 7168 x 28672 at N = 256 / 512 and Split_K 1 .. 4), beyond a full round the whole rounds and
 // what the rest of the last one adds.  The four-wave kernel wins where 256 columns would leave CUs to one workgroup
-// or none (21504 x 7168, N = 512, Split_K 1: 182 against 203 us).
+// or none (7168 x 28672, N = 512, Split_K 2, 224 workgroups of 256 columns: 258 against 261 us).
 double group_step(long workgroups)
 {
     if (workgroups <= 768)
@@ -1370,9 +1391,9 @@ double group_step(long workgroups)
 double wide_step(long workgroups)
 {
     if (workgroups <= 512)
-        return workgroups <= 256 ? 1.15 : 1.78;
+        return workgroups <= 256 ? 1.15 : 1.64;
     const long rest = workgroups % 512;
-    return 1.78 * (workgroups / 512 + (rest == 0 ? 0.0 : rest <= 256 ? 0.6 : 1.0));
+    return 1.64 * (workgroups / 512 + (rest == 0 ? 0.0 : rest <= 256 ? 0.6 : 1.0));
 }
 
 int columns_per_workgroup(int n, int m, int split_k)
