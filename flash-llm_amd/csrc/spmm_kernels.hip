@@ -656,21 +656,12 @@ __global__ __launch_bounds__(kLanes* W* KS) void spmm_stream_kernel(const uint4*
 // places are exact counts that never drain the stream, and the accumulators stay where they are (with early
 // exits from the unrolled round the register allocation more than doubled).  A tile with more than R*256
 // vectors takes its remaining rounds on a slow path.
-//
-// KS > 1: KS such groups of four waves form one workgroup and divide the slice's k tiles in KS consecutive runs, each
-// with its own three tile buffers (3 x 48 KB of LDS: the CU's).  Nothing but the meetings is shared until the end,
-// when the first group adds the others' accumulators to its own, in fp32 and in the order of k, through LDS.  It is
-// for launches of at most one workgroup per CU, which a caller's Split_K can ask for: the step is a chain of waits
-// that one group leaves unfilled.  Split_K = 1, 80 %: 7168 x 28672, N = 512 340 -> 258 us, 7168 x 7168, N = 512
-// 91 -> 73, 2048 x 8192, N = 384 102 -> 81; with more than one workgroup per CU it loses what the meetings couple
-// (36864 x 9216, N = 128 166 -> 172).
-constexpr int kSliceRuns    = 3;
 constexpr int kGroupWaves   = 4;
 constexpr int kGroupThreads = kGroupWaves * kLanes;
 constexpr int kAhead        = 3;  // tiles of the stream in flight per wave = the three buffers' rotation
 
-template<int NBW, int R, int KS>
-__device__ __forceinline__ void spmm_group_body(uint16_t (*const all_tiles)[kTileHalfs],
+template<int NBW, int R>
+__device__ __forceinline__ void spmm_group_body(uint16_t (*const tiles)[kTileHalfs],
                                                 const uint4* __restrict__ comp,
                                                 const int* __restrict__ toff,
                                                 const _Float16* __restrict__ B,
@@ -681,16 +672,14 @@ __device__ __forceinline__ void spmm_group_body(uint16_t (*const all_tiles)[kTil
                                                 int K,
                                                 int kb,
                                                 int ke,
-                                                int steps,
                                                 int col0,
                                                 int vmax,
                                                 int store,
                                                 unsigned w,
                                                 unsigned launch)
 {
-    uint16_t (*const tiles)[kTileHalfs] = all_tiles + (KS > 1 ? threadIdx.x / kGroupThreads * 3 : 0);
     const int lane = threadIdx.x & (kLanes - 1);
-    const int wave = KS > 1 ? threadIdx.x / kLanes % kGroupWaves : threadIdx.x / kLanes;
+    const int wave = threadIdx.x / kLanes;
 
     floatx4 acc[NBW][8];
 #pragma unroll
@@ -732,7 +721,7 @@ __device__ __forceinline__ void spmm_group_body(uint16_t (*const all_tiles)[kTil
         }
     };
     auto load_b = [&](int t) {  // always issued: past the end the last tile's lines are fetched again
-        const int tc = t < ke ? t : (KS > 1 && ke == 0 ? 0 : ke - 1);
+        const int tc = t < ke ? t : ke - 1;
 #pragma unroll
         for (int i = 0; i < 2 * NBW; i++)
             braw[i] = *reinterpret_cast<const uintx4*>(bptr + static_cast<size_t>(i) * 8 * ldb + tc * kTileCols);
@@ -828,8 +817,7 @@ __device__ __forceinline__ void spmm_group_body(uint16_t (*const all_tiles)[kTil
         clear_quarter(tiles[(j + 2) % 3]);
         meet();
     };
-    const int end = KS > 1 ? kb + steps : ke;
-    for (int t = kb; t < end; t += kAhead) {
+    for (int t = kb; t < ke; t += kAhead) {
         step(std::integral_constant<int, 0>{}, t);
         step(std::integral_constant<int, 1>{}, t + 1);
         step(std::integral_constant<int, 2>{}, t + 2);
@@ -842,28 +830,6 @@ __device__ __forceinline__ void spmm_group_body(uint16_t (*const all_tiles)[kTil
     // coordinates are derived afresh (through an opaque statement) so that nothing is carried round the loop for this.
     int lane_again = threadIdx.x & (kLanes - 1);
     asm volatile("" : "+v"(lane_again));
-    if constexpr (KS > 1) {
-        // the runs' sums meet in the first run's waves: everybody is past its last read of a tile (the last meeting)
-        constexpr int kSums = NBW * 8 * kLanes;
-        floatx4*      sums  = reinterpret_cast<floatx4*>(&all_tiles[0][0]);
-        const int     run   = threadIdx.x / kGroupThreads;
-        if (run > 0)
-#pragma unroll
-            for (int nb = 0; nb < NBW; nb++)
-#pragma unroll
-                for (int rb = 0; rb < 8; rb++)
-                    sums[((run - 1) * kGroupWaves + wave) * kSums + (nb * 8 + rb) * kLanes + lane_again] = acc[nb][rb];
-        __syncthreads();
-        if (run > 0)
-            return;
-#pragma unroll
-        for (int r = 0; r < KS - 1; r++)
-#pragma unroll
-            for (int nb = 0; nb < NBW; nb++)
-#pragma unroll
-                for (int rb = 0; rb < 8; rb++)
-                    acc[nb][rb] += sums[(r * kGroupWaves + wave) * kSums + (nb * 8 + rb) * kLanes + lane_again];
-    }
     if (store == kStorePages) {  // o is the workspace itself here; this wave's NBW pages follow those of the waves before it
         store_pages<NBW>(o, acc, static_cast<int>(threadIdx.x / kLanes) * NBW, N, lane_again, w, launch);
         return;
@@ -881,8 +847,8 @@ __device__ __forceinline__ void spmm_group_body(uint16_t (*const all_tiles)[kTil
     }
 }
 
-template<int NBW, int KS>
-__global__ __launch_bounds__(kGroupThreads* KS, 3) void spmm_group_kernel(const uint4* __restrict__ comp,
+template<int NBW>
+__global__ __launch_bounds__(kGroupThreads, 3) void spmm_group_kernel(const uint4* __restrict__ comp,
                                                                   const int* __restrict__ offs,
                                                                   const _Float16* __restrict__ B,
                                                                   int ldb,
@@ -895,28 +861,20 @@ __global__ __launch_bounds__(kGroupThreads* KS, 3) void spmm_group_kernel(const 
                                                                   int store,
                                                                   unsigned units)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t tiles[3 * KS][kTileHalfs];
+    __shared__ __attribute__((aligned(16))) uint16_t tiles[3][kTileHalfs];
     const int   kt    = K / kTileCols;
     const Place place = place_of_workgroup(units, split_k);
     if (!place.valid)
         return;
     const int unit = place.unit, slice = place.part;
     const int rowtile = unit / col_groups;
-    const int col0    = (unit % col_groups) * (kGroupWaves * 16 * NBW) + (threadIdx.x / kLanes % kGroupWaves) * (16 * NBW);
+    const int col0    = (unit % col_groups) * (kGroupWaves * 16 * NBW) + (threadIdx.x / kLanes) * (16 * NBW);
     // the reference's slicing (csrc/SpMM_Kernel.cuh:196-204), clamped to K
     const int avg = (kt - 1) / split_k + 1;
     int       kb  = slice * avg;
     kb            = kb < kt ? kb : kt;
     int ke        = kb + avg;
     ke            = ke < kt ? ke : kt;
-    int steps = ke - kb;  // every wave's, also one whose run is a tile shorter
-    if constexpr (KS > 1) {
-        const int tiles_of_slice = ke - kb, base = kb;
-        const int run = __builtin_amdgcn_readfirstlane(threadIdx.x / kGroupThreads);
-        kb    = base + tiles_of_slice * run / KS;
-        ke    = base + tiles_of_slice * (run + 1) / KS;
-        steps = (tiles_of_slice - 1) / KS + 1;
-    }
     const int* toff = offs + static_cast<size_t>(rowtile) * kt;
     _Float16*  o    = store == kStorePages ? out : out + static_cast<size_t>(slice) * M * N + static_cast<size_t>(rowtile) * kTileRows;
     // last vector any load of this slice may touch (clamped loads re-read it)
@@ -930,9 +888,9 @@ __global__ __launch_bounds__(kGroupThreads* KS, 3) void spmm_group_kernel(const 
     if (whole == 0)
         comp = reinterpret_cast<const uint4*>(B);
     if (whole <= 440LL * (M / kTileRows) * kt)
-        spmm_group_body<NBW, 2, KS>(tiles, comp, toff, B, ldb, o, M, N, K, kb, ke, steps, col0, vmax, store, place.w, units * split_k);
+        spmm_group_body<NBW, 2>(tiles, comp, toff, B, ldb, o, M, N, K, kb, ke, col0, vmax, store, place.w, units * split_k);
     else
-        spmm_group_body<NBW, 3, KS>(tiles, comp, toff, B, ldb, o, M, N, K, kb, ke, steps, col0, vmax, store, place.w, units * split_k);
+        spmm_group_body<NBW, 3>(tiles, comp, toff, B, ldb, o, M, N, K, kb, ke, col0, vmax, store, place.w, units * split_k);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1190,6 +1148,383 @@ __global__ __launch_bounds__(kWideWaves* kLanes, 2) void spmm_wide_kernel(const 
         spmm_wide_body<2>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, vmax, store, place.w, units * split_k);
     else
         spmm_wide_body<3>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, vmax, store, place.w, units * split_k);
+}
+
+// ------------------------------------------------------------------------------------------------
+// spmm_quarter_kernel: N a multiple of 128, for slices that are long and launches that leave the two kernels above with one
+// or two workgroups per CU.  Both are bound by LDS: a tile of 128 columns takes about 1200 clocks of it in the four-wave kernel, of which
+// the four waves' reads of the same 16 KB of operands are 512, and their meetings keep the MFMAs from filling the gaps.
+// Here a workgroup's four waves divide the slice along K and never meet before the end: a wave scatters its own tiles and
+// multiplies each by all 128 columns, 4 x 4 blocks of 32 x 32 in 256 accumulation registers, so that an operand is read
+// once and feeds four MFMAs.  One wave per SIMD has to do by itself what others do by turns: everything that is not an
+// MFMA is dealt out between them in program order, at most about one LDS instruction (a 16-byte store takes a lone wave 30
+// clocks to issue, a 2-byte store 14) per 32-clock MFMA, and scheduling barriers keep it there.  The MFMAs are inline
+// assembly on accumulators that may not move.
+//   * Four phases of sixteen MFMAs per tile: columns 0-63 with k steps 0, 1 and 2, 3 of the tile's four, then columns
+//     64-127.  Phases 3 and 0 take the operands of the next tile / the tile's second half out of LDS and clear behind the
+//     reads, phases 1 and 2 scatter the next tile, and ask for the part of the stream two tiles later.
+//   * B comes as whole 128-byte lines straight into LDS, 64 columns at a time into three rotating windows; what is asked
+//     for in phase 1 (3) of a tile is read from phase 1 (3) of the next one.  Every wait counts exactly what has been asked
+//     for since.
+//   * The ring holds two tiles of the stream (R vectors per lane each, by the matrix's density; a longer tile takes the
+//     rest straight from memory).  With one tile in the ring the compiler's wait before a vector is used, which does not
+//     know of B's loads, also waits for B asked for half a tile ago: 7168 x 28672, N = 512, Split_K 1 240 us, 213 with two.
+//     The loop body is therefore two tiles; an early exit between them makes the compiler move accumulators and spill, so
+//     runs are whole pairs of tiles and an odd one ends with an empty tile, whose B is zeros.
+//   * Lanes past a tile's end load its last vector again and store the same items once more: no masks.
+// 160 KB of LDS and 512 registers: one workgroup per CU.  Measured with the four-wave kernel (where a launch had at most one
+// workgroup per CU, three groups of four waves) and this one, 80 %, Split_K 1: 7168 x 28672, N = 512 247 -> 213 us, 7168 x
+// 7168, N = 512 75 -> 58, N = 128 68 -> 52, 21504 x 7168, N = 384 146 -> 125, N = 512 (256-column kernel) 192 -> 172, 1664 x
+// 27200, N = 128 233 -> 171.  Without loads from memory the first takes 161 us and with nothing but the MFMAs 128: what is
+// left is the latency of B and the stream.  Tried: B through registers and LDS stores 238 us; B's windows by halves of k instead of
+// columns, i.e. 64-byte pieces of lines, 261.
+constexpr int kQuarters      = 4;
+constexpr int kQuarterWindow = 64 * kTileCols * 2;                       // 64 columns of B for one k tile
+constexpr int kQuarterLds    = kTileHalfs * 2 + 3 * kQuarterWindow;      // a wave's: its tile and three windows of B
+using floatx16 = float __attribute__((ext_vector_type(16)));
+
+// what a tile without vectors reads: an item that stores 0 at position 0
+__device__ uint4 g_zero_vector;
+
+template<int R>
+__device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
+                                                  const uint4* __restrict__ comp,
+                                                  const int* __restrict__ toff,
+                                                  const _Float16* __restrict__ B,
+                                                  int ldb,
+                                                  _Float16* __restrict__ o,
+                                                  int M,
+                                                  int kb,
+                                                  int ke,
+                                                  int col0,
+                                                  int store,
+                                                  unsigned w,
+                                                  unsigned launch)
+{
+    using Lds16 = __attribute__((address_space(3))) uint16_t;
+    using Lds128 = __attribute__((address_space(3))) uintx4;
+    using Global = const __attribute__((address_space(1))) char;
+    const int      lane   = threadIdx.x & (kLanes - 1);
+    const int      wave   = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    unsigned char* mine   = lds + wave * (kTileHalfs * 2);
+    const uint32_t tile_l = __builtin_amdgcn_readfirstlane(lds_offset(mine));
+    const uint32_t bwin_l = __builtin_amdgcn_readfirstlane(lds_offset(lds)) + kQuarters * (kTileHalfs * 2) + wave * (3 * kQuarterWindow);
+
+    floatx16 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int e = 0; e < 16; e++)
+                acc[i][j][e] = 0.f;
+
+    if (kb < ke) {
+        const int r32 = lane & 31, hi = lane >> 5;
+        // operand of this lane in k step 0 of a block of 32 rows of the tile, or columns of a window of B; step s: ^ 32 s
+        const uint32_t off   = r32 * (kTileCols * 2) + ((hi ^ (r32 & 7)) << 4);
+        const uint32_t a_off = tile_l + off;
+        uint32_t       b_lane[4];  // where this lane's 16 bytes of 8i columns of B lie, from the first column of the 32
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            b_lane[i] = (static_cast<unsigned>(8 * i + (lane >> 3)) * static_cast<unsigned>(ldb) + (((lane & 7) ^ (lane >> 3)) << 3)) * 2;
+        const _Float16* bcols = B + static_cast<size_t>(col0) * ldb;
+
+        half8    a[4][4], b[2][4];
+        uintx4   ring[2][R];
+        Global*  nothing = (Global*)&g_zero_vector;
+        asm volatile("" : "+s"(nothing));  // its address stays in registers
+        Global*  from;        // the tile that requests are at
+        uint32_t from_last;   // byte of its last vector
+        int      lo[3], n[3]; // first vector and vectors of that tile (2), the one before (1) and the one to scatter (0)
+        int      ahead_lo = toff[kb], ahead_hi = toff[kb + 1];
+
+        auto keep = [&]() { __builtin_amdgcn_sched_barrier(0); };
+        auto next_tile = [&](int t) {  // requests are at tile t from here on; past the end it is empty
+            lo[0] = lo[1], n[0] = n[1];
+            lo[1] = lo[2], n[1] = n[2];
+            lo[2]     = ahead_lo;
+            n[2]      = ahead_hi - ahead_lo;
+            from      = n[2] > 0 ? (Global*)(comp + ahead_lo) : nothing;
+            from_last = n[2] > 0 ? (n[2] - 1) * 16u : 0u;
+            ahead_lo  = ahead_hi;
+            ahead_hi  = toff[t + 2 < ke ? t + 2 : ke];
+        };
+        // Lanes past the tile's end load its last vector again, and store the same items to the same places.
+        auto request = [&](uintx4& slot, int r) {
+            const uint32_t at = lane * 16u + r * (kLanes * 16u);
+            slot = __builtin_nontemporal_load(reinterpret_cast<const __attribute__((address_space(1))) uintx4*>(from + (at < from_last ? at : from_last)));
+        };
+        auto scatter = [&](uint32_t item) {
+            uint32_t position;
+            asm("v_bfe_u32 %0, %1, 16, 13" : "=v"(position) : "v"(item));
+            *reinterpret_cast<Lds16*>(position * 2 + tile_l) = static_cast<uint16_t>(item);
+        };
+        auto scatter_rest = [&]() {  // a tile of more than R chunks: the rest straight from memory
+            for (int v = R * kLanes + lane; v < n[0]; v += kLanes)
+                scatter_vector(reinterpret_cast<uint16_t*>(mine), load_stream(comp + lo[0] + v));
+        };
+        auto read_lds = [&](uint32_t at) { return *reinterpret_cast<const __attribute__((address_space(3))) half8*>(at); };
+        auto read_a   = [&](int s, int i) { a[s][i] = read_lds((a_off ^ (s * 32)) + i * 4096); };
+        auto clear_a  = [&](int s, int i) { *reinterpret_cast<Lds128*>((a_off ^ (s * 32)) + i * 4096) = uintx4{0u, 0u, 0u, 0u}; };
+        // operands of phase p out of its half's window: k step 2 (p % 2) + m / 2, columns 32 (m % 2) .. +31 of the 64
+        auto read_b = [&](int p, uint32_t window, int m) { b[p & 1][m] = read_lds(((off ^ ((2 * (p & 1) + m / 2) * 32)) + window) + (m % 2) * 4096); };
+        // a half: 64 of the 128 columns of a tile's B, as whole lines of eight columns
+        struct Half {
+            Global*  first;
+            size_t   step;  // bytes between 32 columns
+            uint32_t lanes;
+        };
+        auto half_of_b = [&](int half) {  // past the end: zeros (a run of an odd number of tiles ends with an empty one, and Inf and NaN stay out)
+            const bool there = half < 2 * ke;
+            return Half{there ? (Global*)(bcols + (half & 1) * (64 * static_cast<size_t>(ldb)) + (half >> 1) * kTileCols) : nothing,
+                        there ? 64 * static_cast<size_t>(ldb) : 0, there ? ~0u : 0u};
+        };
+        auto fetch_b = [&](const Half& half, uint32_t window, int i) {
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(b_lane[i % 4] & half.lanes), "s"(half.first + (i / 4) * half.step), "s"(window + i * 1024) : "memory", "m0");
+        };
+        auto multiply = [&](int p, int m) {
+            const int s = 2 * (p & 1) + m / 8, i = m / 2 % 4, j = 2 * (p / 2) + m % 2;
+            asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(a[s][i]), "v"(b[p & 1][m / 8 * 2 + m % 2]));
+        };
+        // windows: w0 holds half 0 of the current tile, w1 half 1, w2 half 0 of the next
+        uint32_t w0 = bwin_l, w1 = bwin_l + kQuarterWindow, w2 = bwin_l + 2 * kQuarterWindow;
+
+        // prologue: tile kb in LDS, tiles kb + 1 and kb + 2 in slots 1 and 0 of the ring
+        lo[1] = lo[2] = n[1] = n[2] = 0;
+        next_tile(kb);
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            request(ring[0][r], r);
+        keep();
+        Half first = half_of_b(2 * kb);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            fetch_b(first, w0, i);
+        next_tile(kb + 1);
+        keep();
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            request(ring[1][r], r);
+        keep();
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                clear_a(s, i);
+        first = half_of_b(2 * kb + 1);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            fetch_b(first, w1, i);
+        next_tile(kb + 2);
+        keep();
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                scatter(ring[0][r][e]);
+            request(ring[0][r], r);
+            keep();
+        }
+        if (n[0] > R * kLanes)
+            scatter_rest();
+        keep();
+        first = half_of_b(2 * kb + 2);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            fetch_b(first, w2, i);
+        next_tile(kb + 3);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R + 16) : "memory");
+        keep();
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+            read_b(0, w0, m);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            read_a(i / 4, i % 4);
+        keep();
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            clear_a(i / 4, i % 4);
+        keep();
+
+        constexpr int R0 = (R + 1) / 2, R1 = R - R0;
+        auto tile = [&](auto slot, int t) {
+            uintx4(&next)[R] = ring[decltype(slot)::value];
+            // phase 0: half 0 of B, k steps 0 and 1
+#pragma unroll
+            for (int m = 0; m < 16; m++) {
+                multiply(0, m);
+                if (m < 4)
+                    read_b(1, w0, m);
+                else if (m < 12)
+                    read_a(2 + (m - 4) / 4, m % 4);
+                if (m >= 8)
+                    clear_a(2 + (m - 8) / 4, m % 4);
+                keep();
+            }
+            // phase 1: half 0, k steps 2 and 3.  Half 1 has landed; half 0 is out of LDS
+            asm volatile("" ::"v"(b[1][0]), "v"(b[1][1]), "v"(b[1][2]), "v"(b[1][3]) : "memory");
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + R1) : "memory");
+            const Half b_half1 = half_of_b(2 * t + 3);
+            keep();
+#pragma unroll
+            for (int m = 0; m < 16; m++) {
+                multiply(1, m);
+                if (m < 4)
+                    read_b(2, w1, m);
+                if (m < 8)
+                    fetch_b(b_half1, w0, m);
+#pragma unroll
+                for (int i = m * R0 * 4 / 16; i < (m + 1) * R0 * 4 / 16; i++) {
+                    scatter(next[i / 4][i % 4]);
+                    if (i % 4 == 3)
+                        request(next[i / 4], i / 4);
+                }
+                keep();
+            }
+            // phase 2: half 1, k steps 0 and 1
+#pragma unroll
+            for (int m = 0; m < 16; m++) {
+                multiply(2, m);
+                if (m < 4)
+                    read_b(3, w1, m);
+#pragma unroll
+                for (int i = m * R1 * 4 / 16; i < (m + 1) * R1 * 4 / 16; i++) {
+                    scatter(next[R0 + i / 4][i % 4]);
+                    if (i % 4 == 3)
+                        request(next[R0 + i / 4], R0 + i / 4);
+                }
+                keep();
+            }
+            if (n[0] > R * kLanes)
+                scatter_rest();
+            keep();
+            // phase 3: half 1, k steps 2 and 3.  Half 0 of the next tile has landed; this tile's B is out of LDS
+            asm volatile("" ::"v"(b[1][0]), "v"(b[1][1]), "v"(b[1][2]), "v"(b[1][3]) : "memory");
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + R) : "memory");
+            const Half b_half0 = half_of_b(2 * t + 4);
+            next_tile(t + 4);
+            keep();
+#pragma unroll
+            for (int m = 0; m < 16; m++) {
+                multiply(3, m);
+                if (m < 4)
+                    read_b(0, w2, m);
+                else if (m < 12)
+                    read_a((m - 4) / 4, m % 4);
+                if (m >= 8)
+                    clear_a((m - 8) / 4, m % 4);
+                if (m < 8)
+                    fetch_b(b_half0, w1, m);
+                keep();
+            }
+            // next tile: half 0 is in w2, half 1 on its way to w0, the half 0 after it on its way to w1
+            const uint32_t old = w0;
+            w0 = w2;
+            w2 = w1;
+            w1 = old;
+        };
+        for (int t = kb; t < ke; t += 2) {
+            tile(std::integral_constant<int, 1>{}, t);
+            tile(std::integral_constant<int, 0>{}, t + 1);
+        }
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");  // nothing may land in LDS that other data goes to now; the matrix cores have written back
+    }
+    __syncthreads();
+
+    // Add up: each wave leaves two column blocks of 32 at a time in its own LDS; wave i sums rows 32i .. +31 in the order of k
+    int lane_again = threadIdx.x & (kLanes - 1);
+    asm volatile("" : "+v"(lane_again));
+    const int r32 = lane_again & 31, hi = lane_again >> 5;
+    floatx4*  sums = reinterpret_cast<floatx4*>(lds);
+    constexpr int kPerWave = kQuarterLds / 16;
+#pragma unroll
+    for (int part = 0; part < 2; part++) {
+        if (part)
+            __syncthreads();
+#pragma unroll
+        for (int jj = 0; jj < 2; jj++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    sums[wave * kPerWave + ((jj * 4 + i) * 4 + q) * kLanes + lane_again] =
+                        floatx4{acc[i][2 * part + jj][4 * q], acc[i][2 * part + jj][4 * q + 1], acc[i][2 * part + jj][4 * q + 2], acc[i][2 * part + jj][4 * q + 3]};
+        __syncthreads();
+#pragma unroll
+        for (int jj = 0; jj < 2; jj++) {
+            floatx4 x[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                x[q] = sums[((jj * 4 + wave) * 4 + q) * kLanes + lane_again];
+#pragma unroll
+            for (int v = 1; v < kQuarters; v++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    x[q] += sums[v * kPerWave + ((jj * 4 + wave) * 4 + q) * kLanes + lane_again];
+            const int col = (2 * part + jj) * 32 + r32;  // of the 128; x[q]: rows 32*wave + 8q + 4*hi .. +3
+            if (store == kStorePages) {
+                uint4* page = reinterpret_cast<uint4*>(o) + (static_cast<size_t>(col / 16) * launch + w) * 256 + wave * 64 + (col & 15);
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    const uint2 l = __builtin_bit_cast(uint2, to_half4(x[q], store)), h = __builtin_bit_cast(uint2, to_half4(x[q + 2], store));
+                    page[(2 * q + hi) * 16] = uint4{l.x, l.y, h.x, h.y};
+                }
+            }
+            else {
+                _Float16* at = o + static_cast<size_t>(col0 + col) * M + wave * 32 + hi * 4;
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    *reinterpret_cast<half4*>(at + 8 * q) = to_half4(x[q], store);
+            }
+        }
+    }
+}
+
+__global__ __launch_bounds__(kQuarters* kLanes, 1) void spmm_quarter_kernel(const uint4* __restrict__ comp,
+                                                                   const int* __restrict__ offs,
+                                                                   const _Float16* __restrict__ B,
+                                                                   int ldb,
+                                                                   _Float16* __restrict__ out,
+                                                                   int M,
+                                                                   int N,
+                                                                   int K,
+                                                                   int split_k,
+                                                                   int col_groups,
+                                                                   int store,
+                                                                   unsigned units)
+{
+    __shared__ __attribute__((aligned(16384))) unsigned char lds[kQuarters * kQuarterLds];
+    const int   kt    = K / kTileCols;
+    const Place place = place_of_workgroup(units, split_k);
+    if (!place.valid)
+        return;
+    const int unit = place.unit, slice = place.part;
+    const int rowtile = unit / col_groups;
+    const int col0    = (unit % col_groups) * 128;
+    // slices, the last vector a load may touch and the empty matrix as in spmm_group_kernel
+    const int avg = (kt - 1) / split_k + 1;
+    int       kb  = slice * avg;
+    kb            = kb < kt ? kb : kt;
+    int ke        = kb + avg;
+    ke            = ke < kt ? ke : kt;
+    // the waves' runs: whole pairs of tiles, but for the last one of an odd slice
+    const int pairs = (ke - kb + 1) / 2, base = kb, end = ke;
+    const int run = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    kb            = base + pairs * run / kQuarters * 2;
+    ke            = base + pairs * (run + 1) / kQuarters * 2;
+    ke            = ke < end ? ke : end;
+    const int* toff = offs + static_cast<size_t>(rowtile) * kt;
+    _Float16*  o    = store == kStorePages ? out : out + static_cast<size_t>(slice) * M * N + static_cast<size_t>(rowtile) * kTileRows;
+    const int       whole = offs[static_cast<size_t>(M / kTileRows) * kt];
+    const long long tiles = static_cast<long long>(M / kTileRows) * kt;
+    if (whole <= 236 * tiles)
+        spmm_quarter_body<4>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, store, place.w, units * split_k);
+    else if (whole <= 428 * tiles)
+        spmm_quarter_body<7>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, store, place.w, units * split_k);
+    else
+        spmm_quarter_body<10>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, store, place.w, units * split_k);
 }
 
 __device__ __forceinline__ void add_slab(float (&s)[4], const uint2 v)
@@ -1495,7 +1830,7 @@ extern "C" double flashllm_hip_wide_b_step(int n, int m, int split_k)
 extern "C" int flashllm_hip_launch_spmm_group(
     void* stream, const void* comp, const int* offs, const void* b, int ldb, void* out, int m, int n, int k, int split_k, int store, int runs)
 {
-    const int       cols  = columns_per_workgroup(n, m, split_k);
+    const int       cols  = runs > 1 ? 128 : columns_per_workgroup(n, m, split_k);
     const unsigned  units = static_cast<unsigned>(m / kTileRows) * (n / cols);
     const dim3      grid  = grid_of(units, split_k);
     hipStream_t     s     = static_cast<hipStream_t>(stream);
@@ -1505,10 +1840,10 @@ extern "C" int flashllm_hip_launch_spmm_group(
     store                 = split_k > 1 ? store == kStorePages : store & kStoreRelu;
     if (cols == kWideCols)
         hipLaunchKernelGGL(spmm_wide_kernel, grid, dim3(kWideWaves * kLanes), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / cols, store, units);
-    else if (runs == kSliceRuns)
-        hipLaunchKernelGGL((spmm_group_kernel<2, kSliceRuns>), grid, dim3(kGroupThreads * kSliceRuns), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, store, units);
+    else if (runs > 1)
+        hipLaunchKernelGGL(spmm_quarter_kernel, grid, dim3(kQuarters * kLanes), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, store, units);
     else
-        hipLaunchKernelGGL((spmm_group_kernel<2, 1>), grid, dim3(kGroupThreads), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, store, units);
+        hipLaunchKernelGGL(spmm_group_kernel<2>, grid, dim3(kGroupThreads), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, store, units);
     return static_cast<int>(hipGetLastError());
 }
 

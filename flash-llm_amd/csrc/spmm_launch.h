@@ -51,9 +51,10 @@ int flashllm_hip_launch_spmm(void*       stream,
 void flashllm_hip_set_rows_per_workgroup(int rows);
 int  flashllm_hip_rows_per_workgroup(int n, int m, int split_k);
 
-// The same product for wide B (n % 128 == 0) by workgroups of four waves that share each scattered tile, 128 or 256
-// columns each (a rule of n, m and split_k, which the reduction of its pages follows too).
-// runs: 1, or 3 for workgroups of three such groups (of 128 columns) that divide each slice along K.
+// The same product for wide B (n % 128 == 0).  runs 1: by workgroups of four waves that share each scattered tile, 128
+// or 256 columns each (a rule of n, m and split_k, which the reduction of its pages follows too).  Any other value: by
+// workgroups of four waves, 128 columns each, that divide the slice along K among themselves and add up at the end (pages
+// only where the rule says 128).
 int flashllm_hip_launch_spmm_group(void*       stream,
                                    const void* compressed_a,
                                    const int*  tile_offsets,

@@ -17,12 +17,12 @@ def accepted(kernel, vgprs, occupancy):
 
 
 @pytest.mark.parametrize("kernel,vgprs,occupancy", [("spmm_stream_kernel", 250, 2), ("spmm_group_kernel", 168, 3),
-                                                    ("spmm_wide_kernel", 234, 2), ("encode_tiles_kernel", 79, 6)])
+                                                    ("spmm_wide_kernel", 234, 2), ("spmm_quarter_kernel", 218, 1), ("encode_tiles_kernel", 79, 6)])
 def test_a_kernel_below_its_occupancy_stops_the_build(kernel, vgprs, occupancy):
     assert accepted(kernel, vgprs, occupancy)
     assert not accepted(kernel, vgprs, occupancy - 1)
 
 
-@pytest.mark.parametrize("kernel,vgprs,occupancy", [("spmm_group_kernel", 169, 3), ("spmm_wide_kernel", 241, 2)])
+@pytest.mark.parametrize("kernel,vgprs,occupancy", [("spmm_group_kernel", 169, 3), ("spmm_wide_kernel", 241, 2), ("spmm_quarter_kernel", 225, 1)])
 def test_a_kernel_with_more_registers_than_measured_stops_the_build(kernel, vgprs, occupancy):
     assert not accepted(kernel, vgprs, occupancy)

@@ -88,8 +88,8 @@ def launch_group(product, torch, w, b, n, split_k, pages, runs):
 @pytest.mark.parametrize("tiles,split_k,pages", [(11, 1, 0), (11, 2, 1), (11, 5, 0), (11, 11, 1), (100, 3, 0), (97, 2, 1)])
 @pytest.mark.parametrize("dense", [False, True])
 def test_groups_sharing_a_slice_match_one_group(product, n, tiles, split_k, pages, dense):
-    """The same for wide B: three groups of four waves on runs of a slice, from runs without a tile (slices of 1 and 3)
-    to runs of 11 and 12, 16 and 17; with a dense row tile both kernels hold three rounds of a tile instead of two."""
+    """The same for wide B: four waves with a quarter of a slice each, from quarters without a tile (slices of 1 and 3)
+    to odd ones; with a dense row tile the kernels hold more rounds of a tile in registers."""
     import torch
 
     print(f"groups per slice n={n} tiles={tiles} split_k={split_k} pages={pages} dense={dense}", flush=True)
@@ -107,3 +107,25 @@ def test_groups_sharing_a_slice_match_one_group(product, n, tiles, split_k, page
     # as above, with k products of at most 0.25 * 4.5
     bound = 2 * 2.0 ** -10 * np.abs(want) + k * 1.125 * 2.0 ** -23
     assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want))
+
+
+@pytest.mark.parametrize("sparsity", [0.9, 0.8, 0.7, 0.2, 1.0])  # the three depths of the ring, tiles beyond it, no vectors at all
+@pytest.mark.parametrize("tiles", [1, 2, 3, 7, 8, 17])           # runs of an odd number of tiles end with an empty one
+def test_quarters_keep_inf_and_nan_where_they_are(product, tiles, sparsity):
+    """An Inf or NaN in B shows in its own column only, as with the kernel whose waves share every tile: the empty tile
+    behind an odd run multiplies zeros by zeros."""
+    import torch
+
+    print(f"quarters inf and nan tiles={tiles} sparsity={sparsity}", flush=True)
+    m, k, n = 256, 64 * tiles, 128
+    w = product.SparseWeight(synth.sparse_matrix(m, k, sparsity, 104, dist="normal", sigma=0.05))
+    dense = synth.dense_b(k, n, 105, dist="normal").reshape(n, k)
+    dense[3], dense[77, -1], dense[100, k // 2] = np.inf, np.nan, np.inf
+    b = torch.from_numpy(dense).cuda()
+    want = launch_group(product, torch, w, b, n, 1, 0, 1).astype(np.float64)
+    got = launch_group(product, torch, w, b, n, 1, 0, 4).astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    finite = np.isfinite(want)
+    # two sums of the same k products, of at most 0.25 * 4.5, in another order
+    bound = 2 * 2.0 ** -10 * np.abs(want[finite]) + k * 1.125 * 2.0 ** -23
+    assert np.all(np.abs(got[finite] - want[finite]) <= bound)
