@@ -90,8 +90,9 @@ int flashllm_hip_launch_xcd_probe(void* stream, unsigned* out, int workgroups);
 int flashllm_hip_launch_take_rows(void* stream, void* dst, const void* src, int rows, int cols, int src_ld);
 
 // offs[0..tiles+1] = TileOffsets of the device-resident dense matrix a (M x K halfs, 16-byte aligned,
-// M % 128 == 0, K % 64 == 0): a count kernel and an in-place prefix sum.
-int flashllm_hip_launch_tile_offsets(void* stream, const void* a, int m, int k, int* offs);
+// M % 128 == 0, K % 64 == 0): a count kernel and an in-place prefix sum, which also stores the sum of all counts at
+// vectors (host memory the GPU can write, or null).
+int flashllm_hip_launch_tile_offsets(void* stream, const void* a, int m, int k, int* offs, int* vectors);
 
 // out[offs[t]*4 ...] = the packed nonzeros of tile t in the reference's reordered layout.
 int flashllm_hip_launch_encode(void* stream, const void* a, int m, int k, const int* offs, void* out);

@@ -22,8 +22,10 @@
 // row per load, and the encoder sorts a tile into output order in LDS and stores it as consecutive 16-byte vectors:
 // with every item storing its own 4 bytes at its destination (a line of its own per lane) and one wave counting 128-byte
 // pieces of eight rows at a time the call took 550 us; now 268, and 243 with non-temporal loads and stores (a trace of
-// the former: count 95, encoder 147, i.e. 5.3 and 4.9 TB/s).  About 40 us are a fixed cost: launches, the prefix sum
-// and the copy of its total to the host (2048 x 4096: 43.6 us).
+// the former: count 95, encoder 147, i.e. 5.3 and 4.9 TB/s).  About 25 us are a fixed cost: launches, the prefix sum
+// and the host's wait for its total, which the kernel stores to host memory itself (2048 x 4096: 35.8 us; 44.1 with a copy
+// of it).  Encoding the tiles last counted first, while they may still be in the Infinity Cache, gains nothing (27648 x
+// 9216: 140 us either way, with cached loads in either kernel or both too).
 #include "spmm_launch.h"
 
 #include <hip/hip_runtime.h>
@@ -183,7 +185,8 @@ __device__ __forceinline__ int wave_scan(int x)  // inclusive
     return x;
 }
 
-__global__ __launch_bounds__(kLanes* kScanWaves) void scan_offsets_kernel(int* __restrict__ offs, int tiles)
+// vectors: where the host reads the sum of all counts (host memory), or null.
+__global__ __launch_bounds__(kLanes* kScanWaves) void scan_offsets_kernel(int* __restrict__ offs, int tiles, int* vectors)
 {
     __shared__ int total[kScanWaves];
     const int      lane  = threadIdx.x & (kLanes - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
@@ -225,6 +228,8 @@ __global__ __launch_bounds__(kLanes* kScanWaves) void scan_offsets_kernel(int* _
     if (threadIdx.x == 0) {
         offs[0]         = 0;
         offs[tiles + 1] = carry;
+        if (vectors)
+            __hip_atomic_store(vectors, carry, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -443,7 +448,7 @@ __global__ __launch_bounds__(kEncodeThreads, 6) void encode_tiles_kernel(const u
 
 }  // namespace
 
-extern "C" int flashllm_hip_launch_tile_offsets(void* stream, const void* a, int m, int k, int* offs)
+extern "C" int flashllm_hip_launch_tile_offsets(void* stream, const void* a, int m, int k, int* offs, int* vectors)
 {
     const int   tiles_per_row = k / kTileCols;
     const int   tiles         = (m / kTileRows) * tiles_per_row;
@@ -457,7 +462,7 @@ extern "C" int flashllm_hip_launch_tile_offsets(void* stream, const void* a, int
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return static_cast<int>(e);
-    hipLaunchKernelGGL(scan_offsets_kernel, dim3(1), dim3(kLanes * kScanWaves), 0, s, offs, tiles);
+    hipLaunchKernelGGL(scan_offsets_kernel, dim3(1), dim3(kLanes * kScanWaves), 0, s, offs, tiles, vectors);
     return static_cast<int>(hipGetLastError());
 }
 

@@ -197,3 +197,34 @@ def test_rejects_bad_arguments(product, torch_gpu):
         product.device_compress(torch.zeros(128, 96, dtype=torch.float16, device="cuda"))
     with pytest.raises(TypeError):
         product.device_compress(torch.zeros(128, 64, dtype=torch.float32, device="cuda"))
+
+
+def test_many_threads_compress_at_once(product):
+    """More callers at the same time than there are words for their sizes (64): each gets its own matrix's size and bytes."""
+    import threading
+
+    import torch
+
+    print("threads compressing at once", flush=True)
+    count = 72
+    mats = [synth.sparse_matrix(128 * (1 + i % 3), 64 * (1 + i % 5), 0.6 + 0.005 * i, i) for i in range(count)]
+    devs = [torch.from_numpy(a).cuda() for a in mats]
+    torch.cuda.synchronize()
+    start, got = threading.Barrier(count), [None] * count
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            start.wait()
+            for _ in range(3):
+                comp, offs = product.device_compress(devs[i])
+            got[i] = (comp.cpu().numpy().view(np.uint32), offs.cpu().numpy())
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(count)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    for i, a in enumerate(mats):
+        items, offsets = product.init_sparse_matrix_a(a)
+        assert np.array_equal(got[i][0], items) and np.array_equal(got[i][1], offsets), i
