@@ -6,6 +6,8 @@
 
 #include "flashllm_spmm.h"
 
+#include <stddef.h>
+
 // size of the library-owned slab storage behind flashllm_hip_static_workspace: the limit the public header states
 #define FLASHLLM_STATIC_WORKSPACE_BYTES FLASHLLM_STATIC_WORKSPACE_MAX_BYTES
 
@@ -96,6 +98,12 @@ int flashllm_hip_launch_tile_offsets(void* stream, const void* a, int m, int k, 
 
 // out[offs[t]*4 ...] = the packed nonzeros of tile t in the reference's reordered layout.
 int flashllm_hip_launch_encode(void* stream, const void* a, int m, int k, const int* offs, void* out);
+
+// The same in scan order (the layout of the reference's compressor without reordering).
+int flashllm_hip_launch_encode_scan(void* stream, const void* a, int m, int k, const int* offs, void* out);
+
+// Copies ordinary host memory to the GPU and waits for it.
+int flashllm_hip_upload(void* stream, void* dst, const void* src, size_t bytes);
 
 // Waits for the stream, then *status = the FLASHLLM_ENCODE_* bits the encoder has recorded on the current device
 // since they were last read, and clears them.

@@ -446,6 +446,79 @@ __global__ __launch_bounds__(kEncodeThreads, 6) void encode_tiles_kernel(const u
         report(FLASHLLM_ENCODE_RANGE);
 }
 
+// The encoder without reordering (csrc/SpMM_API.cu:363-489): a tile's items in scan order, row by row; the padding to a
+// multiple of four takes the first zeros of the tile as they are (-0 and NaN among them), each in its place in the order.
+// One workgroup of four waves per tile, half a row (64 bytes) to a thread: the items before it are the nonzeros before it, by
+// a scan over the workgroup, and of the zeros before it at most as many as the tile is padded with.  The tile is put
+// together in LDS and stored as consecutive 16-byte vectors.  32 KB of LDS, four workgroups per CU;
+// bound by HBM like the encoder above (27648 x 9216 with the count 250 us, reordered 254).
+constexpr int kHalfRow = kTileCols / 2;
+
+__global__ __launch_bounds__(kEncodeThreads) void encode_tiles_scan_kernel(const uint16_t* __restrict__ a,
+                                                                         int k,
+                                                                         int tiles_per_row,
+                                                                         const int* __restrict__ offs,
+                                                                         uint32_t* __restrict__ out)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t list[kTileRows * kTileCols];
+    __shared__ int total[kEncodeThreads / kLanes];
+    const int       t    = blockIdx.x;
+    const int       tid  = threadIdx.x, lane = tid & (kLanes - 1), wave = tid / kLanes;
+    const int       row  = tid / 2, col = tid % 2 * kHalfRow;
+    const uint16_t* base = tile_base(a, k, tiles_per_row, t) + static_cast<size_t>(row) * k + col;
+    uint32_t        word[kHalfRow / 2];
+#pragma unroll
+    for (int i = 0; i < kHalfRow / 8; i++) {
+        const uintx4 v = *reinterpret_cast<const uintx4*>(base + i * 8);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            word[4 * i + e] = v[e];
+    }
+    const int first = offs[t], room = (offs[t + 1] - first) * 4;
+
+    int mine = 0;
+#pragma unroll
+    for (int i = 0; i < kHalfRow / 2; i++) {
+        const uint32_t both = keeps_pair(word[i]);
+        mine += static_cast<int>((both & 1u) + (both >> 16));
+    }
+    const int inclusive = wave_scan(mine);
+    if (lane == kLanes - 1)
+        total[wave] = inclusive;
+    __syncthreads();
+    int before = inclusive - mine, nnz = 0;
+#pragma unroll
+    for (int w = 0; w < kEncodeThreads / kLanes; w++) {
+        before += w < wave ? total[w] : 0;
+        nnz += total[w];
+    }
+    const int pad   = (4 - nnz % 4) % 4;
+    const int count = nnz + pad;
+    int       zeros = tid * kHalfRow - before;  // before this half row
+    int       at    = before + (zeros < pad ? zeros : pad);
+    if (room != count && tid == 0)
+        report(FLASHLLM_ENCODE_OFFSETS);
+    const uint32_t flip = static_cast<uint32_t>(row & 7) << 3, row_position = static_cast<uint32_t>(row * kTileCols);
+#pragma unroll
+    for (int i = 0; i < kHalfRow / 2; i++) {
+        const uint32_t both = keeps_pair(word[i]);
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const bool     kept     = (both >> (16 * e)) & 1u;
+            const uint32_t position = row_position + (static_cast<uint32_t>(col + 2 * i + e) ^ flip);
+            if (kept || zeros < pad)
+                list[at++] = ((word[i] >> (16 * e)) & 0xffffu) | (position << 16);
+            zeros += kept ? 0 : 1;
+        }
+    }
+    __syncthreads();
+    // never outside this tile's range of Compressed_A, whatever TileOffsets says
+    const int vectors = (count < room ? count : room) / 4;
+    uintx4*   to      = reinterpret_cast<uintx4*>(out) + first;
+    for (int v = tid; v < vectors; v += kEncodeThreads)
+        __builtin_nontemporal_store(reinterpret_cast<const uintx4*>(list)[v], to + v);
+}
+
 }  // namespace
 
 extern "C" int flashllm_hip_launch_tile_offsets(void* stream, const void* a, int m, int k, int* offs, int* vectors)
@@ -464,6 +537,15 @@ extern "C" int flashllm_hip_launch_tile_offsets(void* stream, const void* a, int
         return static_cast<int>(e);
     hipLaunchKernelGGL(scan_offsets_kernel, dim3(1), dim3(kLanes * kScanWaves), 0, s, offs, tiles, vectors);
     return static_cast<int>(hipGetLastError());
+}
+
+// Plainly: 28.6 GB/s (7168 x 7168, 3.60 ms), and staged through a ring of pinned pieces that eight threads fill 30.0
+// (3.42 ms), the rate of the link.
+extern "C" int flashllm_hip_upload(void* stream, void* dst, const void* src, size_t bytes)
+{
+    hipStream_t      s = static_cast<hipStream_t>(stream);
+    const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
+    return static_cast<int>(e == hipSuccess ? hipStreamSynchronize(s) : e);
 }
 
 extern "C" int flashllm_hip_encode_status(void* stream, unsigned int* status)
@@ -486,6 +568,23 @@ extern "C" int flashllm_hip_launch_encode(void* stream, const void* a, int m, in
     const int tiles_per_row = k / kTileCols;
     const int tiles         = (m / kTileRows) * tiles_per_row;
     hipLaunchKernelGGL(encode_tiles_kernel,
+                       dim3(tiles),
+                       dim3(kEncodeThreads),
+                       0,
+                       static_cast<hipStream_t>(stream),
+                       static_cast<const uint16_t*>(a),
+                       k,
+                       tiles_per_row,
+                       offs,
+                       static_cast<uint32_t*>(out));
+    return static_cast<int>(hipGetLastError());
+}
+
+extern "C" int flashllm_hip_launch_encode_scan(void* stream, const void* a, int m, int k, const int* offs, void* out)
+{
+    const int tiles_per_row = k / kTileCols;
+    const int tiles         = (m / kTileRows) * tiles_per_row;
+    hipLaunchKernelGGL(encode_tiles_scan_kernel,
                        dim3(tiles),
                        dim3(kEncodeThreads),
                        0,

@@ -165,6 +165,12 @@ int flashllm_device_tile_offsets(void* stream, const void* A, int M, int K, int*
 int flashllm_device_compress(void* stream, const void* A, int M, int K, const int* TileOffsets, void* Compressed_A);
 
 /*
+ * The same with the bytes of flashllm_init_sparse_matrix_a_noreorder (reference InitSparseMatrixA_API_NoReorder,
+ * csrc/SpMM_API.cu:363-489): a tile's items in scan order.  TileOffsets are those of flashllm_device_tile_offsets.
+ */
+int flashllm_device_compress_noreorder(void* stream, const void* A, int M, int K, const int* TileOffsets, void* Compressed_A);
+
+/*
  * What flashllm_device_compress found wrong, for callers that want the host compressor's error behaviour from the
  * asynchronous device one: waits for the stream, stores in *Status the bits recorded on the current GPU since the
  * last call of this function (0 = every tile was encoded as the host compressor would), and clears them.

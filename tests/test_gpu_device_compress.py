@@ -228,3 +228,62 @@ def test_many_threads_compress_at_once(product):
     for i, a in enumerate(mats):
         items, offsets = product.init_sparse_matrix_a(a)
         assert np.array_equal(got[i][0], items) and np.array_equal(got[i][1], offsets), i
+
+
+@pytest.mark.parametrize("case", ["pads", "dense", "empty", "late zeros", "special"])
+def test_scan_order_matches_the_host(product, torch_gpu, case):
+    """Every number of padding items (taken from the first zeros, in their place and as they are), none of them, and
+    tiles whose first zeros lie at the end; the bytes are those of InitSparseMatrixA_API_NoReorder."""
+    torch = torch_gpu
+    say("device compress without reordering:", case)
+    rng = np.random.default_rng(7)
+    a = synth.sparse_matrix(384, 256, {"dense": 0.0, "empty": 1.0}.get(case, 0.8), 41)
+    if case == "pads":
+        for tile in range(12):  # tile by tile one more nonzero
+            r, c = tile // 4 * 128, tile % 4 * 64
+            a[r:r + 128, c:c + 64] = 0
+            a[r:r + 128, c:c + 64].flat[rng.choice(8192, tile, replace=False)] = 1
+    elif case == "late zeros":
+        a[:] = 1
+        for tile in range(12):
+            a[tile // 4 * 128 + 127, tile % 4 * 64 + 63 - tile:tile % 4 * 64 + 64] = 0
+    elif case == "special":
+        bits = a.view(np.uint16)
+        for value in (0x8000, 0x7e00, 0xfc01, 0x7c00, 0xfc00, 0x0001, 0x8001):  # -0, NaNs, infinities, subnormals
+            bits.flat[rng.choice(bits.size, 2000, replace=False)] = value
+    want, want_offs = product.init_sparse_matrix_a_noreorder(a)
+    comp, offs = product.device_compress_noreorder(torch.from_numpy(a).cuda())
+    assert np.array_equal(offs.cpu().numpy(), want_offs)
+    assert np.array_equal(comp.cpu().numpy().view(np.uint32), want)
+    assert product.device_compress_status() == 0
+
+
+@pytest.mark.parametrize("reorder", [True, False])
+@pytest.mark.parametrize("form", ["float16", "bits", "read-only", "strided", "empty"])
+def test_loaded_weight_has_the_host_compressors_bytes(product, torch_gpu, form, reorder):
+    torch = torch_gpu
+    say("loaded weight:", form, reorder)
+    a = synth.sparse_matrix(384, 576, 1.0 if form == "empty" else 0.8, 51)
+    given = a
+    if form == "bits":
+        given = a.view(np.uint16)
+    elif form == "read-only":
+        given = np.frombuffer(a.tobytes(), dtype=np.float16).reshape(a.shape)
+    elif form == "strided":
+        given = np.asfortranarray(a)
+    w = product.SparseWeight(given, reorder=reorder)
+    items, offsets = (product.init_sparse_matrix_a if reorder else product.init_sparse_matrix_a_noreorder)(a)
+    assert (w.m, w.k, w.nnz, w.num_offsets) == (384, 576, items.size, offsets.size)
+    assert w.comp.dtype == torch.int32 and w.offs.dtype == torch.int32
+    assert np.array_equal(w.comp.cpu().numpy().view(np.uint32), items if items.size else np.zeros(1, dtype=np.uint32))
+    assert np.array_equal(w.offs.cpu().numpy(), offsets)
+
+
+def test_loading_refuses_what_the_host_compressor_refuses(product, torch_gpu):
+    for bad in (np.zeros((100, 64), np.float16), np.zeros((128, 96), np.float16), np.zeros((0, 64), np.float16)):
+        with pytest.raises(product.CompressError):
+            product.SparseWeight(bad)
+    with pytest.raises(TypeError):
+        product.SparseWeight(np.zeros((128, 64), np.float32))
+    with pytest.raises(ValueError):
+        product.SparseWeight(np.zeros((2, 128, 64), np.float16))
