@@ -1172,7 +1172,11 @@ __global__ __launch_bounds__(kWideWaves* kLanes, 2) void spmm_wide_kernel(const 
 //     The loop body is therefore two tiles; an early exit between them makes the compiler move accumulators and spill, so
 //     runs are whole pairs of tiles and an odd one ends with an empty tile, whose B is zeros.
 //   * Lanes past a tile's end load its last vector again and store the same items once more: no masks.
-// 160 KB of LDS and 512 registers: one workgroup per CU.  Measured with the four-wave kernel (where a launch had at most one
+//   * The stream is loaded as other data is: the column groups of a row tile sit on one XCD and share its L2 (7168 x 28672, N =
+//     512, Split_K 1 242 us with non-temporal loads, 230).
+// With 64 columns (N = 64) a tile is two such phases and one window of B, so that B is asked for two tiles ahead; a tile without
+// vectors takes zeros for B, as the other kernels for N <= 64 leave it out altogether.
+// 160 KB of LDS and 512 registers (64 columns 320): one workgroup per CU.  Measured with the four-wave kernel (where a launch had at most one
 // workgroup per CU, three groups of four waves) and this one, 80 %, Split_K 1: 7168 x 28672, N = 512 247 -> 213 us, 7168 x
 // 7168, N = 512 75 -> 58, N = 128 68 -> 52, 21504 x 7168, N = 384 146 -> 125, N = 512 (256-column kernel) 192 -> 172, 1664 x
 // 27200, N = 128 233 -> 171.  Without loads from memory the first takes 161 us and with nothing but the MFMAs 128: what is
@@ -1186,7 +1190,7 @@ using floatx16 = float __attribute__((ext_vector_type(16)));
 // what a tile without vectors reads: an item that stores 0 at position 0
 __device__ uint4 g_zero_vector;
 
-template<int R>
+template<int NJ, int R>
 __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
                                                   const uint4* __restrict__ comp,
                                                   const int* __restrict__ toff,
@@ -1210,11 +1214,11 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
     const uint32_t tile_l = __builtin_amdgcn_readfirstlane(lds_offset(mine));
     const uint32_t bwin_l = __builtin_amdgcn_readfirstlane(lds_offset(lds)) + kQuarters * (kTileHalfs * 2) + wave * (3 * kQuarterWindow);
 
-    floatx16 acc[4][4];
+    floatx16 acc[4][NJ];
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < NJ; j++)
 #pragma unroll
             for (int e = 0; e < 16; e++)
                 acc[i][j][e] = 0.f;
@@ -1253,7 +1257,7 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
         // Lanes past the tile's end load its last vector again, and store the same items to the same places.
         auto request = [&](uintx4& slot, int r) {
             const uint32_t at = lane * 16u + r * (kLanes * 16u);
-            slot = __builtin_nontemporal_load(reinterpret_cast<const __attribute__((address_space(1))) uintx4*>(from + (at < from_last ? at : from_last)));
+            slot = *reinterpret_cast<const __attribute__((address_space(1))) uintx4*>(from + (at < from_last ? at : from_last));
         };
         auto scatter = [&](uint32_t item) {
             uint32_t position;
@@ -1276,8 +1280,8 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
             uint32_t lanes;
         };
         auto half_of_b = [&](int half) {  // past the end: zeros (a run of an odd number of tiles ends with an empty one, and Inf and NaN stay out)
-            const bool there = half < 2 * ke;
-            return Half{there ? (Global*)(bcols + (half & 1) * (64 * static_cast<size_t>(ldb)) + (half >> 1) * kTileCols) : nothing,
+            const bool there = NJ == 4 ? half < 2 * ke : n[2] > 0;  // NJ == 2: asked where requests are at the same tile
+            return Half{there ? (Global*)(NJ == 4 ? bcols + (half & 1) * (64 * static_cast<size_t>(ldb)) + (half >> 1) * kTileCols : bcols + half * kTileCols) : nothing,
                         there ? 64 * static_cast<size_t>(ldb) : 0, there ? ~0u : 0u};
         };
         auto fetch_b = [&](const Half& half, uint32_t window, int i) {
@@ -1297,7 +1301,7 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
         for (int r = 0; r < R; r++)
             request(ring[0][r], r);
         keep();
-        Half first = half_of_b(2 * kb);
+        Half first = half_of_b(NJ / 2 * kb);
 #pragma unroll
         for (int i = 0; i < 8; i++)
             fetch_b(first, w0, i);
@@ -1312,7 +1316,7 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
 #pragma unroll
             for (int i = 0; i < 4; i++)
                 clear_a(s, i);
-        first = half_of_b(2 * kb + 1);
+        first = half_of_b(NJ / 2 * kb + 1);
 #pragma unroll
         for (int i = 0; i < 8; i++)
             fetch_b(first, w1, i);
@@ -1329,7 +1333,7 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
         if (n[0] > R * kLanes)
             scatter_rest();
         keep();
-        first = half_of_b(2 * kb + 2);
+        first = half_of_b(NJ / 2 * kb + 2);
 #pragma unroll
         for (int i = 0; i < 8; i++)
             fetch_b(first, w2, i);
@@ -1349,7 +1353,7 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
         keep();
 
         constexpr int R0 = (R + 1) / 2, R1 = R - R0;
-        auto tile = [&](auto slot, int t) {
+        auto tile_of_128 = [&](auto slot, int t) {
             uintx4(&next)[R] = ring[decltype(slot)::value];
             // phase 0: half 0 of B, k steps 0 and 1
 #pragma unroll
@@ -1425,6 +1429,69 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
             w2 = w1;
             w1 = old;
         };
+        // 64 columns: phases 0 and 1 are all there is, and B's windows hold three tiles.  w0 holds the current one's.
+        auto tile_of_64 = [&](auto slot, int t) {
+            uintx4(&next)[R] = ring[decltype(slot)::value];
+            auto scatter_part = [&](int m) {  // m of 16
+#pragma unroll
+                for (int i = m * R * 4 / 16; i < (m + 1) * R * 4 / 16; i++) {
+                    scatter(next[i / 4][i % 4]);
+                    if (i % 4 == 3)
+                        request(next[i / 4], i / 4);
+                }
+            };
+#pragma unroll
+            for (int m = 0; m < 16; m++) {
+                multiply(0, m);
+                if (m < 4)
+                    read_b(1, w0, m);
+                if (m < 8)
+                    read_a(2 + m / 4, m % 4);
+                if (m >= 4 && m < 12)
+                    clear_a(2 + (m - 4) / 4, m % 4);
+                if (m >= 12) {
+                    scatter_part(2 * (m - 12));
+                    scatter_part(2 * (m - 12) + 1);
+                }
+                keep();
+            }
+            // this tile's B is out of LDS, the next one's has landed
+            asm volatile("" ::"v"(b[1][0]), "v"(b[1][1]), "v"(b[1][2]), "v"(b[1][3]) : "memory");
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + R) : "memory");
+            const Half b_next = half_of_b(t + 3);
+            keep();
+#pragma unroll
+            for (int m = 0; m < 16; m++) {
+                multiply(1, m);
+                if (m < 4)
+                    read_b(0, w1, m);
+                if (m < 8) {
+                    scatter_part(8 + m);
+                    fetch_b(b_next, w0, m);
+                }
+                if (m == 7) {
+                    if (n[0] > R * kLanes)
+                        scatter_rest();
+                    keep();
+                    next_tile(t + 4);
+                }
+                if (m >= 8) {
+                    read_a((m - 8) / 4, m % 4);
+                    clear_a((m - 8) / 4, m % 4);
+                }
+                keep();
+            }
+            const uint32_t old = w0;
+            w0 = w1;
+            w1 = w2;
+            w2 = old;
+        };
+        auto tile = [&](auto slot, int t) {
+            if constexpr (NJ == 4)
+                tile_of_128(slot, t);
+            else
+                tile_of_64(slot, t);
+        };
         for (int t = kb; t < ke; t += 2) {
             tile(std::integral_constant<int, 1>{}, t);
             tile(std::integral_constant<int, 0>{}, t + 1);
@@ -1440,7 +1507,7 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
     floatx4*  sums = reinterpret_cast<floatx4*>(lds);
     constexpr int kPerWave = kQuarterLds / 16;
 #pragma unroll
-    for (int part = 0; part < 2; part++) {
+    for (int part = 0; part < NJ / 2; part++) {
         if (part)
             __syncthreads();
 #pragma unroll
@@ -1482,6 +1549,7 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
     }
 }
 
+template<int NJ>
 __global__ __launch_bounds__(kQuarters* kLanes, 1) void spmm_quarter_kernel(const uint4* __restrict__ comp,
                                                                    const int* __restrict__ offs,
                                                                    const _Float16* __restrict__ B,
@@ -1502,7 +1570,7 @@ __global__ __launch_bounds__(kQuarters* kLanes, 1) void spmm_quarter_kernel(cons
         return;
     const int unit = place.unit, slice = place.part;
     const int rowtile = unit / col_groups;
-    const int col0    = (unit % col_groups) * 128;
+    const int col0    = (unit % col_groups) * (32 * NJ);
     // slices, the last vector a load may touch and the empty matrix as in spmm_group_kernel
     const int avg = (kt - 1) / split_k + 1;
     int       kb  = slice * avg;
@@ -1520,11 +1588,11 @@ __global__ __launch_bounds__(kQuarters* kLanes, 1) void spmm_quarter_kernel(cons
     const int       whole = offs[static_cast<size_t>(M / kTileRows) * kt];
     const long long tiles = static_cast<long long>(M / kTileRows) * kt;
     if (whole <= 236 * tiles)
-        spmm_quarter_body<4>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, store, place.w, units * split_k);
+        spmm_quarter_body<NJ, 4>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, store, place.w, units * split_k);
     else if (whole <= 428 * tiles)
-        spmm_quarter_body<7>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, store, place.w, units * split_k);
+        spmm_quarter_body<NJ, 7>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, store, place.w, units * split_k);
     else
-        spmm_quarter_body<10>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, store, place.w, units * split_k);
+        spmm_quarter_body<NJ, 10>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, store, place.w, units * split_k);
 }
 
 __device__ __forceinline__ void add_slab(float (&s)[4], const uint2 v)
@@ -1795,6 +1863,12 @@ extern "C" int flashllm_hip_launch_spmm(
 {
     hipStream_t s = static_cast<hipStream_t>(stream);
     store         = split_k > 1 ? store == kStorePages : store & kStoreRelu;
+    if (n == 64 && k_waves == 0) {
+        const unsigned units = static_cast<unsigned>(m / kTileRows);
+        hipLaunchKernelGGL(spmm_quarter_kernel<2>, grid_of(units, split_k), dim3(kQuarters * kLanes), 0, s, static_cast<const uint4*>(comp), offs,
+                           static_cast<const _Float16*>(b), ldb, static_cast<_Float16*>(out), m, n, k, split_k, 1, store, units);
+        return static_cast<int>(hipGetLastError());
+    }
     if (n == 64 && rows_per_workgroup(n, m, split_k) == 8)
         return launch_spmm<4, 8, 8, 2, 1>(s, comp, offs, b, ldb, out, m, n, k, split_k, 1, store);
     if (k_waves == 8)
@@ -1841,7 +1915,7 @@ extern "C" int flashllm_hip_launch_spmm_group(
     if (cols == kWideCols)
         hipLaunchKernelGGL(spmm_wide_kernel, grid, dim3(kWideWaves * kLanes), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / cols, store, units);
     else if (runs > 1)
-        hipLaunchKernelGGL(spmm_quarter_kernel, grid, dim3(kQuarters * kLanes), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, store, units);
+        hipLaunchKernelGGL(spmm_quarter_kernel<4>, grid, dim3(kQuarters * kLanes), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, store, units);
     else
         hipLaunchKernelGGL(spmm_group_kernel<2>, grid, dim3(kGroupThreads), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, store, units);
     return static_cast<int>(hipGetLastError());

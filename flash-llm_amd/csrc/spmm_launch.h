@@ -30,7 +30,8 @@ enum {
 // out: C when split_k == 1, else the slab workspace (split_k * M * N halfs).
 // ldb: halfs between consecutive columns of B (>= K, a multiple of 8; K for a dense column-major B).
 // k_waves: 1, 2, 4 or 8 waves per workgroup divide each (row tile, slice) among themselves along K (ignored by a
-// launch that takes eight row tiles per workgroup, below).
+// launch that takes eight row tiles per workgroup, below).  0, for n = 64: four waves with a quarter of the slice each
+// (spmm_quarter_kernel; pages only with one row tile per workgroup).
 // Requires M % 128 == 0, K % 64 == 0, N in {8,16,32,64} or N % 64 == 0.
 int flashllm_hip_launch_spmm(void*       stream,
                              const void* compressed_a,

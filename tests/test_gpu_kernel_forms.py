@@ -1,5 +1,5 @@
 """Every form a product can take, launched by itself: the kernel for N <= 64 with 1, 2, 4 or 8 waves per slice or eight row
-tiles per workgroup, the four-wave kernel with one or three groups per slice, the 256-column kernel.  Each with the
+tiles per workgroup, four waves with a quarter of a slice each at N = 64 and wide B, the four-wave and the 256-column kernel.  Each with the
 activation stored with the sums, with B's columns farther apart than K (the attention-output linear reads B so), and on a
 matrix without nonzeros, whose Compressed_A holds a single item; the results are compared bit for bit with the plain form's."""
 import ctypes
@@ -12,7 +12,7 @@ import synth
 pytestmark = pytest.mark.gpu
 
 # kernel, N, waves or groups per slice; "rows8" stands for eight row tiles per workgroup
-FORMS = ([("stream", n, waves) for n in (8, 16, 32, 64) for waves in (1, 2, 4, 8)] + [("rows8", 64, 1)]
+FORMS = ([("stream", n, waves) for n in (8, 16, 32, 64) for waves in (1, 2, 4, 8)] + [("rows8", 64, 1), ("stream", 64, 0)]
          + [("group", n, runs) for n in (128, 384) for runs in (1, 3)] + [("wide", 256, 1), ("wide", 512, 1)])
 M, K, SPLIT_K = 3072, 704, 3           # eleven k tiles: slices of 4, 4 and 3
 WIDE_M, WIDE_SPLIT_K = 128 * 132, 3    # enough workgroups for 256 columns each

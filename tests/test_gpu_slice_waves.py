@@ -129,3 +129,30 @@ def test_quarters_keep_inf_and_nan_where_they_are(product, tiles, sparsity):
     # two sums of the same k products, of at most 0.25 * 4.5, in another order
     bound = 2 * 2.0 ** -10 * np.abs(want[finite]) + k * 1.125 * 2.0 ** -23
     assert np.all(np.abs(got[finite] - want[finite]) <= bound)
+
+
+@pytest.mark.parametrize("sparsity", [0.9, 0.8, 0.7, 0.2, 1.0])
+@pytest.mark.parametrize("tiles,split_k,pages", [(1, 1, 0), (3, 1, 0), (7, 2, 1), (8, 3, 0), (17, 1, 0)])
+def test_quarters_at_64_columns_match_one_wave(product, tiles, split_k, pages, sparsity):
+    """N = 64: the one-wave form leaves tiles without vectors out, so an Inf or NaN opposite such a tile does not show."""
+    import torch
+
+    print(f"quarters at 64 columns tiles={tiles} split_k={split_k} pages={pages} sparsity={sparsity}", flush=True)
+    m, k = 384, 64 * tiles
+    a = synth.sparse_matrix(m, k, sparsity, 106, dist="normal", sigma=0.05)
+    a[:128, -64:] = 0
+    w = product.SparseWeight(a)
+    dense = synth.dense_b(k, 64, 107, dist="normal").reshape(64, k)
+    dense[3, -1], dense[40, -64], dense[50, k // 2] = np.inf, np.nan, np.inf
+    b = torch.from_numpy(dense).cuda()
+    product.lib().flashllm_hip_set_rows_per_workgroup(1)
+    try:
+        want = launch(product, torch, w, b, 64, split_k, pages, 1).astype(np.float64)
+        got = launch(product, torch, w, b, 64, split_k, pages, 0).astype(np.float64)
+    finally:
+        product.lib().flashllm_hip_set_rows_per_workgroup(0)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    finite = np.isfinite(want)
+    # two sums of the same k products, of at most 0.25 * 4.5, in another order
+    bound = 2 * 2.0 ** -10 * np.abs(want[finite]) + k * 1.125 * 2.0 ** -23
+    assert np.all(np.abs(got[finite] - want[finite]) <= bound)
