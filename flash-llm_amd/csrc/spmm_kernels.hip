@@ -1571,7 +1571,7 @@ __global__ __launch_bounds__(kQuarters* kLanes, 1) void spmm_quarter_kernel(cons
     const int unit = place.unit, slice = place.part;
     const int rowtile = unit / col_groups;
     const int col0    = (unit % col_groups) * (32 * NJ);
-    // slices, the last vector a load may touch and the empty matrix as in spmm_group_kernel
+    // slices as in spmm_group_kernel
     const int avg = (kt - 1) / split_k + 1;
     int       kb  = slice * avg;
     kb            = kb < kt ? kb : kt;
