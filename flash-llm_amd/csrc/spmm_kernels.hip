@@ -1595,6 +1595,71 @@ __global__ __launch_bounds__(kQuarters* kLanes, 1) void spmm_quarter_kernel(cons
         spmm_quarter_body<NJ, 10>(lds, comp, toff, B, ldb, o, M, kb, ke, col0, store, place.w, units * split_k);
 }
 
+// spmm_even_kernel: the same program for launches of several rounds, or of one that leaves CUs idle: the k tiles of all units
+// (row tile, 128 columns) in a row are divided evenly among 256 workgroups, one per CU, `share` tiles each.  A workgroup
+// takes what it has of one unit after the other, and leaves the sums of each as eight pages in the workspace: the i-th
+// workgroup that has a part of unit u at page 8 * (i * units + u).  splitk_reduce_even_kernel adds the parts up.
+// The ranges of a die's workgroups follow one another, so that the parts of a unit meet in one L2.  224 + 256 registers.  Calls, 80 %: 36864
+// x 9216, N = 128, Split_K 3 120.9 -> 102.5 us (the four-wave kernel, 864 workgroups of which 768 run at once), 49152 x 12288, N = 128, 2
+// 194 -> 183, 17152 x 9536, N = 256, 2 126 -> 108, 5120 x 9216, N = 640, 90 %, 5 84.4 -> 73.7.
+constexpr int kEvenWorkgroups = 256;
+
+template<int R>
+__device__ __forceinline__ void spmm_even_body(unsigned char* lds,
+                                               const uint4* __restrict__ comp,
+                                               const int* __restrict__ offs,
+                                               const _Float16* __restrict__ B,
+                                               int ldb,
+                                               _Float16* __restrict__ ws,
+                                               int kt,
+                                               int col_groups,
+                                               int units,
+                                               int share)
+{
+    const long long all   = static_cast<long long>(units) * kt;
+    const int       range = blockIdx.x * (kEvenWorkgroups / kXcds) + blockIdx.y;
+    long long       at    = static_cast<long long>(range) * share;
+    const long long end   = at + share < all ? at + share : all;
+    const int       run   = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+    while (at < end) {
+        const int       unit  = __builtin_amdgcn_readfirstlane(static_cast<int>(at / kt));
+        const long long first = static_cast<long long>(unit) * kt;
+        const int       base  = __builtin_amdgcn_readfirstlane(static_cast<int>(at - first));
+        const int       stop  = __builtin_amdgcn_readfirstlane(static_cast<int>((end - first < kt ? end - first : kt)));
+        const int       pairs = (stop - base + 1) / 2;
+        const int       kb    = base + pairs * run / kQuarters * 2;
+        const int       ke    = base + pairs * (run + 1) / kQuarters * 2;
+        const int       part  = __builtin_amdgcn_readfirstlane(static_cast<int>(range - first / share));
+        __syncthreads();  // everybody is done with the sums of the unit before
+        spmm_quarter_body<4, R>(lds, comp, offs + static_cast<size_t>(unit / col_groups) * kt, B, ldb, ws, 0, kb, ke < stop ? ke : stop,
+                                unit % col_groups * 128, kStorePages, 8u * (static_cast<unsigned>(part) * units + unit), 1u);
+        at = first + stop;
+    }
+}
+
+__global__ __launch_bounds__(kQuarters* kLanes, 1) void spmm_even_kernel(const uint4* __restrict__ comp,
+                                                                const int* __restrict__ offs,
+                                                                const _Float16* __restrict__ B,
+                                                                int ldb,
+                                                                _Float16* __restrict__ ws,
+                                                                int M,
+                                                                int K,
+                                                                int col_groups,
+                                                                int units,
+                                                                int share)
+{
+    __shared__ __attribute__((aligned(16384))) unsigned char lds[kQuarters * kQuarterLds];
+    const int       kt    = K / kTileCols;
+    const long long tiles = static_cast<long long>(M / kTileRows) * kt;
+    const int       whole = offs[tiles];
+    if (whole <= 236 * tiles)
+        spmm_even_body<4>(lds, comp, offs, B, ldb, ws, kt, col_groups, units, share);
+    else if (whole <= 428 * tiles)
+        spmm_even_body<7>(lds, comp, offs, B, ldb, ws, kt, col_groups, units, share);
+    else
+        spmm_even_body<10>(lds, comp, offs, B, ldb, ws, kt, col_groups, units, share);
+}
+
 __device__ __forceinline__ void add_slab(float (&s)[4], const uint2 v)
 {
     const half4 h = __builtin_bit_cast(half4, v);
@@ -1716,6 +1781,52 @@ __global__ __launch_bounds__(256) void splitk_reduce_pages_kernel(_Float16* __re
     const int n       = ((unit % col_groups) * blocks + sub % blocks) * 16 + r16;
     const int rowtile = (unit / col_groups) * rows_per_unit + sub / blocks;
     _Float16* o = c + static_cast<size_t>(n) * M + static_cast<size_t>(rowtile) * kTileRows + q * 32 + g * 4;
+    *reinterpret_cast<half4*>(o)      = lo;
+    *reinterpret_cast<half4*>(o + 16) = hi;
+}
+
+// The sums over what spmm_even_kernel left: one workgroup per 128-row x 16-column block of C, mostly on the XCD that stored it.
+template<bool RELU>
+__global__ __launch_bounds__(256) void splitk_reduce_even_kernel(_Float16* __restrict__ c,
+                                                                const uint4* __restrict__ ws,
+                                                                int M,
+                                                                int kt,
+                                                                int col_groups,
+                                                                unsigned units,
+                                                                int share)
+{
+    const Place place = place_of_workgroup(units, 8);
+    if (!place.valid)
+        return;
+    const int       unit  = place.unit, t = threadIdx.x;
+    const long long first = static_cast<long long>(unit) * kt;
+    const int       parts = static_cast<int>((first + kt - 1) / share - first / share) + 1;
+    const uint4*    from  = ws + (static_cast<size_t>(unit) * 8 + place.part) * 256 + t;
+    const size_t    step  = static_cast<size_t>(units) * 8 * 256;
+    float           s[8]  = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < parts; k0 += 4) {
+        uint4 v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (k0 + j < parts)
+                v[j] = from[(k0 + j) * step];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (k0 + j < parts) {
+                const half8 h = __builtin_bit_cast(half8, v[j]);
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    s[e] += static_cast<float>(h[e]);
+            }
+    }
+    half4 lo, hi;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        lo[e] = static_cast<_Float16>(RELU && !(s[e] > 0.f) ? 0.f : s[e]);
+        hi[e] = static_cast<_Float16>(RELU && !(s[4 + e] > 0.f) ? 0.f : s[4 + e]);
+    }
+    const int q = t >> 6, g = (t >> 4) & 3, r16 = t & 15;  // as in splitk_reduce_pages_kernel
+    _Float16* o = c + (static_cast<size_t>(unit % col_groups) * 128 + place.part * 16 + r16) * M + static_cast<size_t>(unit / col_groups) * kTileRows + q * 32 + g * 4;
     *reinterpret_cast<half4*>(o)      = lo;
     *reinterpret_cast<half4*>(o + 16) = hi;
 }
@@ -1918,6 +2029,22 @@ extern "C" int flashllm_hip_launch_spmm_group(
         hipLaunchKernelGGL(spmm_quarter_kernel<4>, grid, dim3(kQuarters * kLanes), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, store, units);
     else
         hipLaunchKernelGGL(spmm_group_kernel<2>, grid, dim3(kGroupThreads), 0, s, cp, offs, bp, ldb, op, m, n, k, split_k, n / 128, store, units);
+    return static_cast<int>(hipGetLastError());
+}
+
+extern "C" int flashllm_hip_launch_spmm_even(
+    void* stream, const void* comp, const int* offs, const void* b, int ldb, void* c, void* ws, int m, int n, int k, int share, int relu)
+{
+    const unsigned units = static_cast<unsigned>(m / kTileRows) * (n / 128);
+    hipStream_t    s     = static_cast<hipStream_t>(stream);
+    hipLaunchKernelGGL(spmm_even_kernel, dim3(kXcds, kEvenWorkgroups / kXcds), dim3(kQuarters * kLanes), 0, s, static_cast<const uint4*>(comp), offs,
+                       static_cast<const _Float16*>(b), ldb, static_cast<_Float16*>(ws), m, k, n / 128, static_cast<int>(units), share);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+        return static_cast<int>(e);
+    const auto reduce = relu ? splitk_reduce_even_kernel<true> : splitk_reduce_even_kernel<false>;
+    hipLaunchKernelGGL(reduce, grid_of(units, 8), dim3(256), 0, s, static_cast<_Float16*>(c), static_cast<const uint4*>(ws), m, k / kTileCols, n / 128,
+                       units, share);
     return static_cast<int>(hipGetLastError());
 }
 

@@ -73,6 +73,21 @@ int flashllm_hip_launch_spmm_group(void*       stream,
 
 int flashllm_hip_columns_per_workgroup(int n, int m, int split_k);
 
+// The product and the reduction for wide B (n % 128 == 0) with the k tiles of all (row tile, 128 columns) divided evenly
+// among 256 workgroups, share = tiles of each, at least a 256th of them.  ws: (kt - 1) / share + 2 slabs of M*N halfs, kt = K / 64.
+int flashllm_hip_launch_spmm_even(void*       stream,
+                                  const void* compressed_a,
+                                  const int*  tile_offsets,
+                                  const void* b,
+                                  int         ldb,
+                                  void*       c,
+                                  void*       ws,
+                                  int         m,
+                                  int         n,
+                                  int         k,
+                                  int         share,
+                                  int         relu);
+
 // Time of such a launch per k tile of a slice, in us, with one group per workgroup: what Split_K is chosen by.
 double flashllm_hip_wide_b_step(int n, int m, int split_k);
 

@@ -95,7 +95,9 @@ int flashllm_spmm_splitk_static(void*       stream,
  *                               workgroups, which keeps every page in the L2
  *                               of the one XCD that writes and sums it.  This
  *                               is what flashllm_spmm_splitk does between its
- *                               own two kernels; the contents mean something
+ *                               own two kernels unless, for wide B, it divides
+ *                               K evenly over the GPU instead of in Split_K
+ *                               slices; the contents mean something
  *                               only to flashllm_splitk_reduce with the same
  *                               M, N, Split_K.
  */

@@ -23,6 +23,6 @@ def test_a_kernel_below_its_occupancy_stops_the_build(kernel, vgprs, occupancy):
     assert not accepted(kernel, vgprs, occupancy - 1)
 
 
-@pytest.mark.parametrize("kernel,vgprs,occupancy", [("spmm_group_kernel", 169, 3), ("spmm_wide_kernel", 241, 2), ("spmm_quarter_kernel", 225, 1)])
+@pytest.mark.parametrize("kernel,vgprs,occupancy", [("spmm_group_kernel", 169, 3), ("spmm_wide_kernel", 241, 2), ("spmm_quarter_kernel", 233, 1), ("spmm_even_kernel", 233, 1)])
 def test_a_kernel_with_more_registers_than_measured_stops_the_build(kernel, vgprs, occupancy):
     assert not accepted(kernel, vgprs, occupancy)
