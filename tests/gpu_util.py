@@ -26,7 +26,7 @@ def assert_close(c, ref, what=""):
 
 
 def run_spmm(product, a_host, b_host, n, split_k, reorder=True, poison=True):
-    """Compress on the host, run SpMM_SplitK on cuda:0 through the C ABI, return C as (N, M) fp16."""
+    """Compress (SparseWeight), run SpMM_SplitK on cuda:0 through the C ABI, return C as (N, M) fp16."""
     import torch
 
     m, k = a_host.shape
