@@ -1184,6 +1184,12 @@ __global__ __launch_bounds__(kWideWaves* kLanes, 2) void spmm_wide_kernel(const 
 //     The loop body is therefore two tiles; an early exit between them makes the compiler move accumulators and spill, so
 //     runs are whole pairs of tiles and an odd one ends with an empty tile, whose B is zeros.
 //   * Lanes past a tile's end load its last vector again and store the same items once more: no masks.
+//   * A lone wave issues an instruction in four to five clocks, so that seven fit beside an MFMA and every one more delays the next.
+//     An item's address is one instruction (v_mad_u32_u16 takes the upper half of the item; a position beyond the tile, which no
+//     compressor writes, would land in the workgroup's other LDS), M0 is set for every fourth request for B, requests are two slots
+//     apart, and scalar work is not left to the phases' ends, where nothing covers it: 690 -> 605 instructions per tile of 80 %.  Calls
+//     in turn, before and after: 7168 x 28672, N = 512 214 -> 206 us, 21504 x 7168, N = 384 126 -> 121, 36864 x 9216, N = 128, Split_K 3
+//     at 80 and 90 % 108 -> 106 and 99 -> 94, 28672 x 7168, N = 64 45.2 -> 44.0.
 //   * The stream is loaded as other data is: the column groups of a row tile sit on one XCD and share its L2 (7168 x 28672, N =
 //     512, Split_K 1 210.7 us with non-temporal loads, 202.3).
 // With 64 columns (N = 64) a tile is two such phases and one window of B, so that B is asked for two tiles ahead; a tile without
@@ -1201,8 +1207,8 @@ constexpr int kQuarterWindow = 64 * kTileCols * 2;                       // 64 c
 constexpr int kQuarterLds    = kTileHalfs * 2 + 3 * kQuarterWindow;      // a wave's: its tile and three windows of B
 using floatx16 = float __attribute__((ext_vector_type(16)));
 
-// what a tile without vectors reads: an item that stores 0 at position 0
-__device__ uint4 g_zero_vector;
+// what a tile without vectors reads: an item that stores 0 at position 0; and a tile without B, whose requests are up to 3 KB apart
+__device__ uint4 g_zeros[256];
 
 template<int NJ, int R, int X>
 __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
@@ -1245,13 +1251,13 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
         uint32_t       b_lane[4];  // where this lane's 16 bytes of 8i columns of B lie, from the first column of the 32
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            b_lane[i] = (static_cast<unsigned>(8 * i + (lane >> 3)) * static_cast<unsigned>(ldb) + (((lane & 7) ^ (lane >> 3)) << 3)) * 2;
+            b_lane[i] = (static_cast<unsigned>(8 * i + (lane >> 3)) * static_cast<unsigned>(ldb) + (((lane & 7) ^ (lane >> 3)) << 3)) * 2 - 1024 * i;
         const _Float16* bcols = B + static_cast<size_t>(col0) * ldb;
 
         half8    a[4][4], b[2][4];
         uintx4   ring[2][R];
         uintx4   rest[X];     // of a tile longer than the ring
-        Global*  nothing = (Global*)&g_zero_vector;
+        Global*  nothing = (Global*)g_zeros;
         asm volatile("" : "+s"(nothing));  // its address stays in registers
         Global*  from;        // the tile that requests are at
         uint32_t from_last;   // byte of its last vector
@@ -1275,9 +1281,9 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
             slot = *reinterpret_cast<const __attribute__((address_space(1))) uintx4*>(from + (at < from_last ? at : from_last));
         };
         auto scatter = [&](uint32_t item) {
-            uint32_t position;
-            asm("v_bfe_u32 %0, %1, 16, 13" : "=v"(position) : "v"(item));
-            *reinterpret_cast<Lds16*>(position * 2 + tile_l) = static_cast<uint16_t>(item);
+            uint32_t at;  // 2 * position + tile_l
+            asm("v_mad_u32_u16 %0, %1, 2, %2 op_sel:[1,0,0,0]" : "=v"(at) : "v"(item), "s"(tile_l));
+            *reinterpret_cast<Lds16*>(at) = static_cast<uint16_t>(item);
         };
         // a tile of more than R chunks: chunks R .. R + X - 1 of it; lanes past its end as above
         auto request_rest = [&](int r, int chunk) {
@@ -1324,8 +1330,18 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
             return Half{there ? (Global*)(NJ == 4 ? bcols + (half & 1) * (64 * static_cast<size_t>(ldb)) + (half >> 1) * kTileCols : bcols + half * kTileCols) : nothing,
                         there ? 64 * static_cast<size_t>(ldb) : 0, there ? ~0u : 0u};
         };
+        // eight requests in a row: M0 is set for every fourth, between them the instruction's offset counts in LDS and in memory
         auto fetch_b = [&](const Half& half, uint32_t window, int i) {
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(b_lane[i % 4] & half.lanes), "s"(half.first + (i / 4) * half.step), "s"(window + i * 1024) : "memory", "m0");
+            const uint32_t at    = b_lane[i % 4] & half.lanes;
+            Global* const  first = half.first + (i / 4) * half.step;
+            if (i % 4 == 0)
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(at), "s"(first), "s"(window + i * 1024) : "memory", "m0");
+            else if (i % 4 == 1)
+                asm volatile("global_load_lds_dwordx4 %0, %1 offset:1024" ::"v"(at), "s"(first) : "memory");
+            else if (i % 4 == 2)
+                asm volatile("global_load_lds_dwordx4 %0, %1 offset:2048" ::"v"(at), "s"(first) : "memory");
+            else
+                asm volatile("global_load_lds_dwordx4 %0, %1 offset:3072" ::"v"(at), "s"(first) : "memory");
         };
         auto multiply = [&](int p, int m) {
             const int s = 2 * (p & 1) + m / 8, i = m / 2 % 4, j = 2 * (p / 2) + m % 2;
@@ -1393,33 +1409,40 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
         keep();
 
         constexpr int R0 = (R + 1) / 2, R1 = R - R0;
+        auto clear_some = [&](int m, int s) {  // k steps s and s + 1, behind their reads
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                if (m == 5 + i * 11 / 8)
+                    clear_a(s + i / 4, i % 4);
+        };
         auto tile_of_128 = [&](auto slot, int t) {
             uintx4(&next)[R] = ring[decltype(slot)::value];
             expect_rest();
+            Half b_half1, b_half0;  // what phases 1 and 3 ask for
             // phase 0: half 0 of B, k steps 0 and 1
 #pragma unroll
             for (int m = 0; m < 16; m++) {
                 multiply(0, m);
+                if (m == 5)
+                    b_half1 = half_of_b(2 * t + 3);
                 if (m < 4)
                     read_b(1, w0, m);
                 else if (m < 12)
                     read_a(2 + (m - 4) / 4, m % 4);
-                if (m >= 8)
-                    clear_a(2 + (m - 8) / 4, m % 4);
+                clear_some(m, 2);
                 keep();
             }
             // phase 1: half 0, k steps 2 and 3.  Half 1 has landed; half 0 is out of LDS
             asm volatile("" ::"v"(b[1][0]), "v"(b[1][1]), "v"(b[1][2]), "v"(b[1][3]) : "memory");
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + R1) : "memory");
-            const Half b_half1 = half_of_b(2 * t + 3);
             keep();
 #pragma unroll
             for (int m = 0; m < 16; m++) {
                 multiply(1, m);
                 if (m < 4)
                     read_b(2, w1, m);
-                if (m < 8)
-                    fetch_b(b_half1, w0, m);
+                if (m % 2 == 0)
+                    fetch_b(b_half1, w0, m / 2);
 #pragma unroll
                 for (int i = m * R0 * 4 / 16; i < (m + 1) * R0 * 4 / 16; i++) {
                     scatter(next[i / 4][i % 4]);
@@ -1434,6 +1457,8 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
                 multiply(2, m);
                 if (m < 4)
                     read_b(3, w1, m);
+                if (m == 4)
+                    b_half0 = half_of_b(2 * t + 4);
 #pragma unroll
                 for (int i = m * R1 * 4 / 16; i < (m + 1) * R1 * 4 / 16; i++) {
                     scatter(next[R0 + i / 4][i % 4]);
@@ -1448,8 +1473,6 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
             // phase 3: half 1, k steps 2 and 3.  Half 0 of the next tile has landed; this tile's B is out of LDS
             asm volatile("" ::"v"(b[1][0]), "v"(b[1][1]), "v"(b[1][2]), "v"(b[1][3]) : "memory");
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + R) : "memory");
-            const Half b_half0 = half_of_b(2 * t + 4);
-            next_tile(t + 4);
             keep();
 #pragma unroll
             for (int m = 0; m < 16; m++) {
@@ -1458,10 +1481,11 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
                     read_b(0, w2, m);
                 else if (m < 12)
                     read_a((m - 4) / 4, m % 4);
-                if (m >= 8)
-                    clear_a((m - 8) / 4, m % 4);
-                if (m < 8)
-                    fetch_b(b_half0, w1, m);
+                clear_some(m, 0);
+                if (m % 2 == 0)
+                    fetch_b(b_half0, w1, m / 2);
+                if (m == 13)
+                    next_tile(t + 4);
                 keep();
             }
             // next tile: half 0 is in w2, half 1 on its way to w0, the half 0 after it on its way to w1
