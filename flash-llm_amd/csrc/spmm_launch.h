@@ -122,6 +122,28 @@ int flashllm_hip_launch_encode_scan(void* stream, const void* a, int m, int k, c
 // instead, or gives them back.  Returns how many.
 int flashllm_hip_hold_host_words(int take);
 
+// A weight on its way to the GPU without its zeros, in pieces of 65536 halfs: the index of the first value of each of its 32 groups
+// (4 bytes), a bit per half, the values whose bits are not all zero, and room for what a 16-byte store writes beyond them.
+enum {
+    kPackPiece  = 65536,
+    kPackGroup  = 2048,
+    kPackBits   = kPackPiece / kPackGroup * 4,
+    kPackValues = kPackBits + kPackPiece / 8,
+    kPackStride = kPackValues + kPackPiece * 2 + 128
+};
+
+// One piece of n halfs (at most kPackPiece, a multiple of kPackGroup) at src, at dst.  Host only.
+void flashllm_pack_piece(const unsigned short* src, size_t n, unsigned char* dst);
+
+// Threads that the host compressor would take for so many pieces of work.
+int flashllm_compress_workers(size_t pieces);
+
+// The same matrix at dst (device memory, 16-byte aligned) as flashllm_hip_upload leaves there, by way of packed pieces in stage (pinned
+// host memory, 16-byte aligned, at least flashllm_hip_upload_stage() bytes) that a kernel fetches and expands.  n halfs, a multiple of
+// kPackGroup.  Waits for it.
+int    flashllm_hip_upload_packed(void* stream, void* dst, const void* src, size_t n, void* stage);
+size_t flashllm_hip_upload_stage(void);
+
 // Copies ordinary host memory to the GPU and waits for it.
 int flashllm_hip_upload(void* stream, void* dst, const void* src, size_t bytes);
 

@@ -31,6 +31,10 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+#include <thread>
+#include <vector>
+
 namespace {
 
 constexpr int kTileRows = 128;
@@ -519,6 +523,60 @@ __global__ __launch_bounds__(kEncodeThreads) void encode_tiles_scan_kernel(const
         __builtin_nontemporal_store(reinterpret_cast<const uintx4*>(list)[v], to + v);
 }
 
+// Packed pieces (spmm_launch.h) in pinned host memory -> the dense matrix.  One workgroup per group of 2048 halfs, a byte of the bits and
+// eight halfs to a thread; the group's values come through LDS, so that what crosses the link is whole 16-byte vectors.  The kernel fetches
+// them itself because the pieces lie a full piece apart (a copy would carry that) and 25 launches do for 7168 x 7168.  Bound by the
+// link and the threads that pack: 27 of its 103 MB at 80 %, 1.1 ms.
+constexpr int kExpandThreads = kPackGroup / 8;
+
+__global__ __launch_bounds__(kExpandThreads) void expand_kernel(const unsigned char* __restrict__ pieces, uintx4* __restrict__ dst)
+{
+    __shared__ uintx4 values[kExpandThreads + 1];
+    __shared__ int    total[kExpandThreads / kLanes];
+    constexpr int        kGroups = kPackPiece / kPackGroup;
+    const int            tid = threadIdx.x, lane = tid & (kLanes - 1), wave = tid / kLanes;
+    const unsigned char* piece = pieces + static_cast<size_t>(blockIdx.x / kGroups) * kPackStride;
+    const int            group = blockIdx.x % kGroups;
+    const uint32_t       first = reinterpret_cast<const uint32_t*>(piece)[group];
+    const uint32_t       bits  = piece[kPackBits + group * (kPackGroup / 8) + tid];
+    const int            mine = __builtin_popcount(bits), inclusive = wave_scan(mine);
+    if (lane == kLanes - 1)
+        total[wave] = inclusive;
+    __syncthreads();
+    int before = inclusive - mine, all = 0;
+#pragma unroll
+    for (int w = 0; w < kExpandThreads / kLanes; w++) {
+        before += w < wave ? total[w] : 0;
+        all += total[w];
+    }
+    const uint32_t skip    = first & 7;  // values in front of the group's in its first vector
+    const int      vectors = (static_cast<int>(skip) + all + 7) / 8;
+    const uintx4*  from    = reinterpret_cast<const uintx4*>(piece + kPackValues) + first / 8;
+    if (tid < vectors)
+        values[tid] = from[tid];
+    if (tid == 0 && vectors > kExpandThreads)
+        values[kExpandThreads] = from[kExpandThreads];
+    __syncthreads();
+    const uint16_t* at = reinterpret_cast<const uint16_t*>(values) + skip + before;
+    uintx4          v;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const uint32_t lo = bits >> (2 * e) & 1, hi = bits >> (2 * e + 1) & 1;
+        const uint32_t a = lo ? *at : 0;
+        at += lo;
+        const uint32_t b = hi ? *at : 0;
+        at += hi;
+        v[e] = a | b << 16;
+    }
+    dst[static_cast<size_t>(blockIdx.x) * kExpandThreads + tid] = v;
+}
+
+// The pinned memory is a ring of parts, each of them one launch: while the GPU fetches one part, the threads pack the ones after it.
+// 7168 x 7168, 80 %, whole load with 12 threads: 4 parts of 32 pieces 1.29 ms, 8 of 16 1.22, 16 of 16 1.22, 8 of 32 1.04; seven of 32
+// stay below 32 MB, to which torch rounds up.
+constexpr int kPartPieces = 32;
+constexpr int kParts      = 7;
+
 }  // namespace
 
 extern "C" int flashllm_hip_launch_tile_offsets(void* stream, const void* a, int m, int k, int* offs, int* vectors)
@@ -539,13 +597,90 @@ extern "C" int flashllm_hip_launch_tile_offsets(void* stream, const void* a, int
     return static_cast<int>(hipGetLastError());
 }
 
-// 28 GB/s from pageable memory (7168 x 7168, 3.6 ms), and staged through a ring of pinned pieces that eight threads fill 30 (3.4 ms); the
-// link carries 57 from pinned memory (1.9 ms).  Two halves from two threads take 2.8 ms on some pairs of streams and 4.6 on others.
+// 28 GB/s from pageable memory: 7168 x 7168 in 3.6 ms.
 extern "C" int flashllm_hip_upload(void* stream, void* dst, const void* src, size_t bytes)
 {
     hipStream_t      s = static_cast<hipStream_t>(stream);
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
     return static_cast<int>(e == hipSuccess ? hipStreamSynchronize(s) : e);
+}
+
+extern "C" size_t flashllm_hip_upload_stage(void)
+{
+    return static_cast<size_t>(kParts) * kPartPieces * kPackStride;
+}
+
+// The host's threads leave the zeros out (they read the matrix faster than the link carries it), and what is left crosses the link once,
+// read by the kernel that expands it.  Only the calling thread talks to the runtime.
+extern "C" int flashllm_hip_upload_packed(void* stream, void* dst, const void* src, size_t n, void* stage)
+{
+    hipStream_t  s      = static_cast<hipStream_t>(stream);
+    const size_t pieces = (n + kPackPiece - 1) / kPackPiece, parts = (pieces + kPartPieces - 1) / kPartPieces;
+    const auto*  from   = static_cast<const unsigned short*>(src);
+    auto*        ring   = static_cast<unsigned char*>(stage);
+    if (n == 0 || n % kPackGroup)
+        return static_cast<int>(hipErrorInvalidValue);
+    hipEvent_t free_again[kParts];
+    int        events = 0;
+    hipError_t e      = hipSuccess;
+    while (events < kParts && (e = hipEventCreateWithFlags(&free_again[events], hipEventDisableTiming)) == hipSuccess)
+        events++;
+
+    std::atomic<size_t> next{0}, allowed{kParts};  // the next piece to pack; parts that have a place in the ring
+    std::atomic<int>    packed[kParts];            // pieces of the part in that place that are ready
+    std::atomic<bool>   stop{e != hipSuccess};
+    for (auto& p : packed)
+        p.store(0, std::memory_order_relaxed);
+    auto pack_one = [&]() {  // false: nothing to do now
+        size_t piece = next.load(std::memory_order_relaxed);
+        do
+            if (piece >= pieces || piece / kPartPieces >= allowed.load(std::memory_order_acquire))
+                return false;
+        while (!next.compare_exchange_weak(piece, piece + 1, std::memory_order_relaxed));
+        const size_t first = piece * kPackPiece, slot = piece % (kParts * kPartPieces);
+        flashllm_pack_piece(from + first, n - first < kPackPiece ? n - first : kPackPiece, ring + slot * kPackStride);
+        packed[slot / kPartPieces].fetch_add(1, std::memory_order_release);
+        return true;
+    };
+    std::vector<std::thread> pool;
+    try {  // a thread that cannot be created is left out
+        // a thread for eight pieces: 2048 x 2048 0.21 ms with 6 threads, 0.36 with 16
+        const int workers = flashllm_compress_workers(pieces / 8);
+        pool.reserve(workers);
+        for (int w = 1; w < workers; w++)
+            pool.emplace_back([&]() {
+                while (!stop.load(std::memory_order_relaxed) && next.load(std::memory_order_relaxed) < pieces)
+                    if (!pack_one())
+                        std::this_thread::yield();
+            });
+    }
+    catch (...) {
+    }
+    for (size_t p = 0; p < parts && e == hipSuccess; p++) {
+        const size_t first = p * kPartPieces, count = pieces - first < kPartPieces ? pieces - first : kPartPieces;
+        const int    place = static_cast<int>(p % kParts);
+        while (packed[place].load(std::memory_order_acquire) < static_cast<int>(count))
+            if (!pack_one())
+                std::this_thread::yield();
+        packed[place].store(0, std::memory_order_relaxed);
+        const size_t start = first * kPackPiece, halfs = n - start < count * kPackPiece ? n - start : count * kPackPiece;
+        hipLaunchKernelGGL(expand_kernel, dim3(static_cast<unsigned>(halfs / kPackGroup)), dim3(kExpandThreads), 0, s,
+                           ring + static_cast<size_t>(place) * kPartPieces * kPackStride, static_cast<uintx4*>(dst) + start / 8);
+        e = hipGetLastError();
+        if (e == hipSuccess)
+            e = hipEventRecord(free_again[place], s);
+        if (e == hipSuccess && p + 2 >= kParts) {  // part p + 2 follows part p + 2 - kParts
+            e = hipEventSynchronize(free_again[(p + 2) % kParts]);
+            allowed.store(p + 3, std::memory_order_release);
+        }
+    }
+    stop.store(true, std::memory_order_relaxed);
+    for (auto& t : pool)
+        t.join();
+    const hipError_t done = hipStreamSynchronize(s);  // the ring is the caller's again
+    for (int i = 0; i < events; i++)
+        static_cast<void>(hipEventDestroy(free_again[i]));
+    return static_cast<int>(e == hipSuccess ? done : e);
 }
 
 extern "C" int flashllm_hip_encode_status(void* stream, unsigned int* status)

@@ -305,6 +305,26 @@ def test_loaded_weight_has_the_host_compressors_bytes(product, torch_gpu, form, 
     assert np.array_equal(w.offs.cpu().numpy(), offsets)
 
 
+@pytest.mark.parametrize("threads", [1, 16])
+@pytest.mark.parametrize("shape", [(128, 64), (1024, 1024), (1152, 1088), (4096, 4096), (7168, 2048)])
+def test_a_matrix_arrives_whole_without_its_zeros_on_the_way(product, torch_gpu, monkeypatch, shape, threads):
+    """Pieces of 65536 halfs, parts of 32 of them, seven parts in the ring: less than a piece, a part, a piece and a bit more than whole
+    parts, the ring gone round.  Every bit pattern that is not zero comes back, -0 and NaN too."""
+    say("packed upload:", shape, threads)
+    rng = np.random.default_rng(shape[0])
+    a = synth.sparse_matrix(*shape, 0.8, 52).view(np.uint16).copy()
+    a[::5] = rng.integers(0, 65536, a[::5].shape, dtype=np.uint16)
+    a[3::7] = 0
+    a[1::9, ::2] = 0x8000
+    monkeypatch.setattr(product, "UPLOAD_PACKED_BYTES", 1)
+    product.lib().flashllm_set_compress_threads(threads)
+    try:
+        for _ in range(3):
+            assert np.array_equal(product._upload(a).cpu().numpy().view(np.uint16), a)
+    finally:
+        product.lib().flashllm_set_compress_threads(0)
+
+
 def test_loading_refuses_what_the_host_compressor_refuses(product, torch_gpu):
     for bad in (np.zeros((100, 64), np.float16), np.zeros((128, 96), np.float16), np.zeros((0, 64), np.float16)):
         with pytest.raises(product.CompressError):
