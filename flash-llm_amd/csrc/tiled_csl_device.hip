@@ -21,11 +21,10 @@
 // once: 1.2 GB at 27648 x 9216 and 80 %, HBM-bound when every access is a whole line.  So the count reads 1 KB of a
 // row per load, and the encoder sorts a tile into output order in LDS and stores it as consecutive 16-byte vectors:
 // with every item storing its own 4 bytes at its destination (a line of its own per lane) and one wave counting 128-byte
-// pieces of eight rows at a time the call took 550 us; now 268, and 243 with non-temporal loads and stores (a trace of
-// the former: count 95, encoder 147, i.e. 5.3 and 4.9 TB/s).  About 25 us are a fixed cost: launches, the prefix sum
+// pieces of eight rows at a time the call took 550 us; as it is now 222 (count 76, encoder 122, i.e. 6.7 and 5.9 TB/s).  About 25 us are a fixed cost: launches, the prefix sum
 // and the host's wait for its total, which the kernel stores to host memory itself (2048 x 4096: 35.8 us; 44.1 with a copy
 // of it).  Encoding the tiles last counted first, while they may still be in the Infinity Cache, gains nothing (27648 x
-// 9216: 140 us either way, with cached loads in either kernel or both too).
+// 9216: 122 us either way, with cached loads in either kernel or both too).
 #include "spmm_launch.h"
 
 #include <hip/hip_runtime.h>
@@ -237,6 +236,52 @@ __global__ __launch_bounds__(kLanes* kScanWaves) void scan_offsets_kernel(int* _
     }
 }
 
+// the reference's compare, as above, of one half of a word: finite or infinite and no zero.  By class, with the classes out of the
+// compiler's sight, which makes an ordered compare with zero of them and then, under a ballot, one that NaN passes.
+__device__ __forceinline__ bool keeps_half(uint32_t word, int half)
+{
+    using half2v = _Float16 __attribute__((ext_vector_type(2)));
+    int classes  = 0x39c;
+    asm("" : "+s"(classes));
+    return __builtin_amdgcn_classh(__builtin_bit_cast(half2v, word)[half], classes);
+}
+
+__device__ __forceinline__ uint32_t lds_address(const void* p)
+{
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)(p)));
+}
+
+// Four items to LDS, each at `at` in the lanes of its mask, which step on by STEP bytes: two vector instructions an item, where a branch
+// on a lane's own bit takes five.  For whole waves.  lds_done() waits for these stores, which the compiler does not count.
+template<int STEP>
+__device__ __forceinline__ void store_and_step(uint32_t& at, const uint32_t (&item)[4], const uint64_t (&mask)[4])
+{
+    asm volatile("s_mov_b64 exec, %5\n\tds_write_b32 %0, %1\n\tv_add_u32_e32 %0, %9, %0\n\t"
+                 "s_mov_b64 exec, %6\n\tds_write_b32 %0, %2\n\tv_add_u32_e32 %0, %9, %0\n\t"
+                 "s_mov_b64 exec, %7\n\tds_write_b32 %0, %3\n\tv_add_u32_e32 %0, %9, %0\n\t"
+                 "s_mov_b64 exec, %8\n\tds_write_b32 %0, %4\n\tv_add_u32_e32 %0, %9, %0\n\t"
+                 "s_mov_b64 exec, -1"
+                 : "+v"(at)
+                 : "v"(item[0]), "v"(item[1]), "v"(item[2]), "v"(item[3]), "s"(mask[0]), "s"(mask[1]), "s"(mask[2]), "s"(mask[3]), "n"(STEP)
+                 : "memory");
+}
+
+__device__ __forceinline__ void store_where(uint32_t at, uint32_t item, uint64_t mask)
+{
+    asm volatile("s_mov_b64 exec, %2\n\tds_write_b32 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(at), "v"(item), "s"(mask) : "memory");
+}
+
+__device__ __forceinline__ uint32_t min_pair(uint32_t a, uint32_t b)
+{
+    using ushort2v = uint16_t __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(ushort2v, a), __builtin_bit_cast(ushort2v, b)));
+}
+
+__device__ __forceinline__ void lds_done()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
+
 // The encoder: one workgroup of four waves per tile.
 //
 // Element (m, n) lives at swizzled column sw = n ^ ((m % 8) << 3) (csrc/SpMM_API.cu:252-256); bank sw / 2 owns the word
@@ -245,19 +290,26 @@ __global__ __launch_bounds__(kLanes* kScanWaves) void scan_offsets_kernel(int* _
 //   1. counts of all (bank, segment) meet in LDS: fills, heights, padding (every wave works it out for itself);
 //   2. every thread lists its nonzeros by (height, bank) in LDS;
 //   3. level by level: an item of the level is pop number  (items on higher levels) + (banks before it that reach the
-//      level), a sum and a ballot over the half wave that holds the level; the items move to that place, through
+//      level), a sum over the banks and a ballot over the half wave that holds the level; the items move to that place, through
 //      registers because the list and the pops share their LDS;
 //   4. vector v of the tile gathers its four items, which lie 32 pops apart, and is stored whole.
-// The list holds 128 levels (16 KB; the registers, 79, allow six workgroups per CU).  A tile in which a bank holds more
+// Every element passes through a dozen vector instructions, and those, not memory, were the bound (685 per wave, the units busy all of
+// the time; scalar ones 335): now a compare per half, whose mask the store goes by, two more instructions for the store itself, the sums of
+// all levels at once in 16 lanes, row addresses in scalar registers; 493 and 349.  27648 x 9216, 80 %: 133.8 -> 121.7 us (5.9 TB/s;
+// without its stores 104), 90 % 120 -> 106, 70 % 149 -> 142, 7168 x 7168 32.2 -> 28.9.  Seven or eight workgroups per CU instead of six,
+// with fewer masks held: 3 % faster at 90 %, 4 to 7 % slower at 70 %.
+// The list holds 128 levels (16 KB; the registers, 73, allow six workgroups per CU).  A tile in which a bank holds more
 // (beyond about 45 % of all its elements) takes each item's pop number from a table of the levels instead, and the list in
-// two parts: the pops that fit, up to the end of a pass of four, then the rest.  27648 x 9216, both calls: 332 us at 50 %
-// and 383 at 20 % sparsity (589 and 818 when every nonzero stored itself to its place in memory; 252 at 70 %).
+// two parts: the pops that fit, up to the end of a pass of four, then the rest.  27648 x 9216, both calls: 320 us at 50 %
+// and 366 at 20 % sparsity (589 and 818 when every nonzero stored itself to its place in memory; 244 at 70 %).
 constexpr int kEncodeThreads = 256;
+constexpr int kFarColumns    = 1 << 26;  // FAR: from here on; sixteen rows of fewer are less than 4 GB
 constexpr int kSegments      = kEncodeThreads / kBanks;
 constexpr int kRowsOfThread  = kTileRows / kSegments;
 constexpr int kLevels        = 128;
 constexpr int kLevelsAtOnce  = kEncodeThreads / kBanks;
 
+template<bool FAR>
 __global__ __launch_bounds__(kEncodeThreads, 6) void encode_tiles_kernel(const uint16_t* __restrict__ a,
                                                                        int k,
                                                                        int tiles_per_row,
@@ -266,37 +318,54 @@ __global__ __launch_bounds__(kEncodeThreads, 6) void encode_tiles_kernel(const u
 {
     __shared__ uint32_t list[kLevels * kBanks];            // [height - 1][bank]; then the pops in order
     __shared__ __attribute__((aligned(8))) uint8_t count_s[kBanks][kSegments];
-    __shared__ __attribute__((aligned(8))) uint8_t zero_s[kBanks][kSegments];  // the segment's first zero, 0xff: none
-    __shared__ int   fill_s[kBanks];                       // from here on only for tiles beyond the list
-    __shared__ uint2 level[kMaxFill + 1];                  // items higher than h, over all banks; banks holding at least h
+    __shared__ __attribute__((aligned(16))) uint16_t fill_s[kBanks];
+    __shared__ uint2 level[kMaxFill + 1];                  // only for tiles beyond the list: items higher than h, over all banks; banks holding at least h
 
     const int       t    = blockIdx.x;
     const int       tid  = threadIdx.x;
     const int       bank = tid & (kBanks - 1), segment = tid / kBanks;
-    const uint16_t* base = tile_base(a, k, tiles_per_row, t) + static_cast<size_t>(segment) * kRowsOfThread * k;
 
     uint32_t word[kRowsOfThread];
+    if constexpr (!FAR) {  // an offset of 32 bits from an address of the wave's, one vector instruction a row instead of three
+        const uint16_t* base = tile_base(a, k, tiles_per_row, t) + static_cast<size_t>(__builtin_amdgcn_readfirstlane(tid / kLanes)) * (2 * kRowsOfThread) * k;
+        const uint32_t  from = (tid & 32) * static_cast<uint32_t>(k);
 #pragma unroll
-    for (int i = 0; i < kRowsOfThread; i++)
-        word[i] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(base + static_cast<size_t>(i) * k + (((bank >> 2) ^ (i & 7)) * 4 + (bank & 3)) * 2));
+        for (int i = 0; i < kRowsOfThread; i++)
+            word[i] = __builtin_nontemporal_load(
+                reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(base + static_cast<size_t>(i) * k) + (from + ((bank * 4u) ^ ((i & 7) * 16u)))));
+    }
+    else {
+        const uint16_t* base = tile_base(a, k, tiles_per_row, t) + static_cast<size_t>(segment) * kRowsOfThread * k;
+#pragma unroll
+        for (int i = 0; i < kRowsOfThread; i++)
+            word[i] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(base + static_cast<size_t>(i) * k + (((bank >> 2) ^ (i & 7)) * 4 + (bank & 3)) * 2));
+    }
     const int first = offs[t], room = (offs[t + 1] - first) * 4;
 
-    uint32_t kept = 0;  // bit i + 16e: half e of row i
+    // The lanes that keep half e of row i.  There are scalar registers to hold those of six rows; the others are compared once more.
+    constexpr int kHeldRows = 6;
+    uint64_t      keeps[2 * kHeldRows];
+    int           mine = 0;
+#pragma unroll
+    for (int i = 0; i < kRowsOfThread; i++) {
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const bool kept  = keeps_half(word[i], e);
+            if (i < kHeldRows)
+                keeps[2 * i + e] = __builtin_amdgcn_ballot_w64(kept);
+            mine += kept;
+        }
+    }
+    count_s[bank][segment] = static_cast<uint8_t>(mine);
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < kRowsOfThread; i++)
-        kept |= keeps_pair(word[i]) << i;
-    {
-        const int lo = __builtin_ctz(~kept | 0x10000u), hi = __builtin_ctz((~kept >> 16) | 0x10000u);
-        const int zero = 2 * lo < 2 * hi + 1 ? 2 * lo : 2 * hi + 1;
-        count_s[bank][segment] = static_cast<uint8_t>(__builtin_popcount(kept));
-        zero_s[bank][segment]  = static_cast<uint8_t>(zero < 2 * kRowsOfThread ? zero : 0xff);
-    }
-    __syncthreads();
+        asm volatile("" : "+v"(word[i]));  // compared again where the masks are wanted, not kept in spilled registers
 
     // this thread's bank: its fill (both halves of every wave hold all banks) and the items below this segment
-    int fill, below;
+    int         fill, below;
+    const uint2 c = *reinterpret_cast<const uint2*>(&count_s[bank][0]);
     {
-        const uint2    c    = *reinterpret_cast<const uint2*>(&count_s[bank][0]);
         const uint32_t low  = segment < 4 ? (1u << (8 * segment)) - 1u : 0xffffffffu;
         const uint32_t high = segment < 4 ? 0u : (1u << (8 * (segment - 4))) - 1u;
         fill  = static_cast<int>(__builtin_amdgcn_sad_u8(c.y, 0u, __builtin_amdgcn_sad_u8(c.x, 0u, 0u)));
@@ -309,24 +378,32 @@ __global__ __launch_bounds__(kEncodeThreads, 6) void encode_tiles_kernel(const u
     const int pad      = (4 - nnz % 4) % 4;
     for (int p = 0; p < pad; p++)
         fill += (half_min((fill << 5) | bank) & (kBanks - 1)) == bank;
+    // The thread whose segment has that position puts the bank's padding items there.
     uint32_t pad_item = 0;
+    bool     pads     = false;
     if (fill > unpadded) {
-        const uint64_t z = *reinterpret_cast<const uint64_t*>(&zero_s[bank][0]);
-        if (~z == 0) {  // cannot happen: the emptiest bank holds fewer than 256 items
+        const uint64_t full = (static_cast<uint64_t>(c.y) << 32 | c.x) ^ 0x0101010101010101ull * (2 * kRowsOfThread);
+        if (full == 0) {  // cannot happen: the emptiest bank holds fewer than 256 items
             if (segment == 0)
                 report(FLASHLLM_ENCODE_NO_ZERO);
         }
-        else {
-            const int s = __builtin_ctzll(~z) / 8;
-            const int i = s * (2 * kRowsOfThread) + static_cast<int>((z >> (8 * s)) & 0xff);
-            pad_item    = static_cast<uint32_t>((i >> 1) * kTileCols + 2 * bank + (i & 1)) << 16;
+        else if (__builtin_ctzll(full) / 8 == segment) {
+            pads       = true;
+            int z      = 0;
+#pragma unroll
+            for (int i = 2 * kRowsOfThread - 1; i >= 0; i--)
+                z = keeps_half(word[i / 2], i % 2) ? z : i;
+            pad_item = static_cast<uint32_t>((segment * kRowsOfThread + (z >> 1)) * kTileCols + 2 * bank + (z & 1)) << 16;
         }
     }
+#pragma unroll
+    for (int i = 0; i < kRowsOfThread; i++)
+        asm volatile("" : "+v"(word[i]));
     const int count = nnz + pad;
     const int top   = __builtin_amdgcn_readfirstlane(half_max(fill));
 
-    const int vectors    = count / 4;
-    const int rep        = vectors / kBanks, rem = vectors % kBanks;
+    const int vectors    = count >> 2;
+    const int rep        = vectors >> 5, rem = vectors & (kBanks - 1);
     const int tail_items = rem * 4;
     uint32_t* out_tile   = out + static_cast<size_t>(first) * 4;
     // Never write outside this tile's range of Compressed_A, whatever TileOffsets says: with offsets that were
@@ -334,63 +411,90 @@ __global__ __launch_bounds__(kEncodeThreads, 6) void encode_tiles_kernel(const u
     const int space = count < room ? count : room;
     if (room != count && tid == 0)
         report(FLASHLLM_ENCODE_OFFSETS);
-    const uint32_t first_position = static_cast<uint32_t>(segment * kRowsOfThread * kTileCols + 2 * bank) << 16;
+    // positions of the two halves of this thread's first row; a row further each is 64 more
+    const uint32_t first_positions = static_cast<uint32_t>(segment * kRowsOfThread * kTileCols + 2 * bank) * 0x10001u + 0x10000u;
+    auto           item_of         = [&](int i, int e, uint32_t positions) {
+        return __builtin_amdgcn_perm(positions, word[i], e ? 0x07060302u : 0x05040100u);
+    };
 
     // vector v out of the list, which holds the pops from `from` on
     auto store_vector = [&](int v, int from) {
         // a vector of the main part: pops of four passes, last pass first; of the tail (drained first): every rem-th
         const bool main = v < rep * kBanks;
         const int  step = main ? kBanks : rem;
-        const int  last = (main ? tail_items + (rep - 1 - v / kBanks) * (4 * kBanks) + v % kBanks : v - rep * kBanks) - from;
+        const int  last = (main ? tail_items + (rep - 1 - (v >> 5)) * (4 * kBanks) + (v & (kBanks - 1)) : v - rep * kBanks) - from;
         __builtin_nontemporal_store(uintx4{list[last + 3 * step], list[last + 2 * step], list[last + step], list[last]}, reinterpret_cast<uintx4*>(out_tile) + v);
     };
 
     if (top <= kLevels) {
-        uint32_t* at = &list[below * kBanks + bank];
+        uint32_t       at        = lds_address(list) + (below * kBanks + bank) * 4;
+        uint32_t       positions = first_positions;
 #pragma unroll
-        for (int i = 0; i < kRowsOfThread; i++) {
-            const uint32_t position = first_position + (static_cast<uint32_t>(i * kTileCols) << 16);
-            if (kept & (1u << i)) {
-                *at = (word[i] & 0xffffu) | position;
-                at += kBanks;
+        for (int i = 0; i < kRowsOfThread; i += 2) {
+            uint32_t item[4];
+            uint64_t mask[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                item[j] = item_of(i + j / 2, j % 2, positions + j / 2 * (kTileCols * 0x10001u));
+                mask[j] = i < kHeldRows ? keeps[2 * (i % kHeldRows) + j] : __builtin_amdgcn_ballot_w64(keeps_half(word[i + j / 2], j % 2));
             }
-            if (kept & (1u << (i + 16))) {
-                *at = (word[i] >> 16) | (position + 0x10000u);
-                at += kBanks;
-            }
+            store_and_step<kBanks * 4>(at, item, mask);
+            positions += 2 * kTileCols * 0x10001u;
         }
-        if (segment == 0)
+        if (tid < kBanks)
+            fill_s[tid] = static_cast<uint16_t>(fill);
+        if (pads)
             for (int h = unpadded; h < fill; h++)
                 list[h * kBanks + bank] = pad_item;
+        lds_done();
         __syncthreads();
 
+        // Two levels at a time by the halves of a wave, 8i + 2w + 1 and + 2 in step i of wave w.  An item of a level comes after
+        // those of the levels above it, which are all items but those up to this level.  Lane l of each sixteen works out how many
+        // lie below step l's two levels, sum_b min(fill[b], 8l + 2w): eight banks to a lane, which go together in pairs and quarters.
+        const int      wave  = __builtin_amdgcn_readfirstlane(tid / kLanes);
+        const uint32_t half  = tid & 32 ? ~0u : 0u;
+        const int      high  = fill + static_cast<int>(half);
+        int            under = 0;
+        {
+            const uintx4   fills = *reinterpret_cast<const uintx4*>(&fill_s[(tid & (kLanes - 1)) / 16 * 8]);
+            const uint32_t most  = ((tid & 15) * kLevelsAtOnce + 2 * wave) * 0x10001u;
+            uint32_t       sum   = 0;  // two halfs of at most 4 * 128
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                sum += min_pair(fills[j], most);
+            under = static_cast<int>((sum & 0xffffu) + (sum >> 16));
+            under += __builtin_amdgcn_ds_swizzle(under, 0x401f);  // lane ^ 16
+        }
         uint32_t item[kLevels / kLevelsAtOnce];
-        int      pop[kLevels / kLevelsAtOnce];
+        uint32_t pop[kLevels / kLevelsAtOnce];
+        uint64_t here[kLevels / kLevelsAtOnce];
+        uint64_t beyond = 0;
 #pragma unroll
         for (int i = 0; i < kLevels / kLevelsAtOnce; i++) {
-            pop[i] = -1;
+            here[i] = 0;
             if (i * kLevelsAtOnce < top) {
-                const int      h      = i * kLevelsAtOnce + segment + 1;
-                const uint64_t have   = __builtin_amdgcn_ballot_w64(fill >= h);  // one level per half wave
-                const int      higher = half_sum(fill > h ? fill - h : 0);
-                if (fill >= h) {
-                    const int before = (tid & 32) ? __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(have >> 32), 0u)
-                                                  : __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(have), 0u);
-                    item[i] = list[(h - 1) * kBanks + bank];
-                    pop[i]  = higher + before;
-                }
+                item[i] = list[(i * kLevelsAtOnce + segment) * kBanks + bank];
+                const int      lower = __builtin_amdgcn_readlane(under, i) + __builtin_amdgcn_readlane(under, 32 + i);
+                const uint64_t have  = __builtin_amdgcn_ballot_w64(high > i * kLevelsAtOnce + 2 * wave);
+                const uint32_t lo    = static_cast<uint32_t>(have), hi = static_cast<uint32_t>(have >> 32);
+                // the upper half's lanes count those of the lower level as before them, and its own are not before them
+                const uint32_t above = count - lower - __builtin_popcount(lo);
+                const uint32_t base  = above - (half & __builtin_popcountll(have));
+                pop[i]               = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, base));
+                here[i]              = have & __builtin_amdgcn_ballot_w64(pop[i] < static_cast<uint32_t>(count));
+                beyond |= have ^ here[i];
             }
         }
+        if (beyond && tid % kLanes == 0)  // cannot happen while the closed form is right
+            report(FLASHLLM_ENCODE_RANGE);
         __syncthreads();
+        const uint32_t to = lds_address(list);
 #pragma unroll
-        for (int i = 0; i < kLevels / kLevelsAtOnce; i++) {
-            if (pop[i] >= count) {  // cannot happen while the closed form is right
-                report(FLASHLLM_ENCODE_RANGE);
-                pop[i] = -1;
-            }
-            if (pop[i] >= 0)
-                list[pop[i]] = item[i];
-        }
+        for (int i = 0; i < kLevels / kLevelsAtOnce; i++)
+            if (i * kLevelsAtOnce < top)
+                store_where(to + pop[i] * 4, item[i], here[i]);
+        lds_done();
         __syncthreads();
         for (int v = tid; v < space / 4; v += kEncodeThreads)
             store_vector(v, 0);
@@ -398,7 +502,7 @@ __global__ __launch_bounds__(kEncodeThreads, 6) void encode_tiles_kernel(const u
     }
 
     if (tid < kBanks)
-        fill_s[bank] = fill;
+        fill_s[bank] = static_cast<uint16_t>(fill);
     __syncthreads();
     for (int h = tid; h <= top; h += kEncodeThreads) {
         int      g = 0;
@@ -427,17 +531,20 @@ __global__ __launch_bounds__(kEncodeThreads, 6) void encode_tiles_kernel(const u
         };
         __syncthreads();  // the table is complete / the first part is out of the list
         int      h         = below;
-        uint32_t positions = first_position, mine = kept;
-        asm volatile("" : "+v"(positions), "+v"(mine));  // made here, not kept in registers for both parts
+        uint32_t positions = first_positions;
+        asm volatile("" : "+v"(positions));  // made here, not kept in registers for both parts; nor are the compares
+#pragma unroll
+        for (int i = 0; i < kRowsOfThread; i++)
+            asm volatile("" : "+v"(word[i]));
 #pragma unroll
         for (int i = 0; i < kRowsOfThread; i++) {
-            const uint32_t position = positions + (static_cast<uint32_t>(i * kTileCols) << 16);
-            if (mine & (1u << i))
-                place(++h, (word[i] & 0xffffu) | position);
-            if (mine & (1u << (i + 16)))
-                place(++h, (word[i] >> 16) | (position + 0x10000u));
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+                if (keeps_half(word[i], e))
+                    place(++h, item_of(i, e, positions));
+            positions += kTileCols * 0x10001u;
         }
-        if (segment == 0)
+        if (pads)
             for (int p = unpadded; p < fill; p++)
                 place(p + 1, pad_item);
         __syncthreads();
@@ -703,7 +810,7 @@ extern "C" int flashllm_hip_launch_encode(void* stream, const void* a, int m, in
 {
     const int tiles_per_row = k / kTileCols;
     const int tiles         = (m / kTileRows) * tiles_per_row;
-    hipLaunchKernelGGL(encode_tiles_kernel,
+    hipLaunchKernelGGL(k < kFarColumns ? encode_tiles_kernel<false> : encode_tiles_kernel<true>,
                        dim3(tiles),
                        dim3(kEncodeThreads),
                        0,

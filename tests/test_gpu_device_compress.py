@@ -325,6 +325,41 @@ def test_a_matrix_arrives_whole_without_its_zeros_on_the_way(product, torch_gpu,
         product.lib().flashllm_set_compress_threads(0)
 
 
+@pytest.mark.parametrize("full_rows", [0, 15, 16, 17, 32, 48, 60, 64, 112, 127])
+def test_padding_goes_to_the_first_zero_of_any_segment(product, oracle, torch_gpu, full_rows):
+    """The first rows of the tile dense, so that a bank's first zero is in a later segment of 16 rows (64 rows fill 128 levels, the
+    list's last); -0 and NaN behind them, which are zeros to the compressor; nnz % 4 of every kind."""
+    a = np.zeros((4 * 128, 64), dtype=np.float16)
+    for r in range(4):
+        tile = a[128 * r:128 * r + 128]
+        tile[:full_rows] = 0.5
+        tile[full_rows:, ::3] = np.float16(-0.0)
+        tile[full_rows:, 1::3] = np.float16("nan")
+        tile[127, 2:2 + 3 * r:3] = np.float16(2.0 ** -24)
+    check_against_oracle(product, oracle, torch_gpu, a, f"{full_rows} dense rows")
+
+
+@pytest.mark.parametrize("k", [(1 << 26) - 64, 1 << 26])
+def test_rows_of_the_most_columns_with_offsets_of_32_bits(product, torch_gpu, k):
+    """17 GB with three tiles that are not empty, in the first, the middle and the last columns, whose items follow one another: a row of
+    the other half of a wave lies 32 * k bytes on, up to 2^31 - 2048 by a 32-bit offset and from 2^31 on by a 64-bit address."""
+    say("far columns:", k)
+    torch = torch_gpu
+    three = torch.from_numpy(synth.sparse_matrix(128, 192, 0.8, 61)).cuda()
+    want, tiles = product.device_compress(three)
+    at = [0, k // 128 * 64, k - 64]
+    a = torch.zeros(128, k, dtype=torch.float16, device="cuda")
+    for i, c in enumerate(at):
+        a[:, c:c + 64] = three[:, 64 * i:64 * i + 64]
+    comp, offs = product.device_compress(a)
+    assert torch.equal(comp, want)
+    assert product.device_compress_status() == 0
+    for i, c in enumerate(at):
+        assert offs[c // 64:c // 64 + 2].tolist() == tiles[i:i + 2].tolist()
+    del a, comp, offs
+    torch.cuda.empty_cache()
+
+
 def test_loading_refuses_what_the_host_compressor_refuses(product, torch_gpu):
     for bad in (np.zeros((100, 64), np.float16), np.zeros((128, 96), np.float16), np.zeros((0, 64), np.float16)):
         with pytest.raises(product.CompressError):
