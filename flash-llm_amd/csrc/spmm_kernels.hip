@@ -240,6 +240,20 @@ __device__ __forceinline__ void take_8_and_wait(uintx4 (&a)[8], const uint32_t (
         : "memory");
 }
 
+// An operand by two exchanges that the compiler knows of: the products of the first row blocks run while the operands of the later ones are
+// on their way.  For eight row tiles per workgroup (N = 64), whose waves are in step and would all exchange and then all multiply: 36864
+// x 9216, 80 %, Split_K 7 72.6 -> 67.9 us, 49152 x 12288, 5 121.3 -> 109.3.  Waves that run freely fill each other's gaps, and lose by 16
+// more instructions per tile: 11392 x 18112, N = 64, Split_K 11 46.5 and 48.0, 36864 x 9216, N = 16 52.3 and 53.8, 49152 x 12288, N = 32 93.7
+// and 95.8.  By loads and, behind them, stores of zeros the first took 75.4, 9216 x 36864, N = 64, 90 % 70 instead of 66: 1 KB takes the LDS of a
+// CU 5.7 ns to store, 5.4 to exchange and 1.8 to load.
+__device__ __forceinline__ uintx4 take(uint32_t addr)
+{
+    using Half = __attribute__((address_space(3), may_alias)) uint64_t;
+    const uint64_t lo = __hip_atomic_exchange(reinterpret_cast<Half*>(addr), uint64_t{0}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    const uint64_t hi = __hip_atomic_exchange(reinterpret_cast<Half*>(addr + 8), uint64_t{0}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    return uintx4{static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32), static_cast<uint32_t>(hi), static_cast<uint32_t>(hi >> 32)};
+}
+
 // Sixteen operands (both 32-wide k steps): all sixteen exchanges are issued back to back, then one wait.
 // Two statements, because one statement takes at most thirty operands: the first issues eight exchanges,
 // the second, directly behind it, the other eight and the wait, and carries the first eight as in/out
@@ -544,12 +558,19 @@ __global__ __launch_bounds__(kLanes* W* KS) void spmm_stream_kernel(const uint4*
                             // NB <= 2: all 16 operands in one batch.  NB == 4: one 32-wide k step at a time, which
                             // keeps the kernel within 256 VGPRs (two waves per SIMD).
                             if constexpr (NB >= 4) {
+                                if constexpr (W > 1)
+                                    asm volatile("" ::: "memory");  // the items are in the tile
 #pragma unroll
                                 for (int ks = 0; ks < 2; ks++) {
                                     uintx4 a[8];
-                                    if constexpr (W > 1)
+                                    if constexpr (W > 1) {
                                         read_b(t, ks);
-                                    take_8_and_wait(a, ks ? a_addr1 : a_addr0);
+#pragma unroll
+                                        for (int rb = 0; rb < 8; rb++)
+                                            a[rb] = take((ks ? a_addr1 : a_addr0)[rb]);
+                                    }
+                                    else
+                                        take_8_and_wait(a, ks ? a_addr1 : a_addr0);
 #pragma unroll
                                     for (int rb = 0; rb < 8; rb++)
 #pragma unroll
@@ -557,6 +578,8 @@ __global__ __launch_bounds__(kLanes* W* KS) void spmm_stream_kernel(const uint4*
                                             acc[nb][rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                                                 __builtin_bit_cast(half8, a[rb]), bfrag[ks][nb], acc[nb][rb], 0, 0, 0);
                                 }
+                                if constexpr (W > 1)
+                                    asm volatile("" ::: "memory");  // the next tile's come after
                             }
                             else {
                                 uintx4 a0[8], a1[8];
