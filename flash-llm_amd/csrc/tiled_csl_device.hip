@@ -751,8 +751,7 @@ extern "C" int flashllm_hip_upload_packed(void* stream, void* dst, const void* s
     };
     std::vector<std::thread> pool;
     try {  // a thread that cannot be created is left out
-        // a thread for eight pieces (2048 x 2048 0.21 ms with 6 threads, 0.36 with 16), and at most eight: 7168 x 7168 1.14 ms, 1.09 with
-        // 16, after which the caller's next allocation of that size is touched 2.5 ms slower (with eight 0.6)
+        // a thread for eight pieces (2048 x 2048 0.21 ms with 6 threads, 0.36 with 16), and at most eight: 7168 x 7168 1.14 ms, 1.09 with 16
         const int workers = flashllm_compress_workers(pieces / 8 < 8 ? pieces / 8 : 8);
         pool.reserve(workers);
         for (int w = 1; w < workers; w++)
