@@ -1208,11 +1208,11 @@ __global__ __launch_bounds__(kWideWaves* kLanes, 2) void spmm_wide_kernel(const 
 //     runs are whole pairs of tiles and an odd one ends with an empty tile, whose B is zeros.
 //   * Lanes past a tile's end load its last vector again and store the same items once more: no masks.
 //   * A lone wave issues an instruction in four to five clocks, so that seven fit beside an MFMA and every one more delays the next.
-//     An item's address is one instruction (v_mad_u32_u16 takes the upper half of the item; a position beyond the tile, which no
-//     compressor writes, would land in the workgroup's other LDS), M0 is set for every fourth request for B, requests are two slots
-//     apart, and scalar work is not left to the phases' ends, where nothing covers it: 690 -> 605 instructions per tile of 80 %.  Calls
-//     in turn, before and after: 7168 x 28672, N = 512 214 -> 206 us, 21504 x 7168, N = 384 126 -> 121, 36864 x 9216, N = 128, Split_K 3
-//     at 80 and 90 % 108 -> 106 and 99 -> 94, 28672 x 7168, N = 64 45.2 -> 44.0.
+//     An item's address is a mask, which keeps a position that no compressor writes inside the wave's tile, and one instruction on it
+//     (v_mad_u32_u16 takes the upper half), M0 is set for every fourth request for B, requests are two slots apart, and scalar work is
+//     not left to the phases' ends, where nothing covers it.  Calls in turn, before and after: 7168 x 28672, N = 512 214 -> 206 us, 21504
+//     x 7168, N = 384 126 -> 121, 36864 x 9216, N = 128, Split_K 3 at 80 and 90 % 108 -> 106 and 99 -> 94, 28672 x 7168, N = 64 45.2 ->
+//     44.0.  The mask is 1 % of that (21504 x 7168, N = 384 118.4 us without, 120.0 with it).
 //   * The stream is loaded as other data is: the column groups of a row tile sit on one XCD and share its L2 (7168 x 28672, N =
 //     512, Split_K 1 210.7 us with non-temporal loads, 202.3).
 // With 64 columns (N = 64) a tile is two such phases and one window of B, so that B is asked for two tiles ahead; a tile without
@@ -1303,9 +1303,12 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
             const uint32_t at = lane * 16u + r * (kLanes * 16u);
             slot = *reinterpret_cast<const __attribute__((address_space(1))) uintx4*>(from + (at < from_last ? at : from_last));
         };
+        uint32_t in_tile = (kTileHalfs << 16) - 1u;
+        asm volatile("" : "+s"(in_tile));  // a register, not a literal of every instruction
         auto scatter = [&](uint32_t item) {
-            uint32_t at;  // 2 * position + tile_l
-            asm("v_mad_u32_u16 %0, %1, 2, %2 op_sel:[1,0,0,0]" : "=v"(at) : "v"(item), "s"(tile_l));
+            const uint32_t inside = item & in_tile;  // whatever the item says, it stays in the wave's own tile
+            uint32_t       at;                       // 2 * position + tile_l
+            asm("v_mad_u32_u16 %0, %1, 2, %2 op_sel:[1,0,0,0]" : "=v"(at) : "v"(inside), "s"(tile_l));
             *reinterpret_cast<Lds16*>(at) = static_cast<uint16_t>(item);
         };
         // a tile of more than R chunks: chunks R .. R + X - 1 of it; lanes past its end as above

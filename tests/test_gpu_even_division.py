@@ -116,3 +116,20 @@ def test_calls_that_gain_little_keep_their_slices(product, m, k, n, split_k):
     product.spmm_partials(comp, offs, b, want, m, n, k, ws, split_k)
     product.splitk_reduce(want, ws, m, n, split_k)
     assert torch.equal(c.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("sparsity", [0.99, 0.88, 0.75, 0.6])  # the four depths of the ring
+def test_positions_beyond_the_tile_stay_inside_it(product, sparsity):
+    import copy
+
+    import torch
+
+    print(f"even shares, positions beyond the tile, sparsity={sparsity}", flush=True)
+    m, k, n = 512, 64 * 16, 128
+    a = synth.sparse_matrix(m, k, sparsity, 115, dist="normal", sigma=0.05)
+    a[128:256, 320:384] = 0.5  # and a tile longer than the ring
+    w = product.SparseWeight(a)
+    b = torch.from_numpy(synth.dense_b(k, n, 116, dist="normal")).cuda()
+    damaged = copy.copy(w)
+    damaged.comp = w.comp ^ (torch.randint(0, 8, w.comp.shape, dtype=torch.int32, device="cuda") << 29)
+    assert torch.equal(launch(product, torch, damaged, b, n, 9), launch(product, torch, w, b, n, 9))

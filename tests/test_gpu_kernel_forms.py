@@ -112,3 +112,23 @@ def test_matrix_without_nonzeros(product, form, split_k):
     b = torch.from_numpy(synth.dense_b(k, n, 103, dist="normal")).cuda()
     got = launch(product, torch, form, w, b, k, nan_halfs(torch, split_k * n * m), split_k, 0)
     assert bool((got == 0).all())
+
+
+@pytest.mark.parametrize("form", FORMS, ids=lambda f: "-".join(map(str, f)))
+def test_positions_beyond_the_tile_stay_inside_it(product, weights, form):
+    """An item's position has 13 bits; the three above them, which a damaged Compressed_A may have set, change nothing: no item leaves
+    the tile of the wave that stores it."""
+    import copy
+
+    import torch
+
+    print("positions beyond the tile", form, flush=True)
+    _, n, _ = form
+    w = weights(form[0], 3)
+    b = torch.from_numpy(synth.dense_b(w.k, n, 104, dist="normal")).cuda()
+    damaged = copy.copy(w)
+    damaged.comp = w.comp ^ (torch.randint(0, 8, w.comp.shape, dtype=torch.int32, device="cuda") << 29)
+    assert not torch.equal(damaged.comp, w.comp)
+    want = launch(product, torch, form, w, b, w.k, nan_halfs(torch, 3 * n * w.m), 3, 0)
+    got = launch(product, torch, form, damaged, b, w.k, nan_halfs(torch, 3 * n * w.m), 3, 0)
+    assert bool(torch.isfinite(want).all()) and same_bits(torch, got, want)
