@@ -577,6 +577,12 @@ __global__ __launch_bounds__(kLanes* W* KS) void spmm_stream_kernel(const uint4*
                                         for (int nb = 0; nb < NB; nb++)
                                             acc[nb][rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                                                 __builtin_bit_cast(half8, a[rb]), bfrag[ks][nb], acc[nb][rb], 0, 0, 0);
+                                    // This wave's reads of the window have ended here, before the barrier that gives its LDS to other
+                                    // loads: products that use them could sink below that barrier, and their wait with them.
+                                    if constexpr (W > 1)
+#pragma unroll
+                                        for (int nb = 0; nb < NB; nb++)
+                                            asm volatile("" ::"v"(bfrag[ks][nb]));
                                 }
                                 if constexpr (W > 1)
                                     asm volatile("" ::: "memory");  // the next tile's come after
