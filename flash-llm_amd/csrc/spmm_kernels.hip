@@ -1362,18 +1362,20 @@ __device__ __forceinline__ void spmm_quarter_body(unsigned char* lds,
             return Half{there ? (Global*)(NJ == 4 ? bcols + (half & 1) * (64 * static_cast<size_t>(ldb)) + (half >> 1) * kTileCols : bcols + half * kTileCols) : nothing,
                         there ? 64 * static_cast<size_t>(ldb) : 0, there ? ~0u : 0u};
         };
-        // eight requests in a row: M0 is set for every fourth, between them the instruction's offset counts in LDS and in memory
+        // eight requests in a row: M0 is set for every fourth, between them the instruction's offset counts in LDS and in memory.  It is an
+        // operand of all four, so that the compiler knows it to be in use (carried so it costs no copy: the same instructions)
+        uint32_t m0;
         auto fetch_b = [&](const Half& half, uint32_t window, int i) {
             const uint32_t at    = b_lane[i % 4] & half.lanes;
             Global* const  first = half.first + (i / 4) * half.step;
             if (i % 4 == 0)
-                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(at), "s"(first), "s"(window + i * 1024) : "memory", "m0");
+                asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : "={m0}"(m0) : "v"(at), "s"(first), "s"(window + i * 1024) : "memory");
             else if (i % 4 == 1)
-                asm volatile("global_load_lds_dwordx4 %0, %1 offset:1024" ::"v"(at), "s"(first) : "memory");
+                asm volatile("global_load_lds_dwordx4 %0, %1 offset:1024" ::"v"(at), "s"(first), "{m0}"(m0) : "memory");
             else if (i % 4 == 2)
-                asm volatile("global_load_lds_dwordx4 %0, %1 offset:2048" ::"v"(at), "s"(first) : "memory");
+                asm volatile("global_load_lds_dwordx4 %0, %1 offset:2048" ::"v"(at), "s"(first), "{m0}"(m0) : "memory");
             else
-                asm volatile("global_load_lds_dwordx4 %0, %1 offset:3072" ::"v"(at), "s"(first) : "memory");
+                asm volatile("global_load_lds_dwordx4 %0, %1 offset:3072" ::"v"(at), "s"(first), "{m0}"(m0) : "memory");
         };
         auto multiply = [&](int p, int m) {
             const int s = 2 * (p & 1) + m / 8, i = m / 2 % 4, j = 2 * (p / 2) + m % 2;
