@@ -135,6 +135,9 @@ enum {
 // One piece of n halfs (at most kPackPiece, a multiple of kPackGroup) at src, at dst.  Host only.
 void flashllm_pack_piece(const unsigned short* src, size_t n, unsigned char* dst);
 
+// Whether n halfs at src reach the GPU sooner by way of packed pieces than as they are.
+int flashllm_packing_pays(const unsigned short* src, size_t n);
+
 // Threads that the host compressor would take for so many pieces of work.
 int flashllm_compress_workers(size_t pieces);
 
