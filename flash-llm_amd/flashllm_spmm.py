@@ -269,7 +269,7 @@ def _upload(a_host):
         fn = lib().flashllm_hip_upload_stage
         fn.restype = ctypes.c_size_t
         try:
-            stage = torch.empty(fn(), dtype=torch.uint8, pin_memory=True)
+            stage = torch.empty(fn(), dtype=torch.uint8, device="cpu", pin_memory=True)  # whatever the default device is
         except RuntimeError:  # no pinned memory to be had
             pass
     if stage is not None:

@@ -325,6 +325,24 @@ def test_a_matrix_arrives_whole_without_its_zeros_on_the_way(product, torch_gpu,
         product.lib().flashllm_set_compress_threads(0)
 
 
+def test_the_default_device_has_no_say_in_how_a_matrix_arrives(product, torch_gpu, monkeypatch):
+    """torch refuses to pin memory on the GPU, where torch.empty allocates by default here: the way without zeros is taken all the same."""
+    say("packed upload with the GPU as default device")
+    L, calls = product.lib(), []
+
+    class Watched:
+        def __getattr__(self, name):
+            calls.append(name)
+            return getattr(L, name)
+
+    a = synth.sparse_matrix(2048, 2048, 0.8, 53)
+    monkeypatch.setattr(product, "lib", Watched)
+    with torch_gpu.device("cuda"):
+        got = product._upload(a)
+    assert "flashllm_hip_upload_packed" in calls and "flashllm_hip_upload" not in calls
+    assert np.array_equal(got.cpu().numpy().view(np.uint16), a.view(np.uint16))
+
+
 @pytest.mark.parametrize("full_rows", [0, 15, 16, 17, 32, 48, 60, 64, 112, 127])
 def test_padding_goes_to_the_first_zero_of_any_segment(product, oracle, torch_gpu, full_rows):
     """The first rows of the tile dense, so that a bank's first zero is in a later segment of 16 rows (64 rows fill 128 levels, the

@@ -13,7 +13,7 @@ class Recorded:
     """The library with both uploads replaced by a note of the call."""
 
     def __init__(self, lib):
-        self.lib, self.ways = lib, []
+        self.lib, self.ways, self.nothing_to_pin = lib, [], False
 
     def __getattr__(self, name):
         if name not in ("flashllm_hip_upload", "flashllm_hip_upload_packed"):
@@ -33,14 +33,18 @@ def way_of(product, monkeypatch):
     recorded = Recorded(product.lib())
 
     def empty(*args, pin_memory=False, device=None, **kw):
+        assert not pin_memory or device == "cpu"  # torch pins no memory of another device, and the default one may be the GPU
+        if pin_memory and recorded.nothing_to_pin:
+            raise RuntimeError("out of pinned memory")
         return real(*args, device="cpu", **kw)
 
     monkeypatch.setattr(torch, "empty", empty)
     monkeypatch.setattr(product, "lib", lambda: recorded)
     monkeypatch.setattr(product, "_stream", lambda stream: ctypes.c_void_p(0))
 
-    def way(a, threads):
+    def way(a, threads, nothing_to_pin=False):
         recorded.ways.clear()
+        recorded.nothing_to_pin = nothing_to_pin
         recorded.flashllm_set_compress_threads(threads)
         try:
             assert product._upload(a).shape == a.shape
@@ -67,3 +71,9 @@ def test_a_small_matrix_with_few_zeros_goes_as_it_is(way_of):
     assert way_of(synth.sparse_matrix(1024, 4032, 0.0, 3), 16) == "as it is"
     assert way_of(synth.sparse_matrix(1024, 4096, 0.0, 3), 16) == "_packed"
     assert way_of(synth.sparse_matrix(896, 1024, 0.8, 3), 16) == "as it is"
+
+
+def test_without_pinned_memory_it_goes_as_it_is(way_of):
+    a = synth.sparse_matrix(2048, 2048, 0.8, 3)
+    assert way_of(a, 16) == "_packed"
+    assert way_of(a, 16, nothing_to_pin=True) == "as it is"
