@@ -142,10 +142,10 @@ int flashllm_packing_pays(const unsigned short* src, size_t n);
 int flashllm_compress_workers(size_t pieces);
 
 // The same matrix at dst (device memory, 16-byte aligned) as flashllm_hip_upload leaves there, by way of packed pieces in stage (pinned
-// host memory, 16-byte aligned, at least flashllm_hip_upload_stage() bytes) that a kernel fetches and expands.  n halfs, a multiple of
-// kPackGroup.  Waits for it.
+// host memory, 16-byte aligned, at least flashllm_hip_upload_stage(n) bytes: at most 30 MB) that a kernel fetches and expands.  n halfs, a
+// multiple of kPackGroup.  Waits for it.
 int    flashllm_hip_upload_packed(void* stream, void* dst, const void* src, size_t n, void* stage);
-size_t flashllm_hip_upload_stage(void);
+size_t flashllm_hip_upload_stage(size_t n);
 
 // Copies ordinary host memory to the GPU and waits for it.
 int flashllm_hip_upload(void* stream, void* dst, const void* src, size_t bytes);

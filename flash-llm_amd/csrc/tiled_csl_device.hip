@@ -712,9 +712,10 @@ extern "C" int flashllm_hip_upload(void* stream, void* dst, const void* src, siz
     return static_cast<int>(e == hipSuccess ? hipStreamSynchronize(s) : e);
 }
 
-extern "C" size_t flashllm_hip_upload_stage(void)
+extern "C" size_t flashllm_hip_upload_stage(size_t n)
 {
-    return static_cast<size_t>(kParts) * kPartPieces * kPackStride;
+    const size_t pieces = (n + kPackPiece - 1) / kPackPiece, most = static_cast<size_t>(kParts) * kPartPieces;
+    return (pieces < most ? pieces : most) * kPackStride;
 }
 
 // The host's threads leave the zeros out (they read the matrix faster than the link carries it), and what is left crosses the link once,
@@ -727,9 +728,13 @@ extern "C" int flashllm_hip_upload_packed(void* stream, void* dst, const void* s
     auto*        ring   = static_cast<unsigned char*>(stage);
     if (n == 0 || n % kPackGroup)
         return static_cast<int>(hipErrorInvalidValue);
+    // where the GPU finds it: memory that was pinned after it was allocated may have another address there, and other memory has none
+    void*      ring_there = nullptr;
+    hipError_t e          = hipHostGetDevicePointer(&ring_there, stage, 0);
+    if (e != hipSuccess)
+        return static_cast<int>(e);
     hipEvent_t free_again[kParts];
     int        events = 0;
-    hipError_t e      = hipSuccess;
     while (events < kParts && (e = hipEventCreateWithFlags(&free_again[events], hipEventDisableTiming)) == hipSuccess)
         events++;
 
@@ -772,7 +777,8 @@ extern "C" int flashllm_hip_upload_packed(void* stream, void* dst, const void* s
         packed[place].store(0, std::memory_order_relaxed);
         const size_t start = first * kPackPiece, halfs = n - start < count * kPackPiece ? n - start : count * kPackPiece;
         hipLaunchKernelGGL(expand_kernel, dim3(static_cast<unsigned>(halfs / kPackGroup)), dim3(kExpandThreads), 0, s,
-                           ring + static_cast<size_t>(place) * kPartPieces * kPackStride, static_cast<uintx4*>(dst) + start / 8);
+                           static_cast<const unsigned char*>(ring_there) + static_cast<size_t>(place) * kPartPieces * kPackStride,
+                           static_cast<uintx4*>(dst) + start / 8);
         e = hipGetLastError();
         if (e == hipSuccess)
             e = hipEventRecord(free_again[place], s);

@@ -10,6 +10,7 @@ gen_sparse_matrix_bin_file <-> GenSparseMatrixBinFile.
 """
 import ctypes
 import os
+import threading
 
 import numpy as np
 
@@ -56,6 +57,14 @@ SIGNATURES = {
     "GenSparseMatrixBinFile": (None, [ctypes.c_char_p, ctypes.c_int, ctypes.c_int, ctypes.c_char_p, ctypes.c_char_p, ctypes.c_char_p]),
 }
 
+# what a weight's way to the GPU uses beside them (csrc/spmm_launch.h)
+UPLOAD_SIGNATURES = {
+    "flashllm_packing_pays": (ctypes.c_int, [_vp, ctypes.c_size_t]),
+    "flashllm_hip_upload_stage": (ctypes.c_size_t, [ctypes.c_size_t]),
+    "flashllm_hip_upload_packed": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_size_t, _vp]),
+    "flashllm_hip_upload": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_size_t]),
+}
+
 
 def lib():
     """Loads libSpMM_API.so once.  Raises OSError when it has not been built."""
@@ -71,7 +80,7 @@ def lib():
         except ImportError:
             pass
         handle = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in (SIGNATURES | UPLOAD_SIGNATURES).items():
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
@@ -258,30 +267,29 @@ HIP_ERROR_OUT_OF_MEMORY = 2
 UPLOAD_PACKED_BYTES = 2 << 20  # below, the runtime's copy is as quick: 1024 x 1024 at 80 % 0.09 ms either way
 
 
+_packed_uploads = threading.BoundedSemaphore(4)  # at a time, and with them their pinned memory: one alone takes 1.06 ms, two 0.81 each, four 0.69
+
+
 def _upload(a_host):
     """A dense host matrix (float16, or uint16 bit patterns) as a float16 tensor on the current GPU, complete on return."""
     import torch
 
     a = _bits(a_host)
     dev = torch.empty(a.shape, dtype=torch.float16, device="cuda")
-    stage = None
-    if a.nbytes >= UPLOAD_PACKED_BYTES and lib().flashllm_packing_pays(_vp(a.ctypes.data), ctypes.c_size_t(a.size)):
-        fn = lib().flashllm_hip_upload_stage
-        fn.restype = ctypes.c_size_t
-        try:
-            stage = torch.empty(fn(), dtype=torch.uint8, device="cpu", pin_memory=True)  # whatever the default device is
-        except RuntimeError:  # no pinned memory to be had
-            pass
-    if stage is not None:
-        fn = lib().flashllm_hip_upload_packed  # both take read-only arrays as they are
-        fn.restype = ctypes.c_int
-        fn.argtypes = [_vp, _vp, _vp, ctypes.c_size_t, _vp]
-        rc = fn(_stream(None), _ptr(dev), a.ctypes.data, a.size, _ptr(stage))
-    else:
-        fn = lib().flashllm_hip_upload
-        fn.restype = ctypes.c_int
-        fn.argtypes = [_vp, _vp, _vp, ctypes.c_size_t]
-        rc = fn(_stream(None), _ptr(dev), a.ctypes.data, a.nbytes)
+    L = lib()  # its uploads take read-only arrays as they are
+    if a.nbytes >= UPLOAD_PACKED_BYTES and L.flashllm_packing_pays(a.ctypes.data, a.size):
+        with _packed_uploads:
+            try:
+                stage = torch.empty(L.flashllm_hip_upload_stage(a.size), dtype=torch.uint8, device="cpu", pin_memory=True)  # whatever the default device is
+            except RuntimeError:  # no pinned memory to be had
+                stage = None
+            if stage is not None:
+                rc = L.flashllm_hip_upload_packed(_stream(None), _ptr(dev), a.ctypes.data, a.size, _ptr(stage))
+                del stage  # the block is torch's again before the next one asks for its own
+                if rc:
+                    raise HipError(rc)
+                return dev
+    rc = L.flashllm_hip_upload(_stream(None), _ptr(dev), a.ctypes.data, a.nbytes)
     if rc:
         raise HipError(rc)
     return dev
@@ -311,13 +319,15 @@ class SparseWeight:
         self.offs = torch.from_numpy(offsets).to(device)
 
     def _compress_on_gpu(self, a_host, reorder):
-        """Sends the matrix and compresses it there, to the same bytes.  Its zeros are left out on the way (up to eight
-        threads pack it into 32 MB of pinned memory, from where a kernel fetches and expands it): 7168 x 7168 at 80 % 1.3 ms, of which
-        1.1 are the way there; sent as it is 3.7, at 28 GB/s; compressed on the host (16 threads) and the result sent 17.8.
+        """Sends the matrix and compresses it there, to the same bytes.  Its zeros are left out on the way where that is quicker
+        (flashllm_packing_pays; up to eight threads pack it into pinned memory, from where a kernel fetches and expands it): 7168 x 7168 at
+        80 % 1.1 ms, of which 0.9 are the way there; sent as it is 3.7, at 28 GB/s; compressed on the host (16 threads) and the result sent 17.8.
         The dense matrix needs 2 * M * K bytes of the GPU beside its compressed form.  They come from torch's allocator, which keeps
         the block for later tensors, the next weight's among them; where memory is to be had with hipMalloc after loading,
-        torch.cuda.empty_cache() gives it back.  (Memory of its own, returned by hipFree in each call, makes a load 12 % longer.)  The pinned
-        memory comes from torch's allocator for it, which keeps it for later loads likewise.
+        torch.cuda.empty_cache() gives it back.  (Memory of its own, returned by hipFree in each call, makes a load 12 % longer.)
+        The pinned memory, 2.1 bytes per element and at most 30 MB a call, comes from torch's allocator for it, which rounds up to a power of
+        two and keeps the blocks for later calls, at most four of a size because no more calls pack at a time; a size that is not yet there costs a call 0.03 ... 0.08 ms
+        more.  torch.cuda.empty_cache() does not touch it: torch._C._host_emptyCache() gives it back.
         False: a matrix that only the host compressor has an answer to, or no room for it beside its compressed form."""
         import torch
 

@@ -343,6 +343,37 @@ def test_the_default_device_has_no_say_in_how_a_matrix_arrives(product, torch_gp
     assert np.array_equal(got.cpu().numpy().view(np.uint16), a.view(np.uint16))
 
 
+def test_pinned_memory_of_loading_is_bounded_and_given_back(product, torch_gpu):
+    """Twelve threads load at once, four of them pack at a time; the blocks stay in torch's cache until it is emptied."""
+    import concurrent.futures
+
+    torch = torch_gpu
+    say("pinned memory of concurrent loads")
+    mats = [synth.sparse_matrix(4096, 7168, 0.8, 80 + i) for i in range(12)]  # 14 parts each: the whole ring, 32 MB
+
+    def pinned():
+        return torch.cuda.host_memory_stats()["allocated_bytes.current"]
+
+    torch._C._host_emptyCache()
+    before = pinned()
+
+    def load(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            got = [product.SparseWeight(mats[i]) for _ in range(2)]
+            return [(w.comp.cpu().numpy().view(np.uint32), w.offs.cpu().numpy()) for w in got]
+
+    with concurrent.futures.ThreadPoolExecutor(12) as pool:
+        got = list(pool.map(load, range(12)))
+    for a, weights in zip(mats, got):
+        items, offsets = product.init_sparse_matrix_a(a)
+        for comp, offs in weights:
+            assert np.array_equal(comp, items) and np.array_equal(offs, offsets)
+    say("pinned by loading:", pinned() - before)
+    assert 0 < pinned() - before <= 4 << 25
+    torch._C._host_emptyCache()
+    assert pinned() == before
+
+
 @pytest.mark.parametrize("full_rows", [0, 15, 16, 17, 32, 48, 60, 64, 112, 127])
 def test_padding_goes_to_the_first_zero_of_any_segment(product, oracle, torch_gpu, full_rows):
     """The first rows of the tile dense, so that a bank's first zero is in a later segment of 16 rows (64 rows fill 128 levels, the

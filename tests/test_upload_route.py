@@ -77,3 +77,10 @@ def test_without_pinned_memory_it_goes_as_it_is(way_of):
     a = synth.sparse_matrix(2048, 2048, 0.8, 3)
     assert way_of(a, 16) == "_packed"
     assert way_of(a, 16, nothing_to_pin=True) == "as it is"
+
+
+def test_pinned_memory_for_the_matrix_and_no_more_than_the_ring(product):
+    fn = product.lib().flashllm_hip_upload_stage
+    stride = 128 + 65536 // 8 + 2 * 65536 + 128
+    for n, pieces in ((2048, 1), (65536, 1), (65536 + 2048, 2), (1024 * 1024, 16), (223 * 65536, 223), (224 * 65536, 224), (225 * 65536, 224), (1 << 33, 224)):
+        assert fn(n) == pieces * stride
