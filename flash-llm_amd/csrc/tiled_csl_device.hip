@@ -31,6 +31,8 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <condition_variable>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -754,17 +756,32 @@ extern "C" int flashllm_hip_upload_packed(void* stream, void* dst, const void* s
         packed[slot / kPartPieces].fetch_add(1, std::memory_order_release);
         return true;
     };
+    // A thread that finds no place in the ring looks again for as long as the GPU usually takes over a part (40 us), then sleeps: the stream
+    // may have other work before this (7168 x 7168 behind 320 ms of it took 2560 ms of the host's cores instead of 320, the wait's own).
+    std::mutex              door;
+    std::condition_variable place_free;
+    auto                    pack_all = [&]() {
+        int in_vain = 0;
+        while (!stop.load(std::memory_order_relaxed) && next.load(std::memory_order_relaxed) < pieces)
+            if (pack_one())
+                in_vain = 0;
+            else if (++in_vain < 500)
+                std::this_thread::yield();
+            else {
+                std::unique_lock<std::mutex> lock(door);
+                place_free.wait(lock, [&]() {
+                    return stop.load(std::memory_order_relaxed) || next.load(std::memory_order_relaxed) / kPartPieces < allowed.load(std::memory_order_relaxed);
+                });
+                in_vain = 0;
+            }
+    };
     std::vector<std::thread> pool;
     try {  // a thread that cannot be created is left out
         // a thread for eight pieces (2048 x 2048 0.21 ms with 6 threads, 0.36 with 16), and at most eight: 7168 x 7168 1.14 ms, 1.09 with 16
         const int workers = flashllm_compress_workers(pieces / 8 < 8 ? pieces / 8 : 8);
         pool.reserve(workers);
         for (int w = 1; w < workers; w++)
-            pool.emplace_back([&]() {
-                while (!stop.load(std::memory_order_relaxed) && next.load(std::memory_order_relaxed) < pieces)
-                    if (!pack_one())
-                        std::this_thread::yield();
-            });
+            pool.emplace_back(pack_all);
     }
     catch (...) {
     }
@@ -784,10 +801,18 @@ extern "C" int flashllm_hip_upload_packed(void* stream, void* dst, const void* s
             e = hipEventRecord(free_again[place], s);
         if (e == hipSuccess && p + 2 >= kParts) {  // part p + 2 follows part p + 2 - kParts
             e = hipEventSynchronize(free_again[(p + 2) % kParts]);
-            allowed.store(p + 3, std::memory_order_release);
+            {
+                const std::lock_guard<std::mutex> lock(door);
+                allowed.store(p + 3, std::memory_order_release);
+            }
+            place_free.notify_all();
         }
     }
-    stop.store(true, std::memory_order_relaxed);
+    {
+        const std::lock_guard<std::mutex> lock(door);
+        stop.store(true, std::memory_order_relaxed);
+    }
+    place_free.notify_all();
     for (auto& t : pool)
         t.join();
     const hipError_t done = hipStreamSynchronize(s);  // the ring is the caller's again

@@ -374,6 +374,33 @@ def test_pinned_memory_of_loading_is_bounded_and_given_back(product, torch_gpu):
     assert pinned() == before
 
 
+def test_a_load_behind_other_work_leaves_the_cores_alone(product, torch_gpu):
+    """The ring fills and the GPU is busy for a while: the packing threads sleep, only the caller's wait may take a core."""
+    import time
+
+    torch = torch_gpu
+    say("packed upload behind other work")
+    a = synth.sparse_matrix(4096, 7168, 0.8, 54)  # 14 parts, twice the ring
+    x = torch.randn(8192, 8192, dtype=torch.float16, device="cuda")
+    product.lib().flashllm_set_compress_threads(8)
+    try:
+        product._upload(a)
+        y = x @ x
+        torch.cuda.synchronize()
+        for _ in range(150):
+            y = x @ x
+        cpu, wall = time.process_time(), time.perf_counter()
+        got = product._upload(a)
+        cpu, wall = time.process_time() - cpu, time.perf_counter() - wall
+    finally:
+        product.lib().flashllm_set_compress_threads(0)
+    say(f"{wall * 1e3:.0f} ms, of the cores {cpu * 1e3:.0f}")
+    assert wall > 0.05  # the work was in front of it
+    assert cpu < 3 * wall
+    assert np.array_equal(got.cpu().numpy().view(np.uint16), a.view(np.uint16))
+    del y
+
+
 @pytest.mark.parametrize("full_rows", [0, 15, 16, 17, 32, 48, 60, 64, 112, 127])
 def test_padding_goes_to_the_first_zero_of_any_segment(product, oracle, torch_gpu, full_rows):
     """The first rows of the tile dense, so that a bank's first zero is in a later segment of 16 rows (64 rows fill 128 levels, the
