@@ -358,12 +358,12 @@ int flashllm_compress_workers(size_t pieces)
 
 // Not with a single thread, which packs no faster than the runtime copies: 7168 x 7168 at 50 and 80 % as it is 3.54 and 3.76 ms, with 1
 // thread 4.46 and 4.28, with 2 2.55 and 2.57, with 8 1.42 and 0.91; 2048 x 2048 at 80 % 0.31 and 0.38, 0.26, 0.16.  Below 8 MB only with
-// enough zeros, by a sample of 64 cache lines: 1024 x 1792 as it is 0.131, packed at 0, 50, 70 and 80 % 0.183, 0.128, 0.109 and 0.113,
+// enough zeros, by a sample of 16 cache lines: 1024 x 1792 as it is 0.131, packed at 0, 50, 70 and 80 % 0.183, 0.128, 0.109 and 0.113,
 // 1536 x 1536 0.155 and 0.220, 0.151, 0.133, 0.131; from there on a matrix without zeros takes as long either way (2048 x 2048 0.31 and 0.30,
 // 7168 x 7168 3.62 and 2.36).
 int flashllm_packing_pays(const unsigned short* src, size_t n)
 {
-    constexpr size_t kLines = 64, kLine = 32, kAnyDensity = (8u << 20) / sizeof(uint16_t);
+    constexpr size_t kLines = 16, kLine = 32, kAnyDensity = (8u << 20) / sizeof(uint16_t);
     if (worker_count(2) < 2)
         return 0;
     if (n >= kAnyDensity || n < kLines * kLine)
