@@ -134,6 +134,8 @@ enum {
 
 // One piece of n halfs (at most kPackPiece, a multiple of kPackGroup) at src, at dst.  Host only.
 void flashllm_pack_piece(const unsigned short* src, size_t n, unsigned char* dst);
+// The same in the way of processors without SSSE3, whatever this one has.
+void flashllm_pack_piece_plain(const unsigned short* src, size_t n, unsigned char* dst);
 
 // Whether n halfs at src reach the GPU sooner by way of packed pieces than as they are.
 int flashllm_packing_pays(const unsigned short* src, size_t n);

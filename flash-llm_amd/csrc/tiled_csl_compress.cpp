@@ -14,8 +14,10 @@
 #include "flashllm_spmm.h"
 #include "spmm_launch.h"
 
+#if defined(__x86_64__)
 #include <emmintrin.h>
 #include <tmmintrin.h>
+#endif
 
 #include <atomic>
 #include <climits>
@@ -192,6 +194,7 @@ void for_each_tile(size_t tiles, F&& body)
         th.join();
 }
 
+#if defined(__x86_64__)
 // For each mask of eight halfs the bytes that bring those to the front.
 struct FrontBytes {
     alignas(16) uint8_t of[256][16];
@@ -234,7 +237,9 @@ __attribute__((target("ssse3,popcnt"))) size_t pack_group(const uint16_t* src, u
     }
     return static_cast<size_t>(at - out);
 }
+#endif
 
+// The same on any processor.
 size_t pack_group_plain(const uint16_t* src, uint8_t* bits, uint16_t* out)
 {
     uint16_t* at = out;
@@ -248,6 +253,17 @@ size_t pack_group_plain(const uint16_t* src, uint8_t* bits, uint16_t* out)
         bits[i / 8] = static_cast<uint8_t>(mask);
     }
     return static_cast<size_t>(at - out);
+}
+
+void pack_piece(const uint16_t* src, size_t n, unsigned char* dst, size_t (*pack)(const uint16_t*, uint8_t*, uint16_t*))
+{
+    uint32_t* const first  = reinterpret_cast<uint32_t*>(dst);
+    uint16_t* const values = reinterpret_cast<uint16_t*>(dst + kPackValues);
+    size_t          packed = 0;
+    for (size_t g = 0; g < n / kPackGroup; g++) {
+        first[g] = static_cast<uint32_t>(packed);
+        packed += pack(src + g * kPackGroup, dst + kPackBits + g * (kPackGroup / 8), values + packed);
+    }
 }
 
 int compress(const uint16_t* A, int M, int K, uint32_t** comp_out, int** offs_out, bool reorder)
@@ -377,14 +393,16 @@ int flashllm_packing_pays(const unsigned short* src, size_t n)
 
 void flashllm_pack_piece(const unsigned short* src, size_t n, unsigned char* dst)
 {
-    uint32_t* const first  = reinterpret_cast<uint32_t*>(dst);
-    uint16_t* const values = reinterpret_cast<uint16_t*>(dst + kPackValues);
-    const bool      fast   = __builtin_cpu_supports("ssse3") && __builtin_cpu_supports("popcnt");
-    size_t          packed = 0;
-    for (size_t g = 0; g < n / kPackGroup; g++) {
-        first[g] = static_cast<uint32_t>(packed);
-        packed += (fast ? pack_group : pack_group_plain)(src + g * kPackGroup, dst + kPackBits + g * (kPackGroup / 8), values + packed);
-    }
+#if defined(__x86_64__)
+    if (__builtin_cpu_supports("ssse3") && __builtin_cpu_supports("popcnt"))
+        return pack_piece(src, n, dst, pack_group);
+#endif
+    pack_piece(src, n, dst, pack_group_plain);
+}
+
+void flashllm_pack_piece_plain(const unsigned short* src, size_t n, unsigned char* dst)
+{
+    pack_piece(src, n, dst, pack_group_plain);
 }
 
 void flashllm_set_compress_threads(int n)

@@ -3,12 +3,16 @@
 //   asan_compress dense.bin M K out_prefix
 // writes <prefix>.reorder.bin and <prefix>.noreorder.bin (int32 count of TileOffsets, the offsets, the items) for
 // one and for three worker threads (which must agree), and the exporter's three files as <prefix>.NZWeights.bin,
-// <prefix>.TileOffsets.bin, <prefix>.OutputSizes.bin.  Any sanitizer report ends the process with a non-zero code.
+// <prefix>.TileOffsets.bin, <prefix>.OutputSizes.bin.  Before the exporter the matrix is packed piece by piece, both ways, between buffers
+// of exactly the sizes that the packing may touch, and unpacked again.  Any sanitizer report ends the process with a non-zero code.
 #include "flashllm_spmm.h"
+#include "spmm_launch.h"
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -51,6 +55,30 @@ bool run(compressor fn, const std::vector<uint16_t>& a, int m, int k, const std:
         std::fwrite(first_items.data(), sizeof(uint32_t), first_items.size(), f);
     return std::fclose(f) == 0;
 }
+
+bool pack(const std::vector<uint16_t>& a)
+{
+    for (size_t at = 0; at < a.size(); at += kPackPiece) {
+        const size_t                     n = std::min<size_t>(kPackPiece, a.size() - at);
+        const std::unique_ptr<uint16_t[]> src(new uint16_t[n]);
+        std::copy_n(a.data() + at, n, src.get());
+        for (auto fn : {flashllm_pack_piece, flashllm_pack_piece_plain}) {
+            const std::unique_ptr<unsigned char[]> piece(new unsigned char[kPackStride]);
+            fn(src.get(), n, piece.get());
+            const uint32_t* first  = reinterpret_cast<const uint32_t*>(piece.get());
+            const uint16_t* values = reinterpret_cast<const uint16_t*>(piece.get() + kPackValues);
+            for (size_t i = 0, next = 0; i < n; i++) {
+                if (i % kPackGroup == 0 && first[i / kPackGroup] != next)
+                    return false;
+                const bool     kept  = piece[kPackBits + i / 8] >> (i % 8) & 1;
+                const uint16_t value = kept ? values[next++] : 0;
+                if (value != src[i] || kept != (value != 0))
+                    return false;
+            }
+        }
+    }
+    return true;
+}
 }  // namespace
 
 int main(int argc, char** argv)
@@ -80,6 +108,10 @@ int main(int argc, char** argv)
         return 5;
     if (!run(flashllm_init_sparse_matrix_a_noreorder, a, m, k, prefix + ".noreorder.bin"))
         return 6;
+    if (!pack(a)) {
+        std::fprintf(stderr, "a packed piece does not hold the matrix\n");
+        return 9;
+    }
     const int rc = flashllm_gen_sparse_matrix_bin_file(argv[1], m, k, (prefix + ".NZWeights.bin").c_str(),
                                                       (prefix + ".TileOffsets.bin").c_str(), (prefix + ".OutputSizes.bin").c_str());
     if (rc) {

@@ -1,7 +1,7 @@
 """The host compressors and the .bin exporter under AddressSanitizer and UndefinedBehaviorSanitizer
 (`make -C flash-llm_amd asan`, a host-only build of csrc/tiled_csl_compress.cpp and csrc/bin_export.cpp with the
 driver tests/cxx/asan_compress.cpp): every known-answer tile, the special-value patterns, dense, empty and
-ragged matrices go through both compressors (one and three worker threads) and the exporter; a sanitizer report
+ragged matrices go through both compressors (one and three worker threads), the packing for the way to the GPU and the exporter; a sanitizer report
 ends the driver with a non-zero code, and what it wrote is compared with the oracle's bytes."""
 import os
 import subprocess
@@ -19,7 +19,7 @@ EXE = os.path.join(ROOT, "tests", "cxx", "asan_compress.bin")
 @pytest.fixture(scope="module")
 def driver():
     sources = [os.path.join(ROOT, "tests", "cxx", "asan_compress.cpp"), os.path.join(ROOT, "flash-llm_amd", "csrc", "tiled_csl_compress.cpp"),
-               os.path.join(ROOT, "flash-llm_amd", "csrc", "bin_export.cpp")]
+               os.path.join(ROOT, "flash-llm_amd", "csrc", "bin_export.cpp"), os.path.join(ROOT, "flash-llm_amd", "csrc", "spmm_launch.h")]
     if not os.path.exists(EXE) or any(os.path.getmtime(EXE) < os.path.getmtime(s) for s in sources):
         r = subprocess.run(["make", "-C", os.path.join(ROOT, "flash-llm_amd"), "asan"], capture_output=True, text=True)
         assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
@@ -48,6 +48,7 @@ MATRICES.update({
     "one_column": one_column,
     "empty": lambda: np.zeros((256, 192), dtype=np.float16),
     "dense": lambda: synth.sparse_matrix(128, 128, 0.0, 5),
+    "dense_pieces": lambda: np.ones((384, 256), dtype=np.float16),  # a whole piece and half of one: every value stays, to the last place for them
     "random_80": lambda: synth.sparse_matrix(384, 320, 0.8, 6),
     "random_999": lambda: synth.sparse_matrix(256, 256, 0.999, 7),
 })

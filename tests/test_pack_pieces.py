@@ -23,12 +23,13 @@ def _halfs(form, n):
     return a
 
 
+@pytest.mark.parametrize("way", ["flashllm_pack_piece", "flashllm_pack_piece_plain"])
 @pytest.mark.parametrize("form", ["sparse", "empty", "dense", "special"])
 @pytest.mark.parametrize("n", [GROUP, 3 * GROUP, PIECE - GROUP, PIECE])
-def test_a_piece_holds_every_half_that_is_not_all_zero_bits(product, form, n):
+def test_a_piece_holds_every_half_that_is_not_all_zero_bits(product, form, n, way):
     a = _halfs(form, n)
     out = np.full(STRIDE + 64, 0xa5, dtype=np.uint8)
-    fn = product.lib().flashllm_pack_piece
+    fn = getattr(product.lib(), way)
     fn.restype, fn.argtypes = None, [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
     fn(a.ctypes.data, n, out.ctypes.data)
     kept = a != 0
