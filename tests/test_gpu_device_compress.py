@@ -306,23 +306,37 @@ def test_loaded_weight_has_the_host_compressors_bytes(product, torch_gpu, form, 
 
 
 @pytest.mark.parametrize("threads", [1, 16])
-@pytest.mark.parametrize("shape", [(128, 64), (1024, 1024), (1152, 1088), (4096, 4096), (7168, 2048)])
-def test_a_matrix_arrives_whole_without_its_zeros_on_the_way(product, torch_gpu, monkeypatch, shape, threads):
+@pytest.mark.parametrize("shape", [(128, 64), (1024, 1024), (1152, 1088), (4096, 4096), (7168, 2048), (8320, 4032)])
+def test_a_matrix_arrives_whole_without_its_zeros_on_the_way(product, torch_gpu, shape, threads):
     """Pieces of 65536 halfs, parts of 32 of them, seven parts in the ring: less than a piece, a part, a piece and a bit more than whole
-    parts, the ring gone round.  Every bit pattern that is not zero comes back, -0 and NaN too."""
+    parts, the ring gone round, every place taken again and two of them a third time by a part that is not full.  Every bit pattern that is
+    not zero comes back, -0 and NaN too.  Other contents each time, and neither memory holds those of the time before: what is not written,
+    or not there yet when it is read, shows."""
+    torch, L = torch_gpu, product.lib()
     say("packed upload:", shape, threads)
-    rng = np.random.default_rng(shape[0])
-    a = synth.sparse_matrix(*shape, 0.8, 52).view(np.uint16).copy()
-    a[::5] = rng.integers(0, 65536, a[::5].shape, dtype=np.uint16)
-    a[3::7] = 0
-    a[1::9, ::2] = 0x8000
-    monkeypatch.setattr(product, "UPLOAD_PACKED_BYTES", 1)
-    product.lib().flashllm_set_compress_threads(threads)
+    halfs = shape[0] * shape[1]
+    dst = torch.empty(halfs, dtype=torch.int16, device="cuda")
+    stage = torch.empty(L.flashllm_hip_upload_stage(halfs), dtype=torch.uint8, device="cpu", pin_memory=True)
+    L.flashllm_set_compress_threads(threads)
     try:
-        for _ in range(3):
-            assert np.array_equal(product._upload(a).cpu().numpy().view(np.uint16), a)
+        for turn in range(3):
+            rng = np.random.default_rng([*shape, threads, turn])
+            a = rng.integers(0, 65536, halfs, dtype=np.uint16)
+            part = 32 * 65536
+            for i, at in enumerate(range(0, halfs, part)):  # sparse, nearly empty, dense, half full, ... parts
+                keep = (0.2, 0.01, 1.0, 0.5, 0.1)[(i + turn) % 5]
+                some = a[at:at + part]
+                some[rng.random(some.size, dtype=np.float32) >= keep] = 0
+            a = a.reshape(shape)
+            a[3::7] = 0
+            a[1::9, ::2] = 0x8000
+            dst.fill_(-1)
+            stage.zero_()  # pieces without values, so that one fetched too early is an empty one and no index out of range
+            torch.cuda.synchronize()
+            assert L.flashllm_hip_upload_packed(product._stream(None), dst.data_ptr(), a.ctypes.data, a.size, stage.data_ptr()) == 0
+            assert np.array_equal(dst.cpu().numpy().view(np.uint16).reshape(shape), a), (turn,)
     finally:
-        product.lib().flashllm_set_compress_threads(0)
+        L.flashllm_set_compress_threads(0)
 
 
 def test_the_default_device_has_no_say_in_how_a_matrix_arrives(product, torch_gpu, monkeypatch):
