@@ -264,7 +264,7 @@ def device_compress_status(stream=None):
 HIP_ERROR_OUT_OF_MEMORY = 2
 
 
-UPLOAD_PACKED_BYTES = 2 << 20  # below, the runtime's copy is as quick: 1024 x 1024 at 80 % 0.09 ms either way
+UPLOAD_PACKED_BYTES = 5 << 19  # 1024 x 1280; below, the runtime's copy is as quick: 1024 x 1024 at 80 % 0.09 ms either way, 1024 x 1280 0.104 and 0.092
 
 
 _packed_uploads = threading.BoundedSemaphore(4)  # at a time, and with them their pinned memory: one alone takes 1.06 ms, two 0.81 each, four 0.69

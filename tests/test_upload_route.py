@@ -70,7 +70,8 @@ def test_a_small_matrix_with_few_zeros_goes_as_it_is(way_of):
     assert way_of(synth.sparse_matrix(1280, 1536, 0.7, 3), 16) == "_packed"
     assert way_of(synth.sparse_matrix(1024, 4032, 0.0, 3), 16) == "as it is"
     assert way_of(synth.sparse_matrix(1024, 4096, 0.0, 3), 16) == "_packed"
-    assert way_of(synth.sparse_matrix(896, 1024, 0.8, 3), 16) == "as it is"
+    assert way_of(synth.sparse_matrix(1024, 1024, 0.8, 3), 16) == "as it is"
+    assert way_of(synth.sparse_matrix(1024, 1280, 0.8, 3), 16) == "_packed"
 
 
 def test_without_pinned_memory_it_goes_as_it_is(way_of):
