@@ -242,10 +242,11 @@ __device__ __forceinline__ void take_8_and_wait(uintx4 (&a)[8], const uint32_t (
 
 // An operand by two exchanges that the compiler knows of: the products of the first row blocks run while the operands of the later ones are
 // on their way.  For eight row tiles per workgroup (N = 64), whose waves are in step and would all exchange and then all multiply: 36864
-// x 9216, 80 %, Split_K 7 72.6 -> 67.9 us, 49152 x 12288, 5 121.3 -> 109.3.  Waves that run freely fill each other's gaps, and lose by 16
-// more instructions per tile: 11392 x 18112, N = 64, Split_K 11 46.5 and 48.0, 36864 x 9216, N = 16 52.3 and 53.8, 49152 x 12288, N = 32 93.7
-// and 95.8.  By loads and, behind them, stores of zeros the first took 75.4, 9216 x 36864, N = 64, 90 % 70 instead of 66: 1 KB takes the LDS of a
-// CU 5.7 ns to store, 5.4 to exchange and 1.8 to load.
+// x 9216, Split_K 7, at 70, 80 and 90 % 89.3 -> 88.1, 72.4 -> 68.2 and 65.3 -> 60.7 us, 49152 x 12288, 5 142 -> 140, 116.9 -> 113.6 and 105.2 ->
+// 96.8.  Waves that run freely fill each other's gaps, and lose by 16 more instructions per tile: 11392 x 18112, N = 64, Split_K 11 46.5
+// and 48.0, 36864 x 9216, N = 16 52.3 and 53.8, 49152 x 12288, N = 32 93.7 and 95.8.  By loads and, behind them, stores of zeros the first
+// took 75.4 at 80 % instead of 67.9, 9216 x 36864, N = 64, 90 % 70 instead of 66: 1 KB takes the LDS of a CU 5.7 ns to store, 5.4 to
+// exchange and 1.8 to load.
 __device__ __forceinline__ uintx4 take(uint32_t addr)
 {
     using Half = __attribute__((address_space(3), may_alias)) uint64_t;
@@ -1218,7 +1219,8 @@ __global__ __launch_bounds__(kWideWaves* kLanes, 2) void spmm_wide_kernel(const 
 //     (v_mad_u32_u16 takes the upper half), M0 is set for every fourth request for B, requests are two slots apart, and scalar work is
 //     not left to the phases' ends, where nothing covers it.  Calls in turn, before and after: 7168 x 28672, N = 512 214 -> 206 us, 21504
 //     x 7168, N = 384 126 -> 121, 36864 x 9216, N = 128, Split_K 3 at 80 and 90 % 108 -> 106 and 99 -> 94, 28672 x 7168, N = 64 45.2 ->
-//     44.0.  The mask is 1 % of that (21504 x 7168, N = 384 118.4 us without, 120.0 with it).
+//     44.0.  The mask is 1 % of that (21504 x 7168, N = 384 118.4 us without, 120.0 with it), with 64 columns up to 2.5 % (6528 x 18240, Split_K
+//     5, 78 % 30.5 and 31.2).
 //   * The stream is loaded as other data is: the column groups of a row tile sit on one XCD and share its L2 (7168 x 28672, N =
 //     512, Split_K 1 210.7 us with non-temporal loads, 202.3).
 // With 64 columns (N = 64) a tile is two such phases and one window of B, so that B is asked for two tiles ahead; a tile without
@@ -1227,7 +1229,7 @@ __global__ __launch_bounds__(kWideWaves* kLanes, 2) void spmm_wide_kernel(const 
 // 1, with the kernels before (four waves on every tile, where a launch had at most one workgroup per CU three groups of four; 256
 // columns) and this one: 7168 x 28672, N = 512 244 -> 202 us, 7168 x 7168, N = 512 70.5 -> 55.9, N = 128 69.6 -> 52.2, 21504 x 7168, N =
 // 384 132.8 -> 117.0, N = 512 180.1 -> 166.8, 1664 x 27200, N = 128 232 -> 169, 28672 x 7168, N = 64 47.5 -> 42.6.  21504 x 7168, N = 384 under counters:
-// matrix cores busy half of the time that a workgroup runs, LDS 42 %, 21 % of the waves' time waiting for memory and 17 % for LDS, 83 LDS
+// matrix cores busy half of the time that a workgroup runs, LDS 43 %, 19 % of the waves' time waiting for memory and 17 % for LDS, 83 LDS
 // instructions per tile.  As first built (213 us on the first) it took 161 without loads from memory and 128 with nothing but the
 // MFMAs; with B through registers and LDS stores 238, with B's windows by halves of k instead of columns, i.e. 64-byte pieces of lines,
 // 261.
@@ -1990,9 +1992,11 @@ int launch_by_columns(hipStream_t s, const void* comp, const int* offs, const vo
 // workgroups, each of which fills a CU, number between 192 and 256: one round on at least three quarters of the
 // 256 CUs.  Otherwise 1: fewer, larger workgroups would leave CUs idle (7168 x 7168 at its best Split_K: 23.8 us
 // with one row tile per workgroup, 29.6 us with eight), more would run in two rounds.
-// Measured at 36864 x 9216, 80 %: n = 64 62-64 us against 73.6 with one row tile per workgroup; n = 32 52.4
+// Calls at n = 64, Split_K 7, 80 %: 36864 x 9216 68.2 us, with one row tile per workgroup 84.6, 36864 x 12288 88.6 and 109.8; at 70 and
+// 90 % the first 88.1 and 100.3, 60.7 and 68.0.  At n = 32 52.4
 // against 51.7 (the four fragment loads a tile costs there are no more than the meeting and the LDS reads that
-// replace them), and workgroups of four row tiles meeting at every tile gain nothing at n = 64 (72.9 us).
+// replace them), and workgroups of four row tiles meeting at every tile gain nothing at n = 64 (72.9 us, eight 62 to 64 then).
+// The lines at 192 and 256 are from then; fewer workgroups have not been measured since the form takes 2 to 8 % less.
 // g_rows_override (a measuring and testing aid): 1 forces 1, 8 forces 8 wherever the row tiles allow it.
 std::atomic<int> g_rows_override{0};
 

@@ -300,12 +300,12 @@ __device__ __forceinline__ void lds_done()
 // all levels at once in 16 lanes, row addresses in scalar registers; 493 and 349.  27648 x 9216, 80 %: 133.8 -> 121.7 us (5.9 TB/s;
 // without its stores 104), 90 % 120 -> 106, 70 % 149 -> 142, 7168 x 7168 32.2 -> 28.9.  Seven or eight workgroups per CU instead of six,
 // with fewer masks held: 3 % faster at 90 %, 4 to 7 % slower at 70 %.
-// The list holds 128 levels (16 KB; the registers, 73, allow six workgroups per CU).  A tile in which a bank holds more
+// The list holds 128 levels (16 KB; the registers, 75, allow six workgroups per CU).  A tile in which a bank holds more
 // (beyond about 45 % of all its elements) takes each item's pop number from a table of the levels instead, and the list in
 // two parts: the pops that fit, up to the end of a pass of four, then the rest.  27648 x 9216, both calls: 320 us at 50 %
 // and 366 at 20 % sparsity (589 and 818 when every nonzero stored itself to its place in memory; 244 at 70 %).
 constexpr int kEncodeThreads = 256;
-constexpr int kFarColumns    = 1 << 26;  // FAR: from here on; sixteen rows of fewer are less than 4 GB
+constexpr int kFarColumns    = 1 << 26;  // FAR: from here on; the other half of a wave is 16 rows on, 32 * k bytes, less than 2^31 for fewer
 constexpr int kSegments      = kEncodeThreads / kBanks;
 constexpr int kRowsOfThread  = kTileRows / kSegments;
 constexpr int kLevels        = 128;
@@ -564,7 +564,7 @@ __global__ __launch_bounds__(kEncodeThreads, 6) void encode_tiles_kernel(const u
 // One workgroup of four waves per tile, half a row (64 bytes) to a thread: the items before it are the nonzeros before it, by
 // a scan over the workgroup, and of the zeros before it at most as many as the tile is padded with.  The tile is put
 // together in LDS and stored as consecutive 16-byte vectors.  32 KB of LDS, four workgroups per CU;
-// bound by HBM like the encoder above (27648 x 9216 with the count 250 us, reordered 254).
+// bound by HBM like the encoder above (27648 x 9216 with the count 251 us, reordered 225; 36864 x 9216 326 and 292).
 constexpr int kHalfRow = kTileCols / 2;
 
 __global__ __launch_bounds__(kEncodeThreads) void encode_tiles_scan_kernel(const uint16_t* __restrict__ a,
@@ -635,7 +635,7 @@ __global__ __launch_bounds__(kEncodeThreads) void encode_tiles_scan_kernel(const
 // Packed pieces (spmm_launch.h) in pinned host memory -> the dense matrix.  One workgroup per group of 2048 halfs, a byte of the bits and
 // eight halfs to a thread; the group's values come through LDS, so that what crosses the link is whole 16-byte vectors.  The kernel fetches
 // them itself because the pieces lie a full piece apart (a copy would carry that) and 25 launches do for 7168 x 7168.  Bound by the
-// link and the threads that pack: 27 of its 103 MB at 80 %, 1.1 ms.
+// link and the threads that pack: 27 of its 103 MB at 80 %, 0.92 ms; a launch for 32 pieces takes 26.5 us, i.e. 41 GB/s.
 constexpr int kExpandThreads = kPackGroup / 8;
 
 __global__ __launch_bounds__(kExpandThreads) void expand_kernel(const unsigned char* __restrict__ pieces, uintx4* __restrict__ dst)
@@ -681,7 +681,7 @@ __global__ __launch_bounds__(kExpandThreads) void expand_kernel(const unsigned c
 }
 
 // The pinned memory is a ring of parts, each of them one launch: while the GPU fetches one part, the threads pack the ones after it.
-// 7168 x 7168, 80 %, whole load with 12 threads: 4 parts of 32 pieces 1.29 ms, 8 of 16 1.22, 16 of 16 1.22, 8 of 32 1.04; seven of 32
+// 7168 x 7168, 80 %, whole load, with 12 threads as long as there could be so many: 4 parts of 32 pieces 1.29 ms, 8 of 16 1.22, 16 of 16 1.22, 8 of 32 1.04; seven of 32
 // stay below 32 MB, to which torch rounds up.
 constexpr int kPartPieces = 32;
 constexpr int kParts      = 7;
@@ -777,7 +777,7 @@ extern "C" int flashllm_hip_upload_packed(void* stream, void* dst, const void* s
     };
     std::vector<std::thread> pool;
     try {  // a thread that cannot be created is left out
-        // a thread for eight pieces (2048 x 2048 0.21 ms with 6 threads, 0.36 with 16), and at most eight: 7168 x 7168 1.14 ms, 1.09 with 16
+        // a thread for eight pieces (2048 x 2048 0.21 ms with 6 threads, 0.36 with 16), and at most eight: 16 took 4 % off 7168 x 7168 for twice the cores
         const int workers = flashllm_compress_workers(pieces / 8 < 8 ? pieces / 8 : 8);
         pool.reserve(workers);
         for (int w = 1; w < workers; w++)

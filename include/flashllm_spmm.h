@@ -39,7 +39,9 @@ void flashllm_free(void* p);
 
 /* Worker threads the compressors use (tiles are independent); 0 = one per
  * host core, capped at 16.  The reference is single-threaded
- * (csrc/SpMM_API.cu:235-351); the bytes do not depend on this setting. */
+ * (csrc/SpMM_API.cu:235-351); the bytes do not depend on this setting.
+ * They also pack a host matrix that the Python binding's SparseWeight sends
+ * to the GPU: at most eight of them, and with one it is sent unpacked. */
 void flashllm_set_compress_threads(int n);
 
 /*
